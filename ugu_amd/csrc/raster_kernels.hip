@@ -26,6 +26,7 @@
 #include <float.h>
 #include <limits.h>
 
+#include "binning.h"
 #include "device_common.h"
 
 #pragma clang fp contract(off)
@@ -256,95 +257,6 @@ __global__ void k_face_soup(const float* __restrict__ verts, const int32_t* __re
 // ---------------------------------------------------------------------------
 // k_setup_bin: one thread per (face, view)
 
-// Appends `entry` to a bin segment for every lane with `has`, in two halves.
-// `seg` = 4 * tile for the front segment (filled upwards from the bin's first
-// slot) and 4 * tile + 1 for the back segment (filled downwards from its last
-// slot). append_issue groups the lanes that target the same segment (ballot +
-// popcount rank) and the group leaders issue their atomicAdds together;
-// append_finish broadcasts each group's base and stores the entries. A caller
-// issues several appends before finishing any, so the wavefront waits for
-// one atomic round trip for all of them. Entries of one segment are in no
-// particular order (the rasterizer's result does not depend on it). When the
-// two segments together overflow the bin they overwrite each other's slots;
-// every slot the rasterizer reads still holds a valid entry, and the host
-// renders again with larger bins.
-struct AppendTicket {
-  int ret;   // the group's first slot, in the leader lane
-  int lr;    // leader lane | rank in the group << 8
-  int seg;   // segment, -1 for lanes without an entry
-};
-
-// Lower bound of the skip depths of a wavefront's back-face entries (bits of
-// a non-negative float; 0 when one has no bound): the leaders of back groups
-// fold it into their tile's back-segment minimum.
-UGU_DEV uint32_t back_zmin(bool back, float zskip) {
-  uint32_t zmin = 0xffffffffu;
-  if (__ballot(back))
-    zmin = wave_min_u32(back ? (zskip >= 0.0f ? __float_as_uint(zskip) : 0u) : 0xffffffffu);
-  return zmin;
-}
-
-UGU_DEV AppendTicket append_issue(const DevBins& bins, int seg, uint32_t zmin, bool has) {
-  AppendTicket tk;
-  tk.ret = 0;
-  tk.lr = 0;
-  tk.seg = has ? seg : -1;
-  const uint64_t hasm = __builtin_amdgcn_ballot_w64(has);
-  if (!hasm) return tk;
-  // Each pass takes the lowest pending lane; the lanes with its segment form
-  // one group, whose lowest lane (that one) leads it. A lane keeps its
-  // group's mask; rank, leader and size follow from it after the loop.
-  uint64_t todo = hasm, grp_mine = 0;
-  while (todo) {
-    const int l = __ffsll(static_cast<unsigned long long>(todo)) - 1;
-    const int ls = __builtin_amdgcn_readlane(seg, l);
-    const uint64_t grp = __builtin_amdgcn_ballot_w64(seg == ls) & hasm;
-    grp_mine = (has && seg == ls) ? grp : grp_mine;
-    todo &= ~grp;
-  }
-  const int rank = static_cast<int>(__builtin_amdgcn_mbcnt_hi(
-      static_cast<uint32_t>(grp_mine >> 32),
-      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(grp_mine), 0u)));
-  if (has && rank == 0) {
-    tk.ret = atomicAdd(&bins.counts[seg], __popcll(grp_mine));
-    if (seg & 1) atomicMin(reinterpret_cast<unsigned int*>(bins.counts) + (seg + 1), zmin);
-  }
-  const int leader = has ? __ffsll(static_cast<unsigned long long>(grp_mine)) - 1 : 0;
-  tk.lr = leader | (rank << 8);
-  return tk;
-}
-
-// Finishes the first `used` (wavefront-uniform) of R tickets: every group
-// base is broadcast before the first store, so the wavefront waits once for
-// all its atomics (a store issued before a later wait would be waited for as
-// well).
-template <int R>
-UGU_DEV void append_finish(const DevBins& bins, const AppendTicket* tk, const int2* entry,
-                           int used = R) {
-  int slot[R];
-#pragma unroll
-  for (int r = 0; r < R; r++)
-    slot[r] = r < used ? __shfl(tk[r].ret, tk[r].lr & 0xff) + (tk[r].lr >> 8) : 0;
-#pragma unroll
-  for (int r = 0; r < R; r++) {
-    if (r < used && tk[r].seg >= 0 && slot[r] < bins.cap) {
-      const int64_t row = int64_t(tk[r].seg >> 2) * bins.cap;
-      bins.bins[row + ((tk[r].seg & 1) ? bins.cap - 1 - slot[r] : slot[r])] = *entry;
-    }
-  }
-}
-
-// Entry i of a tile's bin: the front segment's nA entries, then the back
-// segment read from the bin's last slot downwards.
-// Each entry is read once, so the load is non-temporal: the stream of entries
-// does not evict the face records, shading records and texels the rasterizer
-// reads again (64-view batch: rasterizer -2%).
-UGU_DEV int2 bin_entry(const int2* bin, int nA, int cap, int i) {
-  const int2* p = i < nA ? bin + i : bin + (cap - 1 - (i - nA));
-  const long long q = __builtin_nontemporal_load(reinterpret_cast<const long long*>(p));
-  return make_int2(static_cast<int>(q & 0xffffffffll), static_cast<int>(q >> 32));
-}
-
 // Skip depth of a face in a view: a lower bound of every depth the coverage
 // test (cover_test) can compute for the face at a pixel of its bbox, or -1
 // when no useful bound exists. Once every in-view pixel of a tile holds a depth
@@ -374,28 +286,6 @@ UGU_DEV float skip_depth(const float4& a, const float4& b, const float4& c, floa
   // three positive depths: std::min is the hardware min
   return fminf(fminf(a.z, b.z), c.z);
 }
-
-// True when the tile's current depth bound proves the face hidden.
-UGU_DEV bool skip_face(float zskip, float dmax) {
-  return dmax >= 1e-18f && zskip > dmax * 1.00390625f;
-}
-
-// Views per thread: the face's indices are loaded once and reused for
-// kSetupViews consecutive views (grid.y = ceil(n_views / kSetupViews)).
-constexpr int kSetupViews = 8;
-
-// Bin appends a setup thread issues before waiting for their atomics: a face
-// whose pixel bbox spans up to this many tiles costs one atomic round trip
-// per view.
-constexpr int kAppendRounds = 4;
-
-// Chunks whose faces all have at most this many (face, pixel) pairs expand
-// them through an LDS pair list; otherwise by binary search over the prefix.
-constexpr int kScatterMaxPairs = 32;
-
-// Faces whose pixel bbox holds at most this many pixel centres are tested at
-// those centres before they are binned.
-constexpr int kCoverProbe = 4;
 
 // Tiles of a small face's bbox (at most kCoverProbe pixel centres, so at most
 // 2 x 2 tiles) holding a centre the face may cover: bit (tx - tx0) + 2 (ty -

@@ -1,23 +1,80 @@
 // HIP kernel of the gfx950 raytracer: Raytracer::Impl::Render
 // (src/renderer/cpu/raytracer.cc:117-225) for a batch of views.
 //
-// One wave per 8x8 pixel tile, one lane per pixel. The wave walks the BVH
-// (built on the host, nodes hold both children's boxes) as one packet of 64
-// rays, nearer child first, and every lane tests the triangles of every leaf
-// reached with the reference's float64 Moller-Trumbore routine
-// (src/util/geom_util.cc:60-115, epsilon double(1e-8f) of bvh_naive.h:121,
-// standard barycentric conversion).
+// Two ways to the same closest hit, both by the reference's float64
+// Moller-Trumbore routine (src/util/geom_util.cc:60-115, epsilon double(1e-8f) of
+// bvh_naive.h:121, standard barycentric conversion):
+//   k_rt_setup, k_rt_tiles  bins of faces per 16x16 pixel tile, every ray tested
+//                           against its tile's faces (meshes of few layers);
+//   k_raytrace              one wave per 8x8 pixel tile walks the BVH (built on
+//                           the host, nodes hold both children's boxes) as one
+//                           packet of 64 rays, nearer child first, and every
+//                           lane tests the triangles of every leaf reached.
 // The closest hit is the smallest float t; equal t resolve to the lowest face
 // id. The box test is float32 with widened boxes and a relative slack on the
 // ray interval, so it only prunes boxes that cannot hold a hit the float64 test
-// would accept. Then the pixel is culled or shaded as in raytracer.cc:160-218.
+// would accept; the bins' bounds are those of project_ray. Then the pixel is culled or shaded as in raytracer.cc:160-218.
 
+#include "binning.h"
 #include "device_common.h"
 #include "rt_math.h"
 
 #pragma clang fp contract(off)
 
 namespace ugu_hip {
+
+// Writes pixel (x, y): face bf hit at distance bt with the raytracer's weights
+// (bu, bv), or no hit (bf < 0); culling, depth, normal and colour of
+// raytracer.cc:160-218.
+template <bool STREAM>
+UGU_DEV void write_hit(const DevView& v, const DevMesh& m, const DevOptions& o, int x, int y, int bf,
+                       float bt, float bu, float bv, float r0, float r1, float r2) {
+  const int64_t pi = int64_t(y) * v.W + x;
+  bool hit = bf >= 0;
+  // back-face culling: face normal . ray_w > 0 -> background (raytracer.cc:166-172)
+  if (hit && o.culling && backface_of(m.fnormals, bf, r0, r1, r2)) hit = false;
+  if (!hit) {
+    if (v.color) put3<STREAM>(v.color, pi, uint8_t(0), uint8_t(0), uint8_t(0));
+    if (v.depth) put<STREAM>(v.depth, pi, 0.0f);
+    if (v.normal) put3<STREAM>(v.normal, pi, 0.0f, 0.0f, 0.0f);
+    if (v.mask) put<STREAM>(v.mask, pi, uint8_t(0));
+    if (v.face_id) put<STREAM>(v.face_id, pi, -1);
+    return;
+  }
+  // hit_pos_c = w2c_R * (org + ray * t) + w2c_t; depth = z * depth_scale
+  const float h0 = v.c2w_t[0] + r0 * bt, h1 = v.c2w_t[1] + r1 * bt, h2 = v.c2w_t[2] + r2 * bt;
+  const float zc = sum3(v.w2c_R[6] * h0, v.w2c_R[7] * h1, v.w2c_R[8] * h2) + v.w2c_t[2];
+  float n0, n1, n2;
+  FaceShade fs;
+  face_shade(m, bf, o.shading_normal != 0, v.color && o.diffuse_color == 1, fs);
+  if (o.shading_normal == 0) {
+    const float* fn = m.fnormals + int64_t(bf) * 3;
+    n0 = fn[0];
+    n1 = fn[1];
+    n2 = fn[2];
+  } else {
+    // (1 - u - v) n[i0] + u n[i1] + v n[i2] with the raytracer's (u, v)
+    const float* na = fs.na;
+    const float* nb = fs.nb;
+    const float* nc = fs.nc;
+    const float w = 1.0f - bu - bv;
+    n0 = w * na[0] + bu * nb[0] + bv * nc[0];
+    n1 = w * na[1] + bu * nb[1] + bv * nc[1];
+    n2 = w * na[2] + bu * nb[2] + bv * nc[2];
+  }
+  if (v.color) {
+    uint8_t c[3];
+    shade_u8(m, o, bf, fs, bu, bv, r0, r1, r2, n0, n1, n2, c);
+    put3<STREAM>(v.color, pi, c[0], c[1], c[2]);
+  }
+  if (v.depth) put<STREAM>(v.depth, pi, zc * o.depth_scale);
+  if (v.normal)
+    put3<STREAM>(v.normal, pi, sum3(v.w2c_R[0] * n0, v.w2c_R[1] * n1, v.w2c_R[2] * n2),
+                 sum3(v.w2c_R[3] * n0, v.w2c_R[4] * n1, v.w2c_R[5] * n2),
+                 sum3(v.w2c_R[6] * n0, v.w2c_R[7] * n1, v.w2c_R[8] * n2));
+  if (v.mask) put<STREAM>(v.mask, pi, uint8_t(255));
+  if (v.face_id) put<STREAM>(v.face_id, pi, bf);
+}
 
 // Four waves per workgroup, each on its own tile (no cross-wave sharing).
 constexpr int kRtWaves = 4;
@@ -126,66 +183,437 @@ __global__ __launch_bounds__(64 * kRtWaves) void k_raytrace(const DevView* __res
     ref = __builtin_amdgcn_readfirstlane(stack[sp]);
   }
   if (!act) return;
-  const int64_t pi = int64_t(y) * v.W + x;
+  write_hit<false>(v, m, o, x, y, bf, bt, bu, bv, r0, r1, r2);
+}
 
-  bool hit = bf >= 0;
-  // back-face culling: face normal . ray_w > 0 -> background (raytracer.cc:166-172)
-  if (hit && o.culling && backface_of(m.fnormals, bf, r0, r1, r2)) hit = false;
+// ---------------------------------------------------------------------------
+// Binned path. All rays of a view start at the camera, so the face a pixel's
+// ray hits first can be found as a rasterizer finds it: every face is put into
+// the bins of the screen tiles its hits can lie in, and a tile tests its rays
+// against its bin's faces only. The hit test is the same float64 one
+// (mt_hit), so the closest hit is the hierarchy walk's; the bins only decide
+// which tests are made, and they are conservative (project_ray).
 
-  if (!hit) {
-    if (v.color) {
-      v.color[pi * 3 + 0] = 0;
-      v.color[pi * 3 + 1] = 0;
-      v.color[pi * 3 + 2] = 0;
+// Pixel position of a world point as the rays see it: the ray of pixel (x, y)
+// is c2w_R times the normalized ((x - cx) / fx, (y - cy) / fy, 1), so a point P
+// lies on it where q = inverse(c2w_R) (P - c2w_t) is a multiple of that
+// vector. Returns (x, y, q.z, w): rays of pixels further than w from (x, y) in
+// x or y miss the point. w bounds the float32 rounding of this projection and
+// of the rays: with u = 2^-24, S = |P - o| in the 1-norm and K the condition
+// number of c2w_R, rays and q carry less than 25 u K S of absolute error (one
+// rounding of P - o, of the matrix entries and of each product and sum, the
+// same for the ray, whose normalization scales it as a whole); rt_rel is
+// 64 u K, and an error dq of q moves the pixel by at most
+// |dq| / q.z (f + |x - cx| + |y - cy|). The last roundings of x and y are
+// 2^-20 of the same sum and of cx, cy (rt_abs). Points closer to the camera's
+// plane than S / 64, behind it or not finite get w = -1: no bound.
+UGU_DEV float4 project_ray(const DevView& v, float px, float py, float pz) {
+  const float dx = px - v.c2w_t[0], dy = py - v.c2w_t[1], dz = pz - v.c2w_t[2];
+  const float qx = v.inv[0] * dx + v.inv[1] * dy + v.inv[2] * dz;
+  const float qy = v.inv[3] * dx + v.inv[4] * dy + v.inv[5] * dz;
+  const float qz = v.inv[6] * dx + v.inv[7] * dy + v.inv[8] * dz;
+  const float s = fabsf(dx) + fabsf(dy) + fabsf(dz);
+  const float iz = __builtin_amdgcn_rcpf(qz);
+  const float x = v.fx * qx * iz, y = v.fy * qy * iz;
+  float4 r;
+  r.x = x + v.cx;
+  r.y = y + v.cy;
+  r.z = qz;
+  r.w = v.rt_abs + (v.rt_rel * s * iz + 9.5367431640625e-07f) * (v.rt_f + fabsf(x) + fabsf(y));
+  if (!(qz >= s * 0.015625f && r.w < 1e6f)) r.w = -1.0f;
+  return r;
+}
+
+// True when every point of the face lies outside one side of the image's
+// frustum (a pixel wider than the image on each side, minus the error of q),
+// or behind the camera: no ray of the view can hit it. For faces with a corner
+// that project_ray gives no bound for.
+UGU_DEV bool outside_frustum(const DevView& v, const float* P) {
+  int out = 31;
+  for (int k = 0; k < 3; k++) {
+    const float dx = P[3 * k] - v.c2w_t[0], dy = P[3 * k + 1] - v.c2w_t[1],
+                dz = P[3 * k + 2] - v.c2w_t[2];
+    const float qx = v.inv[0] * dx + v.inv[1] * dy + v.inv[2] * dz;
+    const float qy = v.inv[3] * dx + v.inv[4] * dy + v.inv[5] * dz;
+    const float qz = v.inv[6] * dx + v.inv[7] * dy + v.inv[8] * dz;
+    const float s = (fabsf(dx) + fabsf(dy) + fabsf(dz)) * (v.rt_rel + 9.5367431640625e-07f);
+    const float gx = v.fx * qx, gy = v.fy * qy;
+    // pixel x times q.z, against x = -1 and x = W; likewise y
+    const float ex = s * (v.rt_f + fabsf(v.cx) + static_cast<float>(v.W) + 1.0f);
+    const float ey = s * (v.rt_f + fabsf(v.cy) + static_cast<float>(v.H) + 1.0f);
+    int o = 0;
+    if (gx + (v.cx + 1.0f) * qz < -ex) o |= 1;
+    if (gx + (v.cx - static_cast<float>(v.W)) * qz > ex) o |= 2;
+    if (gy + (v.cy + 1.0f) * qz < -ey) o |= 4;
+    if (gy + (v.cy - static_cast<float>(v.H)) * qz > ey) o |= 8;
+    if (qz < -s) o |= 16;
+    out &= o;  // a NaN coordinate sets no bit
+  }
+  return out != 0;
+}
+
+// A bin entry is (face id, depth | box): the upper 16 bits of a float that is
+// at most the q.z of every hit of the face (0: no bound), and its pixel box
+// within the tile, x | y << 4 | (width - 1) << 8 | (height - 1) << 12.
+constexpr int kRtTile = 16;
+
+UGU_DEV int2 rt_entry(int f, float zskip, int x0, int x1, int y0, int y1, int tx, int ty) {
+  const int px = tx * kRtTile, py = ty * kRtTile;
+  const int lx0 = max(x0 - px, 0), lx1 = min(x1 - px, kRtTile - 1);
+  const int ly0 = max(y0 - py, 0), ly1 = min(y1 - py, kRtTile - 1);
+  const uint32_t box = lx0 | (ly0 << 4) | ((lx1 - lx0) << 8) | ((ly1 - ly0) << 12);
+  return make_int2(f, static_cast<int>((__float_as_uint(zskip) & 0xffff0000u) | box));
+}
+
+// One thread per (face, view), as the rasterizer's k_setup_bin: a block's
+// distinct vertices are projected once per view into LDS.
+__global__ __launch_bounds__(256) void k_rt_setup(const DevView* __restrict__ views, int n_views,
+                                                  DevMesh mesh, DevBins bins) {
+  __shared__ float4 sp[768];
+  const int f = blockIdx.x * blockDim.x + threadIdx.x;
+  const int vbase = mesh.blk_off[blockIdx.x];
+  const int nu = mesh.blk_off[blockIdx.x + 1] - vbase;
+  int loc[3] = {0, 0, 0};
+  float P[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  if (f < mesh.F) {
+    const uint32_t lc = mesh.face_loc[f];
+    loc[0] = lc & 1023u;
+    loc[1] = (lc >> 10) & 1023u;
+    loc[2] = lc >> 20;
+  }
+  for (int j = 0; j < 3; j++) {
+    const int k = threadIdx.x + j * 256;
+    if (k < nu) {
+      const float* q = mesh.verts + int64_t(mesh.blk_vid[vbase + k]) * 3;
+      P[j * 3 + 0] = q[0];
+      P[j * 3 + 1] = q[1];
+      P[j * 3 + 2] = q[2];
     }
-    if (v.depth) v.depth[pi] = 0.0f;
-    if (v.normal) {
-      v.normal[pi * 3 + 0] = 0.0f;
-      v.normal[pi * 3 + 1] = 0.0f;
-      v.normal[pi * 3 + 2] = 0.0f;
+  }
+  const int vb = blockIdx.y * kSetupViews;
+  const int ve = min(vb + kSetupViews, n_views);
+  for (int vi = vb; vi < ve; vi++) {
+    const DevView& v = views[vi];
+    for (int j = 0; j < 3; j++) {
+      const int k = threadIdx.x + j * 256;
+      if (k < nu) sp[k] = project_ray(v, P[j * 3 + 0], P[j * 3 + 1], P[j * 3 + 2]);
     }
-    if (v.mask) v.mask[pi] = 0;
-    if (v.face_id) v.face_id[pi] = -1;
+    __syncthreads();
+    const float4 a = sp[loc[0]], b = sp[loc[1]], c = sp[loc[2]];
+    __syncthreads();  // the next view overwrites the window
+    bool has = false, back = false;
+    float zskip = 0.0f;
+    int x0 = 0, x1 = -1, y0 = 0, y1 = -1;
+    uint32_t tmask = ~0u;
+    if (f < mesh.F) {
+      const float zmin = fminf(fminf(a.z, b.z), c.z), zmax = fmaxf(fmaxf(a.z, b.z), c.z);
+      // an accepted hit's barycentrics lie within rt_bary of the triangle; on
+      // screen that is at most rt_bary zmax / zmin of its extent
+      const float rat = v.rt_bary * zmax * __builtin_amdgcn_rcpf(zmin);
+      if (fminf(fminf(a.w, b.w), c.w) >= 0.0f && rat < 0.001953125f) {
+        const float xl = fminf(fminf(a.x, b.x), c.x), xh = fmaxf(fmaxf(a.x, b.x), c.x);
+        const float yl = fminf(fminf(a.y, b.y), c.y), yh = fmaxf(fmaxf(a.y, b.y), c.y);
+        const float ext = (xh - xl) + (yh - yl);
+        const float w = fmaxf(fmaxf(a.w, b.w), c.w) + 2.0f * rat * ext;
+        // |x|, |y| < 1e12 (the bound of w): clamped to the image before the
+        // conversion to int
+        x0 = static_cast<int>(fmaxf(ceilf(xl - w), 0.0f));
+        y0 = static_cast<int>(fmaxf(ceilf(yl - w), 0.0f));
+        x1 = static_cast<int>(fminf(floorf(xh + w), static_cast<float>(v.W - 1)));
+        y1 = static_cast<int>(fminf(floorf(yh + w), static_cast<float>(v.H - 1)));
+        if (!(xl - w <= static_cast<float>(v.W)) || !(yl - w <= static_cast<float>(v.H)) ||
+            !(xh + w >= 0.0f) || !(yh + w >= 0.0f)) x1 = -1;
+        has = x0 <= x1 && y0 <= y1;
+        zskip = zmin * 0.9921875f;
+        back = !(edge_fn(a.x, a.y, b.x, b.y, c.x, c.y) > 0.0f);
+        if (has && (x1 - x0 + 1) * (y1 - y0 + 1) <= kCoverProbe) {
+          // at most 2 x 2 tiles: only those with a pixel centre the face's
+          // hits can reach. A corner moved by w moves an edge function at a
+          // centre of the box by at most 3 w ext + 4 w w (the box is w wider).
+          const float tol = 3.0f * w * (ext + 4.0f * w) + 4.0f * w * w;
+          const int tx0 = x0 / kRtTile, ty0 = y0 / kRtTile;
+          tmask = 0u;
+          int px = x0, py = y0;
+#pragma unroll
+          for (int k = 0; k < kCoverProbe; k++) {
+            if (py <= y1) {
+              const float x = static_cast<float>(px), y = static_cast<float>(py);
+              const float w0 = edge_fn(b.x, b.y, c.x, c.y, x, y);
+              const float w1 = edge_fn(c.x, c.y, a.x, a.y, x, y);
+              const float w2 = edge_fn(a.x, a.y, b.x, b.y, x, y);
+              if (fminf(fminf(w0, w1), w2) >= -tol || fmaxf(fmaxf(w0, w1), w2) <= tol)
+                tmask |= 1u << ((px / kRtTile - tx0) + 2 * (py / kRtTile - ty0));
+              if (++px > x1) {
+                px = x0;
+                py++;
+              }
+            }
+          }
+          has = tmask != 0u;
+        }
+      } else {
+        float Q[9];
+        const float4* r = mesh.soup + int64_t(f) * 3;
+        const float4 r0 = r[0], r1 = r[1], r2 = r[2];
+        Q[0] = r0.x; Q[1] = r0.y; Q[2] = r0.z;
+        Q[3] = r0.w; Q[4] = r1.x; Q[5] = r1.y;
+        Q[6] = r1.z; Q[7] = r1.w; Q[8] = r2.x;
+        has = !outside_frustum(v, Q);
+        x0 = y0 = 0;
+        x1 = v.W - 1;
+        y1 = v.H - 1;
+      }
+    }
+    const int tx0 = x0 / kRtTile, tx1 = has ? x1 / kRtTile : -1;
+    const int ty0 = y0 / kRtTile, ty1 = has ? y1 / kRtTile : -1;
+    const uint32_t zmin = back_zmin(has && back, __uint_as_float(__float_as_uint(zskip) & 0xffff0000u));
+    const int nx = tx1 - tx0 + 1;
+    const int rest = has ? max(nx * (ty1 - ty0 + 1) - kAppendRounds, 0) : 0;
+    int tx = tx0, ty = ty0;
+    const bool probed = tmask != ~0u;
+    uint32_t pm = tmask;
+    AppendTicket tk[kAppendRounds];
+    int2 entry[kAppendRounds];
+    int used = 0;  // rounds issued: until no lane has a tile left
+#pragma unroll
+    for (int r = 0; r < kAppendRounds; r++) {
+      if (!__builtin_amdgcn_ballot_w64(has)) break;
+      used = r + 1;
+      int ax = tx, ay = ty;
+      if (probed) {
+        const int bit = __ffs(pm) - 1;
+        ax = tx0 + (bit & 1);
+        ay = ty0 + (bit >> 1);
+      }
+      entry[r] = rt_entry(f, zskip, x0, x1, y0, y1, ax, ay);
+      tk[r] = append_issue(bins, has ? 4 * (v.tile_base + ay * v.tiles_x + ax) + (back ? 1 : 0) : -1,
+                           zmin, has);
+      if (probed) {
+        pm &= pm - 1u;
+        has = has && pm != 0u;
+      } else if (has && ++tx > tx1) {
+        tx = tx0;
+        if (++ty > ty1) has = false;
+      }
+    }
+    append_finish<kAppendRounds, true>(bins, tk, entry, used);
+    // faces over more tiles: 64 (face, tile) pairs of the wavefront at a time
+    if (__any(rest > 0)) {
+      const int lane = __lane_id();
+      const int incl = wave_incl_sum(rest);
+      const int excl = incl - rest;
+      const int total = __builtin_amdgcn_readlane(incl, 63);
+      for (int base = 0; base < total; base += 64) {
+        const int p = base + lane;
+        int src = 0;
+        for (int step = 32; step >= 1; step >>= 1)
+          if (__shfl(excl, src + step) <= p) src += step;
+        const int k = p - __shfl(excl, src) + kAppendRounds;
+        const int snx = max(__shfl(nx, src), 1);
+        const int sx0 = __shfl(x0, src), sx1 = __shfl(x1, src);
+        const int sy0 = __shfl(y0, src), sy1 = __shfl(y1, src);
+        const int sty = sy0 / kRtTile + k / snx;
+        const int stx = sx0 / kRtTile + k % snx;
+        const int sback = __shfl(back ? 1 : 0, src);
+        const int2 e = rt_entry(__shfl(f, src), __shfl(zskip, src), sx0, sx1, sy0, sy1, stx, sty);
+        const bool act = p < total;
+        const AppendTicket t1 = append_issue(
+            bins, act ? 4 * (v.tile_base + sty * v.tiles_x + stx) + sback : -1, zmin, act);
+        append_finish<1, true>(bins, &t1, &e);
+      }
+    }
+  }
+}
+
+struct RtLds {
+  unsigned long long key[256];  // packed (hit distance bits << 32 | face id)
+  float ray[3][256];            // ray_w of each tile pixel
+  float p[9][256];              // staged faces: corner positions
+  int32_t fid[256];
+  uint16_t box[256];            // rt_entry's pixel box
+  int32_t pairs[2 * 256 + 1];   // as RasterLds::pairs
+  int32_t wsum[4];
+  int32_t wbig[4];
+  uint32_t wmax[4];
+};
+
+// One 16 x 16 pixel tile: its bin's faces are staged 256 at a time, expanded
+// to (face, pixel) pairs (as raster_tile does) and every pair runs the float64
+// hit test; a pixel keeps its smallest (distance, face id) with one LDS
+// atomicMin. Faces whose depth bound lies behind every hit of the tile are
+// dropped before their positions are fetched: the tile's bound is the largest
+// q.z = distance * (z of the normalized camera-space ray) its pixels hold, and a
+// face with all its q.z beyond it (by more than 2^-8, far above the float32
+// rounding of either) is hit later than what each pixel holds.
+// Bound by the latency of a tile's dependent loads (counters, entries, face
+// records, the winner's record and shading inputs), like k_raster. 1.3 M faces
+// at 1080p: setup 26 us + tiles 61 us, where the hierarchy walk (k_raytrace)
+// takes 836 us; 24 mixed views of 492 k faces: 153 + 323 us against 2505 us.
+__global__ __launch_bounds__(256) void k_rt_tiles(const DevView* __restrict__ views, DevMesh m,
+                                                  DevBins bins, DevOptions o) {
+  constexpr int NT = 256;
+  __shared__ RtLds s;
+  const int t = threadIdx.x;
+  const int gtile = xcd_remap(blockIdx.x, gridDim.x);
+  const int4 seg = reinterpret_cast<const int4*>(bins.counts)[gtile];
+  // some bin overflowed (this one: published, the two segments share it): the
+  // host renders again, nothing here is worth finishing
+  if (seg.x + seg.y > bins.cap || bins.status[0] > bins.cap) {
+    if (t == 0 && seg.x + seg.y > bins.cap) atomicMax(&bins.status[0], seg.x + seg.y);
     return;
   }
-  if (v.face_id) v.face_id[pi] = bf;
-  if (v.mask) v.mask[pi] = 255;
-  if (v.depth) {
-    // hit_pos_c = w2c_R * (org + ray * t) + w2c_t; depth = z * depth_scale
-    const float h0 = ox + r0 * bt, h1 = oy + r1 * bt, h2 = oz + r2 * bt;
-    const float zc = sum3(v.w2c_R[6] * h0, v.w2c_R[7] * h1, v.w2c_R[8] * h2) + v.w2c_t[2];
-    v.depth[pi] = zc * o.depth_scale;
+  const DevView& v = views[seg.w];
+  const int lt = gtile - v.tile_base;
+  const int tyi = lt / v.tiles_x, txi = lt - tyi * v.tiles_x;
+  const int gx = txi * kRtTile + t % kRtTile, gy = tyi * kRtTile + t / kRtTile;
+  const bool act = gx < v.W && gy < v.H;
+  const int nA = seg.x, nB = seg.y, n = nA + nB;
+  int bf = -1;
+  float r0 = 0.0f, r1 = 0.0f, r2 = 0.0f;
+  if (n > 0) {
+    const int2* bin = bins.bins + int64_t(gtile) * bins.cap;
+    const int chunks_a = (nA + NT - 1) / NT, chunks = chunks_a + (nB + NT - 1) / NT;
+    int2 e_next = make_int2(0, 0);
+    if (t < (chunks_a > 0 ? nA : n)) e_next = bin_entry(bin, nA, bins.cap, t);
+    ray_w_at(v, static_cast<float>(gx), static_cast<float>(gy), r0, r1, r2);
+    // z of the pixel's normalized camera-space ray: q.z of a hit at distance 1
+    const float u0 = (static_cast<float>(gx) - v.cx) / v.fx;
+    const float u1 = (static_cast<float>(gy) - v.cy) / v.fy;
+    const float zray = __builtin_amdgcn_rsqf(u0 * u0 + u1 * u1 + 1.0f);
+    const double ox = v.c2w_t[0], oy = v.c2w_t[1], oz = v.c2w_t[2];
+    s.key[t] = ~0ull;
+    s.ray[0][t] = r0;
+    s.ray[1][t] = r1;
+    s.ray[2][t] = r2;
+    float dmax = __uint_as_float(0xffffffffu);  // NaN: some pixel has no hit yet
+    for (int ch = 0; ch < chunks; ch++) {
+      if (ch == chunks_a && skip_face(__uint_as_float(static_cast<uint32_t>(seg.z)), dmax)) break;
+      const int base = ch < chunks_a ? ch * NT : nA + (ch - chunks_a) * NT;
+      const int end = ch < chunks_a ? nA : n;
+      const bool more = ch + 1 < chunks;
+      const int2 e = e_next;
+      if (more) {
+        const int nbase = ch + 1 < chunks_a ? (ch + 1) * NT : nA + (ch + 1 - chunks_a) * NT;
+        const int nend = ch + 1 < chunks_a ? nA : n;
+        e_next = nbase + t < nend ? bin_entry(bin, nA, bins.cap, nbase + t) : make_int2(0, 0);
+      }
+      int c = 0;
+      if (base + t < end &&
+          !skip_face(__uint_as_float(static_cast<uint32_t>(e.y) & 0xffff0000u), dmax)) {
+        const float4* r = m.soup + int64_t(e.x) * 3;
+        const float4 a = r[0], b = r[1], d = r[2];
+        s.p[0][t] = a.x; s.p[1][t] = a.y; s.p[2][t] = a.z;
+        s.p[3][t] = a.w; s.p[4][t] = b.x; s.p[5][t] = b.y;
+        s.p[6][t] = b.z; s.p[7][t] = b.w; s.p[8][t] = d.x;
+        s.fid[t] = e.x;
+        s.box[t] = static_cast<uint16_t>(e.y);
+        c = (((e.y >> 8) & 15) + 1) * (((e.y >> 12) & 15) + 1);
+      }
+      const int lane = t & 63, wid = t >> 6;
+      const int x = wave_incl_sum(c);
+      const int cmax = wave_incl_max(c);
+      if (lane == 63) {
+        s.wsum[wid] = x;
+        s.wbig[wid] = cmax;
+      }
+      if (!__syncthreads_or(c > 0)) continue;
+      int wbase = 0, total = 0, big = 0;
+      for (int w = 0; w < NT / 64; w++) {
+        if (w < wid) wbase += s.wsum[w];
+        total += s.wsum[w];
+        big = max(big, s.wbig[w]);
+      }
+      const int pre = wbase + x - c;
+      auto test_pair = [&](int j, int pix) {
+        const float3 p0 = make_float3(s.p[0][j], s.p[1][j], s.p[2][j]);
+        const float3 p1 = make_float3(s.p[3][j], s.p[4][j], s.p[5][j]);
+        const float3 p2 = make_float3(s.p[6][j], s.p[7][j], s.p[8][j]);
+        float ht, hu, hv;
+        if (mt_hit(ox, oy, oz, s.ray[0][pix], s.ray[1][pix], s.ray[2][pix], p0, p1, p2, ht, hu,
+                   hv) &&
+            ht < __builtin_huge_valf()) {
+          // + 0: a distance of -0 becomes 0, so the bits order as the floats
+          const unsigned long long key =
+              (static_cast<unsigned long long>(__float_as_uint(ht + 0.0f)) << 32) |
+              static_cast<unsigned int>(s.fid[j]);
+          atomicMin(&s.key[pix], key);
+        }
+      };
+      if (big <= kScatterMaxPairs) {
+        for (int q0 = 0; q0 < total; q0 += 2 * NT) {
+          const int lo = max(pre, q0), hi = min(pre + c, q0 + 2 * NT);
+          if (lo < hi) {
+            const int bx = s.box[t];
+            const int nx = ((bx >> 8) & 15) + 1;
+            int ry = (lo - pre) / nx;
+            int rx = (lo - pre) - ry * nx;
+            int pix = (((bx >> 4) & 15) + ry) * kRtTile + (bx & 15) + rx;
+            for (int q = lo; q < hi; q++) {
+              s.pairs[q - q0] = t | (pix << 8);
+              if (++rx == nx) {
+                rx = 0;
+                pix += kRtTile - nx + 1;
+              } else {
+                pix++;
+              }
+            }
+          }
+          __syncthreads();
+          const int np = min(total - q0, 2 * NT);
+          for (int pp = t; pp < np; pp += NT) {
+            const int pr = s.pairs[pp];
+            test_pair(pr & 0xff, pr >> 8);
+          }
+          __syncthreads();
+        }
+      } else {
+        s.pairs[t] = pre;
+        if (t == NT - 1) s.pairs[NT] = total;
+        __syncthreads();
+        for (int p = t; p < total; p += NT) {
+          int jl = 0, jh = NT - 1;
+          while (jl < jh) {
+            const int mid = (jl + jh + 1) >> 1;
+            if (s.pairs[mid] <= p) jl = mid; else jh = mid - 1;
+          }
+          const int r = p - s.pairs[jl];
+          const int bx = s.box[jl];
+          const int nx = ((bx >> 8) & 15) + 1;
+          const int qy = r / nx;
+          test_pair(jl, (((bx >> 4) & 15) + qy) * kRtTile + (bx & 15) + (r - qy * nx));
+        }
+        __syncthreads();
+      }
+      if (more) {
+        const unsigned long long k = s.key[t];
+        // depth of the pixel's hit: all ones when it has none, 0 outside the image
+        uint32_t db = 0u;
+        if (act) {
+          const uint32_t tb = static_cast<uint32_t>(k >> 32);
+          db = k == ~0ull ? 0xffffffffu : __float_as_uint(__uint_as_float(tb) * zray);
+        }
+        db = wave_max_u32(db);
+        if (lane == 0) s.wmax[wid] = db;
+        __syncthreads();
+        uint32_t mx = s.wmax[0];
+        for (int w = 1; w < NT / 64; w++) mx = max(mx, s.wmax[w]);
+        dmax = __uint_as_float(mx);
+      }
+    }
+    const unsigned long long k = s.key[t];
+    if (k != ~0ull) bf = static_cast<int>(static_cast<unsigned int>(k & 0xffffffffull));
   }
-  float n0, n1, n2;
-  FaceShade fs;
-  face_shade(m, bf, o.shading_normal != 0, v.color && o.diffuse_color == 1, fs);
-  if (o.shading_normal == 0) {
-    const float* fn = m.fnormals + int64_t(bf) * 3;
-    n0 = fn[0];
-    n1 = fn[1];
-    n2 = fn[2];
-  } else {
-    // (1 - u - v) n[i0] + u n[i1] + v n[i2] with the raytracer's (u, v)
-    const float* na = fs.na;
-    const float* nb = fs.nb;
-    const float* nc = fs.nc;
-    const float w = 1.0f - bu - bv;
-    n0 = w * na[0] + bu * nb[0] + bv * nc[0];
-    n1 = w * na[1] + bu * nb[1] + bv * nc[1];
-    n2 = w * na[2] + bu * nb[2] + bv * nc[2];
+  if (!act) return;
+  float bt = 0.0f, bu = 0.0f, bv = 0.0f;
+  if (bf >= 0) {
+    // the winner's distance and weights, by the test that accepted it
+    const float4* r = m.soup + int64_t(bf) * 3;
+    const float4 a = r[0], b = r[1], d = r[2];
+    const float3 p0 = make_float3(a.x, a.y, a.z), p1 = make_float3(a.w, b.x, b.y),
+                 p2 = make_float3(b.z, b.w, d.x);
+    mt_hit(v.c2w_t[0], v.c2w_t[1], v.c2w_t[2], r0, r1, r2, p0, p1, p2, bt, bu, bv);
   }
-  if (v.normal) {
-    v.normal[pi * 3 + 0] = sum3(v.w2c_R[0] * n0, v.w2c_R[1] * n1, v.w2c_R[2] * n2);
-    v.normal[pi * 3 + 1] = sum3(v.w2c_R[3] * n0, v.w2c_R[4] * n1, v.w2c_R[5] * n2);
-    v.normal[pi * 3 + 2] = sum3(v.w2c_R[6] * n0, v.w2c_R[7] * n1, v.w2c_R[8] * n2);
-  }
-  if (v.color) {
-    uint8_t c[3];
-    shade_u8(m, o, bf, fs, bu, bv, r0, r1, r2, n0, n1, n2, c);
-    v.color[pi * 3 + 0] = c[0];
-    v.color[pi * 3 + 1] = c[1];
-    v.color[pi * 3 + 2] = c[2];
-  }
+  write_hit<true>(v, m, o, gx, gy, bf, bt, bu, bv, r0, r1, r2);
 }
 
 // ---------------------------------------------------------------------------
@@ -350,6 +778,16 @@ int launch_visibility(hipStream_t st, const DevView& v, const uint8_t* color, co
   hipLaunchKernelGGL(k_visibility, dim3((n + 63) / 64), dim3(64), 0, st, v, color, depth, mask, o,
                      n, pos, vert, nrm, bvh.nodes, bvh.leaves, bvh.tris,
                      static_cast<DevVisItem*>(out));
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+// views[i].tile_base = first 16x16 tile of view i; the bins' counters cleared
+int launch_raytrace_binned(hipStream_t st, const DevView* views, int n_views, const DevMesh& m,
+                           const DevBins& bins, const DevOptions& o) {
+  if (n_views < 1 || bins.total_tiles < 1 || m.F < 1) return 0;
+  const dim3 grid((m.F + 255) / 256, (n_views + kSetupViews - 1) / kSetupViews);
+  hipLaunchKernelGGL(k_rt_setup, grid, dim3(256), 0, st, views, n_views, m, bins);
+  hipLaunchKernelGGL(k_rt_tiles, dim3(bins.total_tiles), dim3(256), 0, st, views, m, bins, o);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
