@@ -14,7 +14,6 @@
 //                 packed 64-bit (depth bits << 32 | face id) LDS atomicMin,
 //                 then shades and writes every output pixel of the tile once
 //                 (resolve loop rasterizer.cc:243-301, pixel_shader.h).
-//   k_bwd_*       differentiable backward pass (no reference counterpart).
 //
 // Bit-exactness: all coverage arithmetic follows the reference's expression
 // order; this file is compiled with -ffp-contract=off and correctly rounded
@@ -1145,428 +1144,6 @@ __global__ __launch_bounds__(TW * TH, MODE == 0 ? 7 : 6) void k_raster(
 }
 
 // ---------------------------------------------------------------------------
-// Differentiable backward pass: dL/d(vertices, vertex colours, texture) at
-// fixed visibility. The covered pixels of all views are sorted by face id
-// into (face, view, pixel) items with a counting sort:
-//   k_bwd_count    one thread per pixel: per-face pixel counts
-//   k_scan_*       exclusive scan of the counts (face offsets, item total)
-//   k_bwd_scatter  one thread per pixel: item at offset + (count - 1), the
-//                  counts decrement back to zero
-//   k_bwd_items    one thread per item: shading derivatives in float64;
-//                  contributions of contiguous items of one face (all its
-//                  pixels in every view) are summed across the wavefront,
-//                  then one atomic per vertex component and run
-// Grouping by face turns a face's gradient into a handful of atomics instead
-// of one set per pixel.
-
-__global__ void k_zero_i32(int32_t* p, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) p[i] = 0;
-}
-
-// face 0 is never shaded (rasterizer.cc:250), so it has no gradient
-// Runs of equal face ids among a wavefront's consecutive pixels: `head` for
-// the first lane of a run, `first` = that lane, `len` = the run's length (in
-// the head lane). Lanes without a face form runs of their own.
-struct FaceRun {
-  bool head;
-  int first, len;
-};
-
-UGU_DEV FaceRun face_run(int key) {
-  const int lane = __lane_id();
-  const int prev = wave_prev(key, key);
-  FaceRun r;
-  r.head = lane == 0 || prev != key;
-  const uint64_t heads = __ballot(r.head);
-  const uint64_t upto = heads & ((2ull << lane) - 1ull);
-  r.first = 63 - __clzll(static_cast<long long>(upto));
-  const uint64_t after = heads & ~((2ull << lane) - 1ull);
-  r.len = (after ? __ffsll(static_cast<unsigned long long>(after)) - 1 : 64) - lane;
-  return r;
-}
-
-// One thread per pixel; one atomic per run of equal face ids.
-__global__ __launch_bounds__(256) void k_bwd_count(const DevView* __restrict__ views,
-                                                   int32_t F, int32_t* __restrict__ cnt) {
-  const DevView& v = views[blockIdx.y];
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (int64_t(blockIdx.x) * blockDim.x >= int64_t(v.W) * v.H) return;  // whole block idle
-  const int fid = p < v.W * v.H ? v.face_id[p] : 0;
-  const bool valid = fid > 0 && fid < F;
-  const FaceRun r = face_run(valid ? fid : -1 - __lane_id());
-  if (valid && r.head) atomicAdd(&cnt[fid], r.len);
-}
-
-// One thread per pixel: the run's head takes len slots from the face's
-// counter (which counts back down to zero); lane j of the run writes slot
-// base - 1 - j of the face's range.
-__global__ __launch_bounds__(256) void k_bwd_scatter(const DevView* __restrict__ views,
-                                                     int32_t F, const int32_t* __restrict__ off,
-                                                     int32_t* __restrict__ cnt,
-                                                     int4* __restrict__ items) {
-  const DevView& v = views[blockIdx.y];
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (int64_t(blockIdx.x) * blockDim.x >= int64_t(v.W) * v.H) return;  // whole block idle
-  const int fid = p < v.W * v.H ? v.face_id[p] : 0;
-  const bool valid = fid > 0 && fid < F;
-  const FaceRun r = face_run(valid ? fid : -1 - __lane_id());
-  int base = 0;
-  if (valid && r.head) base = atomicAdd(&cnt[fid], -r.len);
-  base = __shfl(base, r.first);
-  if (valid) items[off[fid] + base - 1 - (__lane_id() - r.first)] = make_int4(fid, blockIdx.y, p, 0);
-}
-
-// Exclusive scan of n counters (n + 1 outputs, out[n] = total) in three
-// kernels: per-block scans of 4096 values, a scan of the block sums, the add.
-constexpr int kScanBlock = 4096;
-
-__global__ __launch_bounds__(1024) void k_scan_blocks(const int32_t* __restrict__ in, int n,
-                                                      int32_t* __restrict__ out,
-                                                      int32_t* __restrict__ sums) {
-  __shared__ int32_t wsum[16];
-  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
-  const int64_t b0 = int64_t(blockIdx.x) * kScanBlock + t * 4;
-  int v[4], tot = 0;
-  for (int k = 0; k < 4; k++) {
-    v[k] = b0 + k < n ? in[b0 + k] : 0;
-    tot += v[k];
-  }
-  const int x = wave_incl_sum(tot);
-  if (lane == 63) wsum[wid] = x;
-  __syncthreads();
-  int base = 0, all = 0;
-  for (int w = 0; w < 16; w++) {
-    if (w < wid) base += wsum[w];
-    all += wsum[w];
-  }
-  base += x - tot;
-  for (int k = 0; k < 4; k++) {
-    if (b0 + k < n) out[b0 + k] = base;
-    base += v[k];
-  }
-  if (t == 0) sums[blockIdx.x] = all;
-}
-
-// one block: exclusive scan of the block sums in place, total in sums[nb]
-__global__ __launch_bounds__(1024) void k_scan_sums(int32_t* __restrict__ sums, int nb) {
-  __shared__ int32_t wsum[16];
-  __shared__ int32_t carry;
-  const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
-  if (t == 0) carry = 0;
-  __syncthreads();
-  for (int c0 = 0; c0 < nb; c0 += 1024) {
-    const int val = c0 + t < nb ? sums[c0 + t] : 0;
-    const int x = wave_incl_sum(val);
-    if (lane == 63) wsum[wid] = x;
-    __syncthreads();
-    int base = carry, all = 0;
-    for (int w = 0; w < 16; w++) {
-      if (w < wid) base += wsum[w];
-      all += wsum[w];
-    }
-    if (c0 + t < nb) sums[c0 + t] = base + x - val;
-    __syncthreads();
-    if (t == 0) carry += all;
-    __syncthreads();
-  }
-  if (t == 0) sums[nb] = carry;
-}
-
-__global__ void k_scan_add(int32_t* __restrict__ out, int n, const int32_t* __restrict__ sums,
-                           int nb) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i < n) out[i] += sums[i / kScanBlock];
-  if (i == 0) out[n] = sums[nb];
-}
-
-
-// Texel gradients of a block's items are first summed in an LDS hash table
-// (open addressing on the texel index, linear probing); a block's items cover
-// a few faces in every view that sees them, so many items hit the same texels.
-// Texels that find no free slot go straight to global atomics.
-constexpr int kTexSlots = 2048;
-constexpr int kTexProbes = 8;
-
-UGU_DEV int tex_slot(int key) {
-  return static_cast<int>((static_cast<uint32_t>(key) * 2654435761u) >> 21);  // 11 bits
-}
-
-// Items per thread of k_bwd_items: a block handles kBwdRounds x 256
-// consecutive items (round r: items r*256 .. r*256+255 of the block's range,
-// so each wavefront sees consecutive items) and merges the texel gradients
-// of all of them in its LDS table before the global atomics.
-constexpr int kBwdRounds = 4;
-
-// Geometry of the image model at one pixel of a face, in float64 (the values
-// diff_eval computes): screen positions, inverse camera depths and camera x, y
-// of the corners, the edge functions' quotients q_i = e_i / (A Z_i), 1 / A,
-// 1 / (q0 + q1 + q2) and the weights b1, b2 of the second and third corner.
-struct DiffGeo {
-  double X[3], Y[3], iZ[3], Qx[3], Qy[3], q[3], iA, is, b1, b2;
-};
-
-UGU_DEV void diff_geo(const DevView& v, const float* __restrict__ verts, const int32_t* vid,
-                      int px, int py, DiffGeo& e) {
-  for (int i = 0; i < 3; i++) {
-    const float* P = verts + int64_t(vid[i]) * 3;
-    double Q[3];
-    for (int r = 0; r < 3; r++)
-      Q[r] = double(v.w2c_R[r * 3 + 0]) * P[0] + double(v.w2c_R[r * 3 + 1]) * P[1] +
-             double(v.w2c_R[r * 3 + 2]) * P[2] + double(v.w2c_t[r]);
-    e.Qx[i] = Q[0];
-    e.Qy[i] = Q[1];
-    e.iZ[i] = 1.0 / Q[2];
-    e.X[i] = double(v.fx) * Q[0] * e.iZ[i] + double(v.cx);
-    e.Y[i] = double(v.fy) * Q[1] * e.iZ[i] + double(v.cy);
-  }
-  auto E = [](double ax, double ay, double bx, double by, double cx, double cy) {
-    return (cx - ax) * (by - ay) - (cy - ay) * (bx - ax);
-  };
-  const double x = px, y = py;
-  const double A = E(e.X[0], e.Y[0], e.X[1], e.Y[1], e.X[2], e.Y[2]);
-  e.iA = 1.0 / A;
-  e.q[0] = E(e.X[1], e.Y[1], e.X[2], e.Y[2], x, y) * e.iA * e.iZ[0];
-  e.q[1] = E(e.X[2], e.Y[2], e.X[0], e.Y[0], x, y) * e.iA * e.iZ[1];
-  e.q[2] = E(e.X[0], e.Y[0], e.X[1], e.Y[1], x, y) * e.iA * e.iZ[2];
-  e.is = 1.0 / (e.q[0] + e.q[1] + e.q[2]);
-  e.b1 = e.q[1] * e.is;
-  e.b2 = e.q[2] * e.is;
-}
-
-// One thread per item. The work is ordered so that few float64 values are
-// live at a time (the kernel is bound by the latency of its gathers, so
-// registers buy occupancy): the weights, then the colour and texture terms
-// channel by channel into the colour and texel gradients and dL/du, dL/dv,
-// whose atomics are issued next; the geometry is then evaluated again for the
-// position gradients.
-__global__ __launch_bounds__(256) void k_bwd_items(
-    const DevView* __restrict__ views, DevMesh mesh, const int4* __restrict__ items,
-    const int32_t* __restrict__ cursor, DevGrads g) {
-  static_assert(kTexSlots == 2048, "tex_slot returns 11 bits");
-  __shared__ int32_t hkey[kTexSlots];
-  __shared__ float hval[3][kTexSlots];
-  const int n_items = *cursor;
-  const int64_t first = int64_t(blockIdx.x) * blockDim.x * kBwdRounds;
-  if (first >= n_items) return;  // whole block idle
-  const bool tex = g.texture && mesh.ftex;  // uniform over the block
-  if (tex) {
-    for (int j = threadIdx.x; j < kTexSlots; j += blockDim.x) {
-      hkey[j] = -1;
-      hval[0][j] = hval[1][j] = hval[2][j] = 0.0f;
-    }
-    __syncthreads();
-  }
-  for (int round = 0; round < kBwdRounds; round++) {
-  const int64_t i = first + int64_t(round) * blockDim.x + threadIdx.x;
-  const bool valid = i < n_items;
-  int4 item = make_int4(-1, 0, 0, 0);
-  if (valid) item = items[i];
-  const int fid = item.x;
-  int vid[3] = {0, 0, 0};
-  double gu = 0.0, gv = 0.0, b1 = 0.0, b2 = 0.0;
-  int px = 0, py = 0;
-  const DevView* vp = views;
-
-  // ---- colour and texture terms: dL/dC, dL/dT and dL/du, dL/dv
-  // (dL/dc = G t, dL/dt = G c; u = b1, v = b2, b0 = 1 - u - v)
-  {
-    float gcol[9], gtex[12];
-    for (int k = 0; k < 9; k++) gcol[k] = 0.0f;
-    for (int k = 0; k < 12; k++) gtex[k] = 0.0f;
-    int tx0 = 0, ty0 = 0, tx1 = 0, ty1 = 0;
-    if (valid) {
-      vp = views + item.y;
-      const DevView& v = *vp;
-      const int p = item.z;
-      px = p % v.W;
-      py = p / v.W;
-      const int32_t* fi = mesh.faces + int64_t(fid) * 3;
-      vid[0] = fi[0]; vid[1] = fi[1]; vid[2] = fi[2];
-      const float* gp = v.grad + int64_t(p) * 3;
-      const double G[3] = {gp[0], gp[1], gp[2]};
-      {
-        DiffGeo e;
-        diff_geo(v, mesh.verts, vid, px, py, e);
-        b1 = e.b1;
-        b2 = e.b2;
-      }
-      const double b0 = 1.0 - b1 - b2;
-      const float *C0 = nullptr, *C1 = nullptr, *C2 = nullptr;
-      if (mesh.vcolors) {
-        C0 = mesh.vcolors + int64_t(vid[0]) * 3;
-        C1 = mesh.vcolors + int64_t(vid[1]) * 3;
-        C2 = mesh.vcolors + int64_t(vid[2]) * 3;
-      }
-      double lu = 0.0, lv = 0.0, dlu_du = 0.0, dlu_dv = 0.0, dlv_du = 0.0, dlv_dv = 0.0;
-      const float *p00 = nullptr, *p01 = nullptr, *p10 = nullptr, *p11 = nullptr;
-      if (mesh.ftex) {
-        const int32_t* ui = mesh.uvidx + int64_t(fid) * 3;
-        const float* a = mesh.uv + int64_t(ui[0]) * 2;
-        const float* b = mesh.uv + int64_t(ui[1]) * 2;
-        const float* c = mesh.uv + int64_t(ui[2]) * 2;
-        const double iu = b0 * a[0] + b1 * b[0] + b2 * c[0];
-        const double iv = b0 * a[1] + b1 * b[1] + b2 * c[1];
-        const int tw = mesh.ftex_w, th = mesh.ftex_h;
-        const double fxp = iu * (tw - 1), fyp = (1.0 - iv) * (th - 1);
-        const double flx = floor(fxp), fly = floor(fyp);
-        lu = fxp - flx;
-        lv = fyp - fly;
-        tx0 = clamp_texel(flx, tw - 1);
-        ty0 = clamp_texel(fly, th - 1);
-        tx1 = clamp_texel(flx + 1.0, tw - 1);
-        ty1 = clamp_texel(fly + 1.0, th - 1);
-        p00 = mesh.ftex + (int64_t(ty0) * tw + tx0) * 3;
-        p01 = mesh.ftex + (int64_t(ty0) * tw + tx1) * 3;
-        p10 = mesh.ftex + (int64_t(ty1) * tw + tx0) * 3;
-        p11 = mesh.ftex + (int64_t(ty1) * tw + tx1) * 3;
-        const double sx = tw - 1, sy = -(th - 1.0);
-        dlu_du = sx * (double(b[0]) - a[0]);
-        dlu_dv = sx * (double(c[0]) - a[0]);
-        dlv_du = sy * (double(b[1]) - a[1]);
-        dlv_dv = sy * (double(c[1]) - a[1]);
-      }
-      const double wq[4] = {(1 - lu) * (1 - lv), lu * (1 - lv), (1 - lu) * lv, lu * lv};
-      for (int k = 0; k < 3; k++) {
-        double cc = 1.0, dcdu = 0.0, dcdv = 0.0;
-        if (C0) {
-          cc = b0 * C0[k] + b1 * C1[k] + b2 * C2[k];
-          dcdu = double(C1[k]) - C0[k];
-          dcdv = double(C2[k]) - C0[k];
-        }
-        double t = 1.0, dtdu = 0.0, dtdv = 0.0;
-        if (p00) {
-          t = wq[0] * p00[k] + wq[1] * p01[k] + wq[2] * p10[k] + wq[3] * p11[k];
-          const double da = (1 - lv) * (double(p01[k]) - p00[k]) + lv * (double(p11[k]) - p10[k]);
-          const double db = (1 - lu) * (double(p10[k]) - p00[k]) + lu * (double(p11[k]) - p01[k]);
-          dtdu = da * dlu_du + db * dlv_du;
-          dtdv = da * dlu_dv + db * dlv_dv;
-        }
-        const double gc = G[k] * t, gt = G[k] * cc;
-        gcol[0 * 3 + k] = static_cast<float>(gc * b0);
-        gcol[1 * 3 + k] = static_cast<float>(gc * b1);
-        gcol[2 * 3 + k] = static_cast<float>(gc * b2);
-        for (int q = 0; q < 4; q++) gtex[q * 3 + k] = static_cast<float>(gt * wq[q]);
-        gu += gc * dcdu + gt * dtdu;
-        gv += gc * dcdv + gt * dtdv;
-      }
-    }
-
-    // wavefront pre-reduction over runs of equal face id, then atomics
-    // from each run's last lane
-    const int lane = __lane_id();
-    const int prev_fid = wave_prev(fid, INT_MIN);
-    const int next_fid = wave_next(fid, INT_MIN);
-    const bool head = valid && (lane == 0 || prev_fid != fid);
-    const bool tail = valid && (lane == 63 || next_fid != fid);
-    const uint64_t heads = __ballot(head);
-    const uint64_t vmask = __ballot(valid);
-    const bool reduce = heads != vmask;  // some run longer than one lane
-    const int run = valid ? __popcll(heads & ((2ull << lane) - 1ull)) : -1 - lane;
-    if (g.colors && mesh.vcolors) {
-      for (int k = 0; k < 9; k++) {
-        const float val = reduce ? run_sum(gcol[k], run) : gcol[k];
-        if (tail) unsafeAtomicAdd(&g.colors[int64_t(vid[k / 3]) * 3 + (k % 3)], val);
-      }
-    }
-    if (tex && valid) {
-      const int tw = mesh.ftex_w;
-      const int tidx[4] = {ty0 * tw + tx0, ty0 * tw + tx1, ty1 * tw + tx0, ty1 * tw + tx1};
-      for (int q = 0; q < 4; q++) {
-        const int key = tidx[q];
-        int h = tex_slot(key);
-        bool done = false;
-        for (int probe = 0; probe < kTexProbes && !done; probe++) {
-          const int old = atomicCAS(&hkey[h], -1, key);
-          if (old == -1 || old == key) {
-            for (int k = 0; k < 3; k++) atomicAdd(&hval[k][h], gtex[q * 3 + k]);
-            done = true;
-          }
-          h = (h + 1) & (kTexSlots - 1);
-        }
-        if (!done)
-          for (int k = 0; k < 3; k++)
-            unsafeAtomicAdd(&g.texture[int64_t(key) * 3 + k], gtex[q * 3 + k]);
-      }
-    }
-  }
-
-  // ---- positions (the geometry again): b_i = q_i / s
-  if (g.verts) {
-    float gpos[9];
-    for (int k = 0; k < 9; k++) gpos[k] = 0.0f;
-    if (valid) {
-      const DevView& v = *vp;
-      DiffGeo e;
-      diff_geo(v, mesh.verts, vid, px, py, e);
-      // dL/dq_j = (dL/db_j - (gu b1 + gv b2)) / s
-      const double S = gu * b1 + gv * b2;
-      const double gq[3] = {-S * e.is, (gu - S) * e.is, (gv - S) * e.is};
-      // q_j = e_j / (A Z_j)
-      double ge[3], gZ[3], gA = 0.0;
-      for (int j = 0; j < 3; j++) {
-        ge[j] = gq[j] * e.iA * e.iZ[j];
-        gZ[j] = -gq[j] * e.q[j] * e.iZ[j];
-        gA -= gq[j] * e.q[j] * e.iA;
-      }
-      // E(a,b,c): dE/da = (c.y-b.y, b.x-c.x), dE/db = (a.y-c.y, c.x-a.x),
-      //           dE/dc = (b.y-a.y, a.x-b.x)
-      // e0 = E(v1, v2, p), e1 = E(v2, v0, p), e2 = E(v0, v1, p), A = E(v0, v1, v2)
-      double gX[3] = {0, 0, 0}, gY[3] = {0, 0, 0};
-      const double x = px, y = py;
-      const int ea[3] = {1, 2, 0}, eb[3] = {2, 0, 1};
-      for (int j = 0; j < 3; j++) {
-        const int ia = ea[j], ib = eb[j];
-        gX[ia] += ge[j] * (y - e.Y[ib]);
-        gY[ia] += ge[j] * (e.X[ib] - x);
-        gX[ib] += ge[j] * (e.Y[ia] - y);
-        gY[ib] += ge[j] * (x - e.X[ia]);
-      }
-      gX[0] += gA * (e.Y[2] - e.Y[1]);
-      gY[0] += gA * (e.X[1] - e.X[2]);
-      gX[1] += gA * (e.Y[0] - e.Y[2]);
-      gY[1] += gA * (e.X[2] - e.X[0]);
-      gX[2] += gA * (e.Y[1] - e.Y[0]);
-      gY[2] += gA * (e.X[0] - e.X[1]);
-      // X = fx Qx / Qz + cx, Y = fy Qy / Qz + cy, Z = Qz; Q = R P + t
-      for (int j = 0; j < 3; j++) {
-        const double iz = e.iZ[j];
-        const double gQx = gX[j] * v.fx * iz;
-        const double gQy = gY[j] * v.fy * iz;
-        const double gQz = gZ[j] - gX[j] * v.fx * e.Qx[j] * iz * iz -
-                           gY[j] * v.fy * e.Qy[j] * iz * iz;
-        for (int cdim = 0; cdim < 3; cdim++)
-          gpos[j * 3 + cdim] = static_cast<float>(double(v.w2c_R[0 * 3 + cdim]) * gQx +
-                                                  double(v.w2c_R[1 * 3 + cdim]) * gQy +
-                                                  double(v.w2c_R[2 * 3 + cdim]) * gQz);
-      }
-    }
-    const int lane = __lane_id();
-    const int prev_fid = wave_prev(fid, INT_MIN);
-    const int next_fid = wave_next(fid, INT_MIN);
-    const bool head = valid && (lane == 0 || prev_fid != fid);
-    const bool tail = valid && (lane == 63 || next_fid != fid);
-    const uint64_t heads = __ballot(head);
-    const uint64_t vmask = __ballot(valid);
-    const bool reduce = heads != vmask;
-    const int run = valid ? __popcll(heads & ((2ull << lane) - 1ull)) : -1 - lane;
-    for (int k = 0; k < 9; k++) {
-      const float val = reduce ? run_sum(gpos[k], run) : gpos[k];
-      if (tail) unsafeAtomicAdd(&g.verts[int64_t(vid[k / 3]) * 3 + (k % 3)], val);
-    }
-  }
-  }  // rounds
-  if (tex) {
-    __syncthreads();
-    for (int j = threadIdx.x; j < kTexSlots; j += blockDim.x) {
-      const int key = hkey[j];
-      if (key >= 0)
-        for (int k = 0; k < 3; k++) unsafeAtomicAdd(&g.texture[int64_t(key) * 3 + k], hval[k][j]);
-    }
-  }
-}
-
-// ---------------------------------------------------------------------------
 // RenderW depth conversion: uint16(1.0 * (double)d), truncating as x86 does.
 __global__ void k_depth_to_u16(const float* __restrict__ d, int64_t n,
                                uint16_t* __restrict__ out) {
@@ -1664,36 +1241,6 @@ int raster_blocks_per_cu(int tw, int th, int mode) {
   UGU_OCC_CASE(32, 8)
 #undef UGU_OCC_CASE
   return e == hipSuccess ? nb : 0;
-}
-
-// Scratch of the backward pass: cnt (F + 1), off (F + 1) and the block sums.
-int64_t backward_scratch_ints(int32_t F) {
-  return 2 * (int64_t(F) + 1) + (int64_t(F) + kScanBlock - 1) / kScanBlock + 1;
-}
-
-int launch_backward(hipStream_t st, const DevView* views, int n_views,
-                    int max_pixels, int64_t total_pixels, const DevMesh& mesh,
-                    const DevGrads& g, int4* items, int32_t* scratch, hipEvent_t before_items) {
-  if (max_pixels <= 0 || total_pixels <= 0 || mesh.F <= 0) return 0;
-  const int F = mesh.F;
-  int32_t* cnt = scratch;
-  int32_t* off = scratch + (F + 1);
-  int32_t* sums = off + (F + 1);
-  const int nb = (F + kScanBlock - 1) / kScanBlock;
-  const dim3 pgrid((max_pixels + 255) / 256, n_views);
-  hipLaunchKernelGGL(k_zero_i32, dim3((F + 256) / 256), dim3(256), 0, st, cnt, F + 1);
-  hipLaunchKernelGGL(k_bwd_count, pgrid, dim3(256), 0, st, views, F, cnt);
-  hipLaunchKernelGGL(k_scan_blocks, dim3(nb), dim3(1024), 0, st, cnt, F, off, sums);
-  hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(1024), 0, st, sums, nb);
-  hipLaunchKernelGGL(k_scan_add, dim3((F + 255) / 256), dim3(256), 0, st, off, F, sums, nb);
-  hipLaunchKernelGGL(k_bwd_scatter, pgrid, dim3(256), 0, st, views, F, off, cnt, items);
-  if (before_items) (void)hipEventRecord(before_items, st);
-  // at most one item per pixel; blocks past the item count (off[F]) exit at once
-  hipLaunchKernelGGL(k_bwd_items,
-                     dim3(static_cast<unsigned>((total_pixels + 256 * kBwdRounds - 1) /
-                                                (256 * kBwdRounds))),
-                     dim3(256), 0, st, views, mesh, items, off + F, g);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int launch_depth_to_u16(hipStream_t st, const float* d, int64_t n, uint16_t* out) {

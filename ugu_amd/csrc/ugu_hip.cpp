@@ -33,10 +33,11 @@ int launch_raster(hipStream_t st, int tw, int th, int mode, const DevView* views
                   const DevMesh& mesh, const DevBins& bins,
                   const DevOptions& opt, int persistent_blocks);
 int raster_blocks_per_cu(int tw, int th, int mode);
-int64_t backward_scratch_ints(int32_t F);
-int launch_backward(hipStream_t st, const DevView* views, int n_views,
-                    int max_pixels, int64_t total_pixels, const DevMesh& mesh,
-                    const DevGrads& g, int4* items, int32_t* scratch, hipEvent_t before_items);
+int64_t backward_scratch_ints();
+int64_t backward_total_at(int32_t F);
+int launch_backward(hipStream_t st, const DevView* views, int n_views, int max_squares,
+                    int64_t total_pixels, const DevMesh& mesh, const DevGrads& g, int4* items,
+                    int32_t* scratch, hipEvent_t before_items);
 int launch_depth_to_u16(hipStream_t st, const float* d, int64_t n, uint16_t* out);
 int launch_raytrace(hipStream_t st, const DevView* views, int n_views, int total_tiles,
                     const DevBvh& bvh, const DevMesh& m, const DevOptions& o);
@@ -168,7 +169,8 @@ struct ugu_hip_ctx {
   // work buffers
   DevBuf counts, bins, status, views, tile_base, stage_out, diff_fn;
   DevBuf bwd_items;  // (face, view, pixel) items of the backward pass, 16 B each
-  DevBuf bwd_scratch;  // per-face counts and offsets of the backward pass
+  DevBuf bwd_scratch;  // face group counts and cursors of the backward pass
+  bool bwd_zeroed = false;  // the counts are zero (every completed pass leaves them so)
   DevBuf soup, diff_soup;  // 48-byte face records (prepared mesh / differentiable path)
   DevBuf shade;            // 64-byte per-face shading records (DevMesh::shade)
   TexInfo tex0{};          // host copy of the first material's TexInfo
@@ -1765,7 +1767,7 @@ int ugu_hip_diff_backward(ugu_hip_ctx* c, const UguCamera* cams, int n,
   DevMesh dm;
   int err = diff_mesh(c, p, &dm);
   if (err) return err;
-  int max_px = 0;
+  int max_squares = 0;  // 16 x 16 pixel squares of the largest view
   int64_t total_px = 0;
   if ((err = ensure(c, c->views, size_t(n) * sizeof(DevView)))) return err;
   const size_t view_bytes = size_t(n) * sizeof(DevView) + size_t(n + 1) * 4;
@@ -1793,12 +1795,16 @@ int ugu_hip_diff_backward(ugu_hip_ctx* c, const UguCamera* cams, int n,
     std::memcpy(v.c2w_R, cams[i].c2w_R, sizeof(v.c2w_R));
     v.face_id = const_cast<int32_t*>(face_ids[i]);
     v.grad = grad_images[i];
-    max_px = std::max(max_px, v.W * v.H);
+    max_squares = std::max(max_squares, ((v.W + 15) / 16) * ((v.H + 15) / 16));
     total_px += int64_t(v.W) * v.H;
   }
   if (total_px > INT32_MAX) return fail(c, UGU_HIP_ERR_INVALID_ARGUMENT, "too many pixels");
   if ((err = ensure(c, c->bwd_items, size_t(total_px) * 16))) return err;
-  if ((err = ensure(c, c->bwd_scratch, size_t(backward_scratch_ints(dm.F)) * 4))) return err;
+  const size_t scratch_bytes = size_t(backward_scratch_ints()) * 4;
+  if ((err = ensure(c, c->bwd_scratch, scratch_bytes))) return err;
+  if (!c->bwd_zeroed)
+    UGU_HIP_CHECK(c, hipMemsetAsync(c->bwd_scratch.p, 0, scratch_bytes, c->stream));
+  c->bwd_zeroed = false;  // until this pass has completed
   UGU_HIP_CHECK(c, hipMemcpyAsync(c->views.p, c->h_views, size_t(n) * sizeof(DevView),
                                   hipMemcpyHostToDevice, c->stream));
   const DevView* dv = c->views.as<DevView>();
@@ -1807,17 +1813,18 @@ int ugu_hip_diff_backward(ugu_hip_ctx* c, const UguCamera* cams, int n,
   g.colors = p->vertex_colors ? grad_vertex_colors : nullptr;
   g.texture = p->texture ? grad_texture : nullptr;
   if (c->profile) (void)hipEventRecord(c->ev[4], c->stream);
-  if (launch_backward(c->stream, dv, n, max_px, total_px, dm, g, c->bwd_items.as<int4>(),
+  if (launch_backward(c->stream, dv, n, max_squares, total_px, dm, g, c->bwd_items.as<int4>(),
                       c->bwd_scratch.as<int32_t>(), c->profile ? c->ev[5] : nullptr))
     return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
   if (c->profile) {
     // item total (the scan's last offset) and the two phases' times
     (void)hipEventRecord(c->ev[3], c->stream);
     UGU_HIP_CHECK(c, hipMemcpyAsync(c->h_status + 4,
-                                    c->bwd_scratch.as<int32_t>() + (int64_t(dm.F) + 1) + dm.F, 4,
+                                    c->bwd_scratch.as<int32_t>() + backward_total_at(dm.F), 4,
                                     hipMemcpyDeviceToHost, c->stream));
   }
   UGU_HIP_CHECK(c, hipStreamSynchronize(c->stream));
+  c->bwd_zeroed = true;
   if (c->profile) {
     float a = 0.0f, b = 0.0f;
     (void)hipEventElapsedTime(&a, c->ev[4], c->ev[5]);
