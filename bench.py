@@ -4,7 +4,7 @@
 Headline workload (default): the 1,310,720-face perturbed icosphere (subdivision
 level 8, 2048x2048 RGB8 texture, bilinear, vertex normals, back-face culling)
 rendered from 64 ring cameras of mixed resolution (320x240 .. 1920x1080) in
-one batched pipeline (one hipGraph replay per step), all five outputs written
+one batched pipeline, all five outputs written
 to device memory. A step = one forward render of the 64 views; inputs are
 resident in HBM before timing starts.
 
@@ -398,7 +398,7 @@ def main():
         tiling = r.get_tiling()
     log(f"tiling {tiling}")
 
-    # ---- headline: batched 64-view forward (graph replay), called through a
+    # ---- headline: batched 64-view forward, called through a
     # binding of the output tensors (arguments marshalled once, as a C/C++
     # caller of ugu_hip_render_batch passes them); render_device, which
     # rebuilds the ctypes arguments every call, is timed beside it

@@ -211,15 +211,15 @@ int ugu_hip_render(ugu_hip_ctx* ctx, const UguCamera* camera,
                    int memory);
 
 /* Render n views of possibly different resolutions in one batched pipeline
- * (clear, setup+bin, raster launched back to back, captured once in a
- * hipGraph and replayed). outputs[i] belongs to cameras[i]. Results are
- * bitwise identical to n separate ugu_hip_render calls. */
+ * (begin, setup+bin, raster launched back to back). outputs[i] belongs to
+ * cameras[i]. Results are bitwise identical to n separate ugu_hip_render
+ * calls. */
 int ugu_hip_render_batch(ugu_hip_ctx* ctx, const UguCamera* cameras, int n,
                          const UguOptions* options, const UguOutputs* outputs,
                          int memory);
 
-/* Same as ugu_hip_render_batch without the graph: the per-kernel launches are
- * issued directly on the stream (used for per-kernel timing). */
+/* Same as ugu_hip_render_batch (whose launches were once replayed as a graph,
+ * which took longer than issuing them). */
 int ugu_hip_render_batch_eager(ugu_hip_ctx* ctx, const UguCamera* cameras,
                                int n, const UguOptions* options,
                                const UguOutputs* outputs, int memory);
@@ -239,7 +239,7 @@ int ugu_hip_render_batch_eager(ugu_hip_ctx* ctx, const UguCamera* cameras,
  * more faces than the array can give each tile of that view. Calls on one
  * GPU share the array: the library serialises them within a process; any
  * other overlapping use on the GPU would race. The context's tiling is used
- * as by ugu_hip_render_batch; kernels are launched directly (no graph). */
+ * as by ugu_hip_render_batch. */
 int ugu_hip_render_batch_noalloc(ugu_hip_ctx* ctx, const UguCamera* cameras,
                                  int n, const UguOptions* options,
                                  const UguOutputs* outputs);

@@ -341,6 +341,23 @@ UGU_DEV void shade_u8(const DevMesh& m, const DevOptions& o, int fid, const Face
   }
 }
 
+// Copies the first n_views descriptors of a kernel's InlineViews argument, which
+// must be its first, to device memory: read as words, lane by lane, from the
+// argument segment.
+UGU_DEV void store_inline_views(DevView* out, int n_views) {
+  static_assert(sizeof(DevView) % 4 == 0, "copied as words");
+  typedef const __attribute__((address_space(4))) uint32_t* arg_words;
+  arg_words w = (arg_words)__builtin_amdgcn_kernarg_segment_ptr();
+  const int n = n_views * static_cast<int>(sizeof(DevView) / 4);
+  for (int k = threadIdx.x; k < n; k += blockDim.x) reinterpret_cast<uint32_t*>(out)[k] = w[k];
+}
+
+UGU_DEV void clear_status(int32_t* status) {
+  const int t = threadIdx.x;
+  if (t < 4) status[t] = 0;
+  if (t < kQueues) status[kQueueStride * (t + 1)] = 0;
+}
+
 UGU_DEV int xcd_remap(int b, int nb) {
   // Blocks are dispatched round-robin over the 8 XCDs; give each XCD a
   // contiguous run of tiles so neighbouring tiles share its L2.

@@ -2,7 +2,7 @@
 //
 // Pipeline for a batch of views (a single view is a batch of one):
 //   k_face_soup   48-byte face records (positions, face normal) per mesh
-//   k_clear       zero per-tile bin counters and the status words
+//   k_begin       view descriptors, per-tile bin counters and status words
 //   k_setup_bin   per-face setup of the face loop (rasterizer.cc:162-193):
 //                 z<0 reject, bbox, off-screen cull, pixel bbox, area; then
 //                 appends (face id, skip depth) to the front or back segment
@@ -139,24 +139,43 @@ UGU_DEV bool cover_test(float ax, float ay, float az, float bx, float by,
 // ---------------------------------------------------------------------------
 // k_clear
 
-// Four words per tile: front and back segment counters and the minimum skip
-// depth of the back segment. The fourth word holds the tile's view (largest v
-// with tile_base[v] <= tile), so the rasterizer reads its counters and finds
-// its view with one load.
-__global__ void k_clear(int32_t* counts, int32_t n, int32_t* status,
-                        const int32_t* __restrict__ tile_base, int32_t n_views) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) {
-    int lo = 0, hi = n_views - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi + 1) >> 1;
-      if (tile_base[mid] <= i) lo = mid; else hi = mid - 1;
+// Starts a pass: clears the tiles' counters and the status words and, with
+// N > 0, writes the view descriptors it got as arguments to device memory (one
+// launch in place of a host copy and a clear: the copy's start and the wait
+// between it and the next kernel cost more than either).
+// Four words per tile: front and back segment counters, the minimum skip depth
+// of the back segment (bits; +inf) and the tile's view (largest v with
+// views[v].tile_base <= tile), so the tile kernels read their counters and find
+// their view with one load. The tile kernels put the first three words back, so
+// a pass of one view (view word 0) needs no clearing when the counters it uses
+// were left by such passes: its setup kernel takes the descriptor and clears the
+// status. 32 k faces at 640x480: 93 us with two copies, a clear and a status
+// copy around setup and raster, 75 us with this kernel and the status in a
+// pinned word, 69 us without it.
+template <int N>
+__global__ __launch_bounds__(256) void k_begin(InlineViews<N == 0 ? 1 : N> arg,
+                                               const DevView* __restrict__ views, DevView* out,
+                                               int32_t n_views, int32_t* counts, int32_t n_tiles,
+                                               int32_t* status) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n_tiles) {
+    int view = 0;
+    if (N > 0) {
+#pragma unroll
+      for (int k = 1; k < N; k++) view = (k < n_views && arg.v[k].tile_base <= i) ? k : view;
+    } else {
+      int hi = n_views - 1;
+      while (view < hi) {
+        const int mid = (view + hi + 1) >> 1;
+        if (views[mid].tile_base <= i) view = mid; else hi = mid - 1;
+      }
     }
-    // front count, back count, back-segment skip-depth minimum (bits; +inf), view
-    reinterpret_cast<int4*>(counts)[i] = make_int4(0, 0, 0x7f800000, lo);
+    reinterpret_cast<int4*>(counts)[i] = make_int4(0, 0, 0x7f800000, view);
   }
-  if (i < 4) status[i] = 0;
-  if (i < kQueues) status[kQueueStride * (i + 1)] = 0;
+  if (blockIdx.x == 0) {
+    if (status) clear_status(status);
+    if (N > 0) store_inline_views(out, n_views);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -320,10 +339,15 @@ UGU_DEV uint32_t probe_cover(const float4& a, const float4& b, const float4& c, 
   return m;
 }
 
-template <int TW, int TH>
+// INL: a pass of one view, its descriptor an argument (see k_begin).
+template <int TW, int TH, bool INL>
 __global__ __launch_bounds__(256) void k_setup_bin(
-    const DevView* __restrict__ views, int n_views, DevMesh mesh,
+    InlineViews<1> arg, const DevView* __restrict__ views, DevView* out, int n_views, DevMesh mesh,
     DevBins bins) {
+  if (INL && blockIdx.x == 0) {
+    clear_status(bins.status);
+    store_inline_views(out, 1);
+  }
   // The block's 256 faces share their vertices (about 150 distinct ones on a
   // regular mesh): every distinct vertex is projected once per view into LDS
   // and the faces read their corners from there, about 0.6 projections per
@@ -360,7 +384,7 @@ __global__ __launch_bounds__(256) void k_setup_bin(
   const int vb = blockIdx.y * kSetupViews;
   const int ve = min(vb + kSetupViews, n_views);
   for (int vi = vb; vi < ve; vi++) {
-    const DevView& v = views[vi];
+    const DevView& v = INL ? arg.v[0] : views[vi];
     bool has = false, back = false;
     float zskip = -1.0f;
     int tx0 = 0, tx1 = -1, ty0 = 0, ty1 = -1;
@@ -811,7 +835,10 @@ UGU_DEV void raster_tile(RasterLds<TW * TH>& s, int gtile, const int4 seg, const
   bool wbf = false;
   // overflowing tiles report their true occupancy; the host re-renders with
   // bins that large (one same-address atomic per overflowing tile only)
-  if (t == 0 && count > bins.cap) atomicMax(&bins.status[0], count);
+  if (t == 0 && count > bins.cap) {
+    atomicMax(&bins.status[0], count);
+    *bins.host_flag = 1;
+  }
   __syncthreads();
 
   // Largest depth any in-view pixel of the tile holds after the previous
@@ -1079,6 +1106,10 @@ UGU_DEV void raster_tile(RasterLds<TW * TH>& s, int gtile, const int4 seg, const
     put3<S>(v.image, pidx, img[0], img[1], img[2]);
     if (v.face_id) put<S>(v.face_id, pidx, fid);
   }
+  // The tile's counters, cleared for the next pass (an empty tile's are clear).
+  // Last: a wavefront's later loads wait for an earlier store, and here none
+  // follow (after the first barrier the store cost the 64-view step 50 us).
+  if (t == 0) reinterpret_cast<int4*>(bins.counts)[gtile] = make_int4(0, 0, 0x7f800000, seg.w);
 }
 
 template <int TW, int TH, int MODE>
@@ -1157,11 +1188,25 @@ __global__ void k_depth_to_u16(const float* __restrict__ d, int64_t n,
 // ---------------------------------------------------------------------------
 // host-side launchers (called from ugu_hip.cpp)
 
-int launch_clear(hipStream_t st, int32_t* counts, int32_t n, int32_t* status,
-                 const int32_t* tile_base, int32_t n_views) {
-  int m = n > 4 ? n : 4;
-  hipLaunchKernelGGL(k_clear, dim3((m + 255) / 256), dim3(256), 0, st, counts, n, status,
-                     tile_base, n_views);
+// hv: the host descriptors of n_views <= kInlineViews views, written to `views`;
+// null: `views` holds them already. counts / status: null when the pass has none.
+int launch_begin(hipStream_t st, const DevView* hv, int n_views, DevView* views, int32_t* counts,
+                 int32_t n_tiles, int32_t* status) {
+  const dim3 grid((n_tiles > 256 ? n_tiles + 255 : 256) / 256);
+  if (hv && n_views == 1) {
+    InlineViews<1> a;
+    a.v[0] = hv[0];
+    hipLaunchKernelGGL(k_begin<1>, grid, dim3(256), 0, st, a, nullptr, views, n_views, counts, n_tiles,
+                       status);
+  } else if (hv) {
+    InlineViews<kInlineViews> a;
+    for (int k = 0; k < n_views; k++) a.v[k] = hv[k];
+    hipLaunchKernelGGL(k_begin<kInlineViews>, grid, dim3(256), 0, st, a, nullptr, views, n_views,
+                       counts, n_tiles, status);
+  } else {
+    hipLaunchKernelGGL(k_begin<0>, grid, dim3(256), 0, st, InlineViews<1>{}, views, nullptr, n_views,
+                       counts, n_tiles, status);
+  }
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -1180,20 +1225,30 @@ int launch_face_soup(hipStream_t st, const float* verts, const int32_t* faces,
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int launch_setup_bin(hipStream_t st, int tw, int th, const DevView* views,
+// one: the host descriptor of a pass of one view whose counters are clear (no
+// launch_begin), written to `views`; otherwise null
+int launch_setup_bin(hipStream_t st, int tw, int th, const DevView* one, DevView* views,
                      int n_views, const DevMesh& mesh,
                      const DevBins& bins) {
   if (mesh.F <= 0) return 0;
   dim3 grid((mesh.F + 255) / 256, (n_views + kSetupViews - 1) / kSetupViews), block(256);
-  if (tw == 8 && th == 8)
-    hipLaunchKernelGGL((k_setup_bin<8, 8>), grid, block, 0, st, views, n_views, mesh, bins);
-  else if (tw == 16 && th == 16)
-    hipLaunchKernelGGL((k_setup_bin<16, 16>), grid, block, 0, st, views, n_views, mesh, bins);
-  else if (tw == 32 && th == 8)
-    hipLaunchKernelGGL((k_setup_bin<32, 8>), grid, block, 0, st, views, n_views, mesh, bins);
-  else
-    return -2;
-  return hipGetLastError() == hipSuccess ? 0 : -1;
+  InlineViews<1> a{};
+  if (one) a.v[0] = *one;
+#define UGU_SETUP_CASE(TWV, THV)                                                          \
+  if (tw == TWV && th == THV) {                                                           \
+    if (one)                                                                              \
+      hipLaunchKernelGGL((k_setup_bin<TWV, THV, true>), grid, block, 0, st, a, nullptr,   \
+                         views, 1, mesh, bins);                                           \
+    else                                                                                  \
+      hipLaunchKernelGGL((k_setup_bin<TWV, THV, false>), grid, block, 0, st, a, views,    \
+                         nullptr, n_views, mesh, bins);                                   \
+    return hipGetLastError() == hipSuccess ? 0 : -1;                                      \
+  }
+  UGU_SETUP_CASE(8, 8)
+  UGU_SETUP_CASE(16, 16)
+  UGU_SETUP_CASE(32, 8)
+#undef UGU_SETUP_CASE
+  return -2;
 }
 
 template <int TW, int TH, int MODE>

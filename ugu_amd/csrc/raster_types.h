@@ -124,8 +124,16 @@ struct DevBins {
   int32_t total_tiles;
   int32_t* status;   // [0] max bin count seen; [kQueueStride (q + 1)] head of
                      // work queue q (kStatusBytes in all)
-  const int32_t* tile_base;  // n_views + 1 prefix of tiles per view
-  int32_t n_views;
+  int32_t* host_flag;  // pinned host word, set when a bin overflows: the host
+                       // reads the status only then
+};
+
+// View descriptors passed as kernel arguments: at most kInlineViews, which keeps
+// the arguments below 4 KB. Larger batches are copied to the device first.
+constexpr int kInlineViews = 12;
+template <int N>
+struct InlineViews {
+  DevView v[N];
 };
 
 // Work queues of the persistent rasterizer: run r (kQueueRun consecutive

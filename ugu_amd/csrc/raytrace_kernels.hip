@@ -267,8 +267,16 @@ UGU_DEV int2 rt_entry(int f, float zskip, int x0, int x1, int y0, int y1, int tx
 
 // One thread per (face, view), as the rasterizer's k_setup_bin: a block's
 // distinct vertices are projected once per view into LDS.
-__global__ __launch_bounds__(256) void k_rt_setup(const DevView* __restrict__ views, int n_views,
-                                                  DevMesh mesh, DevBins bins) {
+// INL: a pass of one view, its descriptor an argument (see k_begin).
+template <bool INL>
+__global__ __launch_bounds__(256) void k_rt_setup(InlineViews<1> arg,
+                                                  const DevView* __restrict__ views, DevView* out,
+                                                  int n_views, DevMesh mesh, DevBins bins) {
+  if (INL && blockIdx.x == 0) {
+    // an occupancy published before this store is published again by its tile
+    clear_status(bins.status);
+    store_inline_views(out, 1);
+  }
   __shared__ float4 sp[768];
   const int f = blockIdx.x * blockDim.x + threadIdx.x;
   const int vbase = mesh.blk_off[blockIdx.x];
@@ -293,7 +301,7 @@ __global__ __launch_bounds__(256) void k_rt_setup(const DevView* __restrict__ vi
   const int vb = blockIdx.y * kSetupViews;
   const int ve = min(vb + kSetupViews, n_views);
   for (int vi = vb; vi < ve; vi++) {
-    const DevView& v = views[vi];
+    const DevView& v = INL ? arg.v[0] : views[vi];
     for (int j = 0; j < 3; j++) {
       const int k = threadIdx.x + j * 256;
       if (k < nu) sp[k] = project_ray(v, P[j * 3 + 0], P[j * 3 + 1], P[j * 3 + 2]);
@@ -459,7 +467,10 @@ __global__ __launch_bounds__(256) void k_rt_tiles(const DevView* __restrict__ vi
   // some bin overflowed (this one: published, the two segments share it): the
   // host renders again, nothing here is worth finishing
   if (seg.x + seg.y > bins.cap || bins.status[0] > bins.cap) {
-    if (t == 0 && seg.x + seg.y > bins.cap) atomicMax(&bins.status[0], seg.x + seg.y);
+    if (t == 0 && seg.x + seg.y > bins.cap) {
+      atomicMax(&bins.status[0], seg.x + seg.y);
+      *bins.host_flag = 1;
+    }
     return;
   }
   const DevView& v = views[seg.w];
@@ -614,6 +625,9 @@ __global__ __launch_bounds__(256) void k_rt_tiles(const DevView* __restrict__ vi
     mt_hit(v.c2w_t[0], v.c2w_t[1], v.c2w_t[2], r0, r1, r2, p0, p1, p2, bt, bu, bv);
   }
   write_hit<true>(v, m, o, gx, gy, bf, bt, bu, bv, r0, r1, r2);
+  // the tile's counters, cleared for the next pass (see raster_tile)
+  if (t == 0 && n > 0)
+    reinterpret_cast<int4*>(bins.counts)[gtile] = make_int4(0, 0, 0x7f800000, seg.w);
 }
 
 // ---------------------------------------------------------------------------
@@ -781,12 +795,19 @@ int launch_visibility(hipStream_t st, const DevView& v, const uint8_t* color, co
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-// views[i].tile_base = first 16x16 tile of view i; the bins' counters cleared
-int launch_raytrace_binned(hipStream_t st, const DevView* views, int n_views, const DevMesh& m,
-                           const DevBins& bins, const DevOptions& o) {
+// views[i].tile_base = first 16x16 tile of view i; the bins' counters cleared.
+// one: as launch_setup_bin's
+int launch_raytrace_binned(hipStream_t st, const DevView* one, DevView* views, int n_views,
+                           const DevMesh& m, const DevBins& bins, const DevOptions& o) {
   if (n_views < 1 || bins.total_tiles < 1 || m.F < 1) return 0;
   const dim3 grid((m.F + 255) / 256, (n_views + kSetupViews - 1) / kSetupViews);
-  hipLaunchKernelGGL(k_rt_setup, grid, dim3(256), 0, st, views, n_views, m, bins);
+  InlineViews<1> a{};
+  if (one) {
+    a.v[0] = *one;
+    hipLaunchKernelGGL(k_rt_setup<true>, grid, dim3(256), 0, st, a, nullptr, views, 1, m, bins);
+  } else {
+    hipLaunchKernelGGL(k_rt_setup<false>, grid, dim3(256), 0, st, a, views, nullptr, n_views, m, bins);
+  }
   hipLaunchKernelGGL(k_rt_tiles, dim3(bins.total_tiles), dim3(256), 0, st, views, m, bins, o);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }

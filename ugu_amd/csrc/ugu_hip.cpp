@@ -20,13 +20,13 @@
 #include "raster_types.h"
 
 namespace ugu_hip {
-int launch_clear(hipStream_t st, int32_t* counts, int32_t n, int32_t* status,
-                 const int32_t* tile_base, int32_t n_views);
+int launch_begin(hipStream_t st, const DevView* hv, int n_views, DevView* views, int32_t* counts,
+                 int32_t n_tiles, int32_t* status);
 int launch_shade_rec(hipStream_t st, const DevMesh& m, float4* out);
 int launch_face_soup(hipStream_t st, const float* verts, const int32_t* faces,
                      const float* fnormals, int32_t F, int compute_normals, float4* soup,
                      float* fn_out);
-int launch_setup_bin(hipStream_t st, int tw, int th, const DevView* views,
+int launch_setup_bin(hipStream_t st, int tw, int th, const DevView* one, DevView* views,
                      int n_views, const DevMesh& mesh,
                      const DevBins& bins);
 int launch_raster(hipStream_t st, int tw, int th, int mode, const DevView* views,
@@ -41,8 +41,8 @@ int launch_backward(hipStream_t st, const DevView* views, int n_views, int max_s
 int launch_depth_to_u16(hipStream_t st, const float* d, int64_t n, uint16_t* out);
 int launch_raytrace(hipStream_t st, const DevView* views, int n_views, int total_tiles,
                     const DevBvh& bvh, const DevMesh& m, const DevOptions& o);
-int launch_raytrace_binned(hipStream_t st, const DevView* views, int n_views, const DevMesh& m,
-                           const DevBins& bins, const DevOptions& o);
+int launch_raytrace_binned(hipStream_t st, const DevView* one, DevView* views, int n_views,
+                           const DevMesh& m, const DevBins& bins, const DevOptions& o);
 int launch_texture_map(hipStream_t st, const void* faces, int n, const void* images, int cols,
                        int rows, int hk, int32_t* owner, uint8_t* tex0, uint8_t* mask0,
                        uint8_t* tex, uint8_t* mask);
@@ -66,13 +66,10 @@ namespace {
 constexpr int kNoAllocMaxViews = 1024;
 constexpr int kMaxDevices = 64;
 // Layout of the scratch array (offsets 256-B aligned): status words (max bin
-// count, work-queue heads), the view descriptors, the views' first global
-// tiles, then per render group the tiles' counters and the bins.
+// count, work-queue heads), the view descriptors, then per render group the tiles' counters and the bins.
 constexpr size_t kNaViewsOff = (size_t(kStatusBytes) + 255) / 256 * 256;
-constexpr size_t kNaTileBaseOff =
-    (kNaViewsOff + size_t(kNoAllocMaxViews) * sizeof(DevView) + 255) / 256 * 256;
 constexpr size_t kNaCountsOff =
-    (kNaTileBaseOff + size_t(kNoAllocMaxViews + 1) * 4 + 255) / 256 * 256;
+    (kNaViewsOff + size_t(kNoAllocMaxViews) * sizeof(DevView) + 255) / 256 * 256;
 static_assert(kNaCountsOff < kScratchBytes / 2, "descriptor area fits the scratch");
 
 std::mutex g_scratch_mu;                          // guards the two tables below
@@ -128,24 +125,6 @@ struct DevBuf {
   T* as() const { return static_cast<T*>(p); }
 };
 
-struct GraphKey {
-  int n, total_tiles, V, F, tw, th, persistent_blocks, mode, cap;
-  int64_t buf_gen, mesh_gen;
-  DevOptions opt;
-  const void* verts;
-  const void* vcolors;
-  const void* ftex;
-  int ftex_w, ftex_h;
-  bool operator==(const GraphKey& o) const { return std::memcmp(this, &o, sizeof(*this)) == 0; }
-};
-
-struct GraphEntry {
-  GraphKey key;
-  hipGraphExec_t exec;
-};
-
-constexpr size_t kMaxGraphs = 16;
-
 }  // namespace
 
 struct ugu_hip_ctx {
@@ -167,7 +146,7 @@ struct ugu_hip_ctx {
       texinfo, texdata;
 
   // work buffers
-  DevBuf counts, bins, status, views, tile_base, stage_out, diff_fn;
+  DevBuf counts, bins, status, views, stage_out, diff_fn;
   DevBuf bwd_items;  // (face, view, pixel) items of the backward pass, 16 B each
   DevBuf bwd_scratch;  // face group counts and cursors of the backward pass
   bool bwd_zeroed = false;  // the counts are zero (every completed pass leaves them so)
@@ -184,16 +163,14 @@ struct ugu_hip_ctx {
   float rt_max_coord = 0.0f, rt_max_edge = 0.0f;  // 1-norms, for the binned path's bounds
   bool rt_bins = false;      // few enough layers of faces for the binned path
   int32_t rt_cap = 1024;     // entries per tile of the raytracer's bins
-  int64_t buf_gen = 0;
+  int clean_tiles = 0;  // leading tile counters known to be clear, of view 0
   void* h_views = nullptr;
   size_t h_views_bytes = 0;
-  int32_t* h_status = nullptr;
-  std::vector<int32_t> h_tile_base;
+  int32_t* h_status = nullptr;  // pinned: [0] overflow flag / occupancy, [4] item total
 
   UguTiling tiling{16, 16, 1024, 1};
   int cu_count = 0;
   std::string arch;  // gcnArchName of the device (tuning-cache key)
-  std::vector<GraphEntry> graphs;
 
   bool profile = false;
   UguTimings tm{};
@@ -203,7 +180,6 @@ struct ugu_hip_ctx {
   // first tiles (sized at create), and the per-tile bin capacity the last
   // calls needed (groups are formed so every tile gets at least this much)
   std::vector<DevView> na_views;
-  std::vector<int32_t> na_tile_base;
   int64_t na_cap_hint = 0;
 };
 
@@ -232,20 +208,39 @@ int hip_fail(ugu_hip_ctx* c, hipError_t e, const char* where) {
 // queues afterwards sees the results.
 int order_after_user(ugu_hip_ctx* c) {
   UGU_HIP_CHECK(c, hipEventRecord(c->ev_user, c->user));
+  // nothing was queued there: no wait needs to be queued here
+  const hipError_t e = hipEventQuery(c->ev_user);
+  if (e == hipSuccess) return 0;
+  (void)hipGetLastError();  // "not ready" would be taken for the next launch's error
+  if (e != hipErrorNotReady) return hip_fail(c, e, "hipEventQuery");
   UGU_HIP_CHECK(c, hipStreamWaitEvent(c->stream, c->ev_user, 0));
+  return 0;
+}
+
+// The largest bin occupancy an overflowing pass saw (0: none overflowed), once
+// the stream is idle. The kernels set the pinned flag; the status is fetched only
+// then.
+int read_overflow(ugu_hip_ctx* c, const int32_t* status, int32_t* most) {
+  *most = 0;
+  if (*static_cast<volatile int32_t*>(c->h_status) == 0) return 0;
+  UGU_HIP_CHECK(c, hipMemcpyAsync(c->h_status, status, 4, hipMemcpyDeviceToHost, c->stream));
+  UGU_HIP_CHECK(c, hipStreamSynchronize(c->stream));
+  *most = c->h_status[0];
   return 0;
 }
 
 int ensure(ugu_hip_ctx* c, DevBuf& b, size_t n) {
   int r = b.ensure(n);
   if (r < 0) return fail(c, UGU_HIP_ERR_OUT_OF_MEMORY, "device allocation failed");
-  if (r > 0) c->buf_gen++;
   return 0;
 }
 
-void drop_graphs(ugu_hip_ctx* c) {
-  for (auto& g : c->graphs) (void)hipGraphExecDestroy(g.exec);
-  c->graphs.clear();
+// The tile counters. A pass takes the count of clear ones (clean_tiles), and puts
+// it back when it has completed as a pass of one view.
+int ensure_counts(ugu_hip_ctx* c, int64_t tiles) {
+  const int r = c->counts.ensure(size_t(tiles) * 16);
+  if (r != 0) c->clean_tiles = 0;
+  return r < 0 ? fail(c, UGU_HIP_ERR_OUT_OF_MEMORY, "device allocation failed") : 0;
 }
 
 int upload(ugu_hip_ctx* c, DevBuf& b, const void* src, size_t n) {
@@ -494,10 +489,9 @@ void fill_view_camera(DevView& v, const UguCamera& cam, int tw, int th, int32_t 
 int run_pipeline(ugu_hip_ctx* c, const UguCamera* cams, int n, const DevMesh& dm,
                  const DevOptions& dopt, int mode, const UguOutputs* outs,
                  int memory, float* const* images, int32_t* const* fids,
-                 bool use_graph, const UguGBuffer* gbufs = nullptr) {
+                 const UguGBuffer* gbufs = nullptr) {
   const int tw = c->tiling.tile_w, th = c->tiling.tile_h;
   // layout
-  c->h_tile_base.resize(n + 1);
   int64_t total = 0;
   int64_t stage_bytes = 0;
   std::vector<int64_t> stage_off(size_t(n) * kPlanes, -1);
@@ -505,7 +499,6 @@ int run_pipeline(ugu_hip_ctx* c, const UguCamera* cams, int n, const DevMesh& dm
     int err = check_camera(c, cams[i]);
     if (err) return err;
     const int tx = (cams[i].width + tw - 1) / tw, ty = (cams[i].height + th - 1) / th;
-    c->h_tile_base[i] = static_cast<int32_t>(total);
     total += int64_t(tx) * ty;
     if (mode == 0 && memory == UGU_HIP_MEMORY_HOST) {
       const int64_t px = int64_t(cams[i].width) * cams[i].height;
@@ -520,16 +513,14 @@ int run_pipeline(ugu_hip_ctx* c, const UguCamera* cams, int n, const DevMesh& dm
     }
   }
   if (total > INT32_MAX / 2) return fail(c, UGU_HIP_ERR_INVALID_ARGUMENT, "too many tiles");
-  c->h_tile_base[n] = static_cast<int32_t>(total);
   const int total_tiles = static_cast<int>(total);
 
   int err;
-  if ((err = ensure(c, c->counts, size_t(total_tiles) * 16))) return err;  // 4 per tile
+  if ((err = ensure_counts(c, total_tiles))) return err;
   if ((err = ensure(c, c->status, kStatusBytes))) return err;
   if ((err = ensure(c, c->views, size_t(n) * sizeof(DevView)))) return err;
-  if ((err = ensure(c, c->tile_base, size_t(n + 1) * 4))) return err;
   if (stage_bytes > 0 && (err = ensure(c, c->stage_out, size_t(stage_bytes)))) return err;
-  const size_t view_bytes = size_t(n) * sizeof(DevView) + size_t(n + 1) * 4;
+  const size_t view_bytes = size_t(n) * sizeof(DevView);
   if (c->h_views_bytes < view_bytes) {
     if (c->h_views) (void)hipHostFree(c->h_views);
     c->h_views = nullptr;
@@ -540,9 +531,11 @@ int run_pipeline(ugu_hip_ctx* c, const UguCamera* cams, int n, const DevMesh& dm
 
   // view descriptors
   DevView* hv = static_cast<DevView*>(c->h_views);
+  int32_t tile_base = 0;
   for (int i = 0; i < n; i++) {
     DevView& v = hv[i];
-    fill_view_camera(v, cams[i], tw, th, c->h_tile_base[i]);
+    fill_view_camera(v, cams[i], tw, th, tile_base);
+    tile_base += v.tiles_x * v.tiles_y;
     if (mode == 0) {
       void* p[kPlanes];
       plane_ptrs(outs[i], gbufs ? &gbufs[i] : nullptr, p);
@@ -557,9 +550,6 @@ int run_pipeline(ugu_hip_ctx* c, const UguCamera* cams, int n, const DevMesh& dm
       v.face_id = fids ? fids[i] : nullptr;
     }
   }
-  std::memcpy(reinterpret_cast<uint8_t*>(c->h_views) + size_t(n) * sizeof(DevView),
-              c->h_tile_base.data(), size_t(n + 1) * 4);
-
   int persistent_blocks = 0;
   if (c->tiling.persistent) {
     const int per_cu = raster_blocks_per_cu(tw, th, mode);
@@ -576,76 +566,33 @@ int run_pipeline(ugu_hip_ctx* c, const UguCamera* cams, int n, const DevMesh& dm
     b.cap = c->tiling.bin_capacity;
     b.total_tiles = total_tiles;
     b.status = c->status.as<int32_t>();
-    b.tile_base = c->tile_base.as<int32_t>();
-    b.n_views = n;
-    const DevView* dv = c->views.as<DevView>();
+    b.host_flag = c->h_status;
+    DevView* dv = c->views.as<DevView>();
+    c->h_status[0] = 0;
 
-    UGU_HIP_CHECK(c, hipMemcpyAsync(c->views.p, c->h_views, size_t(n) * sizeof(DevView),
-                                    hipMemcpyHostToDevice, c->stream));
-    UGU_HIP_CHECK(c, hipMemcpyAsync(c->tile_base.p,
-                                    reinterpret_cast<uint8_t*>(c->h_views) + size_t(n) * sizeof(DevView),
-                                    size_t(n + 1) * 4, hipMemcpyHostToDevice, c->stream));
-
-    auto launch_all = [&](bool timed) -> int {
-      if (timed) (void)hipEventRecord(c->ev[0], c->stream);
-      if (launch_clear(c->stream, b.counts, total_tiles, b.status, b.tile_base, n))
-        return -1;
-      if (timed) (void)hipEventRecord(c->ev[1], c->stream);
-      if (launch_setup_bin(c->stream, tw, th, dv, n, dm, b)) return -1;
-      if (timed) (void)hipEventRecord(c->ev[2], c->stream);
-      if (launch_raster(c->stream, tw, th, mode, dv, dm, b, dopt, persistent_blocks)) return -1;
-      if (timed) (void)hipEventRecord(c->ev[3], c->stream);
-      return 0;
-    };
-
-    if (use_graph && !c->profile) {
-      GraphKey key;
-      std::memset(&key, 0, sizeof(key));
-      key.n = n;
-      key.total_tiles = total_tiles;
-      key.V = dm.V;
-      key.F = dm.F;
-      key.tw = tw;
-      key.th = th;
-      key.persistent_blocks = persistent_blocks;
-      key.mode = mode;
-      key.cap = b.cap;  // the capacity is baked into the captured launches
-      key.buf_gen = c->buf_gen;
-      key.mesh_gen = c->mesh_gen;
-      key.opt = dopt;
-      key.verts = dm.verts;
-      key.vcolors = dm.vcolors;
-      key.ftex = dm.ftex;
-      key.ftex_w = dm.ftex_w;
-      key.ftex_h = dm.ftex_h;
-      hipGraphExec_t exec = nullptr;
-      for (auto& g : c->graphs)
-        if (g.key == key) exec = g.exec;
-      if (!exec) {
-        hipGraph_t graph = nullptr;
-        UGU_HIP_CHECK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-        int le = launch_all(false);
-        hipError_t ce = hipStreamEndCapture(c->stream, &graph);
-        if (le || ce != hipSuccess) {
-          if (graph) (void)hipGraphDestroy(graph);
-          return fail(c, UGU_HIP_ERR_HIP, "graph capture failed");
-        }
-        hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(graph);
-        if (ie != hipSuccess) return hip_fail(c, ie, "hipGraphInstantiate");
-        if (c->graphs.size() >= kMaxGraphs) {
-          (void)hipGraphExecDestroy(c->graphs.front().exec);
-          c->graphs.erase(c->graphs.begin());
-        }
-        c->graphs.push_back(GraphEntry{key, exec});
-      }
-      UGU_HIP_CHECK(c, hipGraphLaunch(exec, c->stream));
-    } else {
-      if (launch_all(c->profile)) return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
-    }
-    UGU_HIP_CHECK(c, hipMemcpyAsync(c->h_status, c->status.p, 16, hipMemcpyDeviceToHost, c->stream));
+    // Direct launches: a graph of these three takes 13 us more than they do.
+    const bool fresh = n == 1 && total_tiles <= c->clean_tiles && dm.F > 0;
+    const int clean = c->clean_tiles;
+    c->clean_tiles = 0;  // until the pass has completed
+    if (n > kInlineViews)
+      UGU_HIP_CHECK(c, hipMemcpyAsync(dv, hv, size_t(n) * sizeof(DevView), hipMemcpyHostToDevice,
+                                      c->stream));
+    const bool timed = c->profile;
+    if (timed) (void)hipEventRecord(c->ev[0], c->stream);
+    if (!fresh && launch_begin(c->stream, n <= kInlineViews ? hv : nullptr, n, dv, b.counts,
+                               total_tiles, b.status))
+      return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
+    if (timed) (void)hipEventRecord(c->ev[1], c->stream);
+    if (launch_setup_bin(c->stream, tw, th, fresh ? hv : nullptr, dv, n, dm, b))
+      return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
+    if (timed) (void)hipEventRecord(c->ev[2], c->stream);
+    if (launch_raster(c->stream, tw, th, mode, dv, dm, b, dopt, persistent_blocks))
+      return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
+    if (timed) (void)hipEventRecord(c->ev[3], c->stream);
     UGU_HIP_CHECK(c, hipStreamSynchronize(c->stream));
-    const int max_count = c->h_status[0];
+    if (n == 1) c->clean_tiles = std::max(clean, total_tiles);
+    int32_t max_count = 0;
+    if ((err = read_overflow(c, b.status, &max_count))) return err;
     c->tm.max_bin_count = std::max(c->tm.max_bin_count, max_count);
     if (c->profile) {
       float ms[3] = {0, 0, 0};
@@ -685,8 +632,7 @@ int run_pipeline(ugu_hip_ctx* c, const UguCamera* cams, int n, const DevMesh& dm
 }
 
 int render_common(ugu_hip_ctx* c, const UguCamera* cams, int n, const UguOptions* o,
-                  const UguOutputs* outs, int memory, bool use_graph,
-                  const UguGBuffer* gbufs = nullptr) {
+                  const UguOutputs* outs, int memory, const UguGBuffer* gbufs = nullptr) {
   if (!c) return UGU_HIP_ERR_INVALID_ARGUMENT;
   if (n < 1 || cams == nullptr || outs == nullptr)
     return fail(c, n < 1 ? UGU_HIP_ERR_INVALID_ARGUMENT : UGU_HIP_ERR_NO_CAMERA,
@@ -704,12 +650,10 @@ int render_common(ugu_hip_ctx* c, const UguCamera* cams, int n, const UguOptions
   UGU_HIP_CHECK(c, hipSetDevice(c->device));
   if (int oe = order_after_user(c)) return oe;
   DevMesh dm = dev_mesh(c);
-  return run_pipeline(c, cams, n, dm, dev_options(*o), 0, outs, memory, nullptr, nullptr, use_graph,
-                      gbufs);
+  return run_pipeline(c, cams, n, dm, dev_options(*o), 0, outs, memory, nullptr, nullptr, gbufs);
 }
 
-// The pipeline of run_pipeline (clear, setup+bin, raster; eager launches, no
-// graph) over the scratch array at `base` instead of the context's buffers.
+// The pipeline of run_pipeline (begin, setup+bin, raster) over the scratch array at `base` instead of the context's buffers.
 // Views are rendered in consecutive groups whose tiles all get at least
 // `want` bin entries; a group in which a tile overflows is rendered again as
 // smaller groups with the measured occupancy as the new `want` (the tiles of
@@ -723,7 +667,6 @@ int run_noalloc(ugu_hip_ctx* c, uint8_t* base, const UguCamera* cams, int n, con
   const int tw = c->tiling.tile_w, th = c->tiling.tile_h;
   int32_t* status = reinterpret_cast<int32_t*>(base);
   DevView* dviews = reinterpret_cast<DevView*>(base + kNaViewsOff);
-  int32_t* dtile_base = reinterpret_cast<int32_t*>(base + kNaTileBaseOff);
   const size_t avail = kScratchBytes - kNaCountsOff;
   auto tiles_of = [&](const UguCamera& cam) {
     return int64_t((cam.width + tw - 1) / tw) * int64_t((cam.height + th - 1) / th);
@@ -765,10 +708,8 @@ int run_noalloc(ugu_hip_ctx* c, uint8_t* base, const UguCamera* cams, int n, con
       void* p[kPlanes];
       plane_ptrs(outs[s + i], nullptr, p);
       set_view_planes(v, p);
-      c->na_tile_base[size_t(i)] = tb;
       tb += static_cast<int32_t>(tiles_of(cams[s + i]));
     }
-    c->na_tile_base[size_t(g)] = tb;
     const int total_tiles = static_cast<int>(tiles);
     DevBins b;
     b.counts = reinterpret_cast<int32_t*>(base + kNaCountsOff);
@@ -776,21 +717,23 @@ int run_noalloc(ugu_hip_ctx* c, uint8_t* base, const UguCamera* cams, int n, con
     b.cap = static_cast<int32_t>(cap);
     b.total_tiles = total_tiles;
     b.status = status;
-    b.tile_base = dtile_base;
-    b.n_views = g;
+    b.host_flag = c->h_status;
+    c->h_status[0] = 0;
     int persistent_blocks = persistent_blocks_per_cu * std::max(1, c->cu_count);
     if (!c->tiling.persistent || persistent_blocks > total_tiles) persistent_blocks = 0;
-    UGU_HIP_CHECK(c, hipMemcpyAsync(dviews, c->na_views.data(), size_t(g) * sizeof(DevView),
-                                    hipMemcpyHostToDevice, c->stream));
-    UGU_HIP_CHECK(c, hipMemcpyAsync(dtile_base, c->na_tile_base.data(), size_t(g + 1) * 4,
-                                    hipMemcpyHostToDevice, c->stream));
-    if (launch_clear(c->stream, b.counts, total_tiles, b.status, b.tile_base, g) ||
-        launch_setup_bin(c->stream, tw, th, dviews, g, dm, b) ||
+    const bool inline_views = g <= kInlineViews;
+    if (!inline_views)
+      UGU_HIP_CHECK(c, hipMemcpyAsync(dviews, c->na_views.data(), size_t(g) * sizeof(DevView),
+                                      hipMemcpyHostToDevice, c->stream));
+    if (launch_begin(c->stream, inline_views ? c->na_views.data() : nullptr, g, dviews, b.counts,
+                     total_tiles, b.status) ||
+        launch_setup_bin(c->stream, tw, th, nullptr, dviews, g, dm, b) ||
         launch_raster(c->stream, tw, th, 0, dviews, dm, b, dopt, persistent_blocks))
       return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
-    UGU_HIP_CHECK(c, hipMemcpyAsync(c->h_status, status, 16, hipMemcpyDeviceToHost, c->stream));
     UGU_HIP_CHECK(c, hipStreamSynchronize(c->stream));
-    const int64_t max_count = c->h_status[0];
+    int32_t most = 0;
+    if (int err = read_overflow(c, status, &most)) return err;
+    const int64_t max_count = most;
     if (max_count <= cap) {
       s = e;
       continue;
@@ -897,28 +840,25 @@ constexpr int32_t kRtMaxCap = 4096;
 int raytrace_binned(ugu_hip_ctx* c, DevView* hv, int n, const DevMesh& dm, const DevOptions& dopt) {
   if (!c->rt_bins) return 0;
   int64_t total = 0;
-  int32_t* tb = reinterpret_cast<int32_t*>(hv + n);
   for (int i = 0; i < n; i++) {
     if (!rt_view_bounds(c, &hv[i])) return 0;
     hv[i].tiles_x = (hv[i].W + 15) / 16;
     hv[i].tiles_y = (hv[i].H + 15) / 16;
-    hv[i].tile_base = tb[i] = static_cast<int32_t>(total);
+    hv[i].tile_base = static_cast<int32_t>(total);
     total += int64_t(hv[i].tiles_x) * hv[i].tiles_y;
     if (total > INT32_MAX / 2) return 0;
   }
-  tb[n] = static_cast<int32_t>(total);
   int err;
   if ((err = ensure(c, c->status, kStatusBytes))) return err;
-  if ((err = ensure(c, c->tile_base, size_t(n + 1) * 4))) return err;
   // a failed allocation's error would be taken for the next launch's
-  if (ensure(c, c->counts, size_t(total) * 16)) {
+  if (ensure_counts(c, total)) {
     (void)hipGetLastError();
     return 0;
   }
-  UGU_HIP_CHECK(c, hipMemcpyAsync(c->views.p, hv, size_t(n) * sizeof(DevView),
-                                  hipMemcpyHostToDevice, c->stream));
-  UGU_HIP_CHECK(c, hipMemcpyAsync(c->tile_base.p, tb, size_t(n + 1) * 4, hipMemcpyHostToDevice,
-                                  c->stream));
+  const bool inline_views = n <= kInlineViews;
+  if (!inline_views)
+    UGU_HIP_CHECK(c, hipMemcpyAsync(c->views.p, hv, size_t(n) * sizeof(DevView),
+                                    hipMemcpyHostToDevice, c->stream));
   for (;;) {
     if (total * c->rt_cap * 8 > (int64_t(32) << 30)) return 0;
     if (ensure(c, c->bins, size_t(total) * size_t(c->rt_cap) * 8)) {
@@ -931,17 +871,25 @@ int raytrace_binned(ugu_hip_ctx* c, DevView* hv, int n, const DevMesh& dm, const
     b.cap = c->rt_cap;
     b.total_tiles = static_cast<int32_t>(total);
     b.status = c->status.as<int32_t>();
-    b.tile_base = c->tile_base.as<int32_t>();
-    b.n_views = n;
-    if (launch_clear(c->stream, b.counts, b.total_tiles, b.status, b.tile_base, n) ||
-        launch_raytrace_binned(c->stream, c->views.as<DevView>(), n, dm, b, dopt))
+    b.host_flag = c->h_status;
+    c->h_status[0] = 0;
+    DevView* dv = c->views.as<DevView>();
+    const bool fresh = n == 1 && b.total_tiles <= c->clean_tiles;
+    const int clean = c->clean_tiles;
+    c->clean_tiles = 0;  // until the pass has completed
+    if (!fresh &&
+        launch_begin(c->stream, inline_views ? hv : nullptr, n, dv, b.counts, b.total_tiles, b.status))
       return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
-    UGU_HIP_CHECK(c, hipMemcpyAsync(c->h_status, c->status.p, 16, hipMemcpyDeviceToHost, c->stream));
+    if (launch_raytrace_binned(c->stream, fresh ? hv : nullptr, dv, n, dm, b, dopt))
+      return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
     UGU_HIP_CHECK(c, hipStreamSynchronize(c->stream));
-    const int64_t most = c->h_status[0];
+    int32_t most = 0;
+    if ((err = read_overflow(c, b.status, &most))) return err;
+    // tiles that saw an overflow left their counters as they were
+    if (n == 1 && most == 0) c->clean_tiles = std::max(clean, b.total_tiles);
     if (most <= c->rt_cap) return 1;
     if (most > kRtMaxCap) return 0;
-    c->rt_cap = static_cast<int32_t>(std::min<int64_t>(kRtMaxCap, (most + most / 8 + 63) / 64 * 64));
+    c->rt_cap = static_cast<int32_t>(std::min<int64_t>(kRtMaxCap, (int64_t(most) + most / 8 + 63) / 64 * 64));
   }
 }
 
@@ -994,13 +942,12 @@ int raytrace_common(ugu_hip_ctx* c, const UguCamera* cams, int n, const UguOptio
   if ((err = ensure(c, c->views, size_t(n) * sizeof(DevView)))) return err;
   if (stage_bytes > 0 && (err = ensure(c, c->stage_out, size_t(stage_bytes)))) return err;
   const size_t view_bytes = size_t(n) * sizeof(DevView);
-  const size_t host_bytes = view_bytes + size_t(n + 1) * 4;
-  if (c->h_views_bytes < host_bytes) {
+  if (c->h_views_bytes < view_bytes) {
     if (c->h_views) (void)hipHostFree(c->h_views);
     c->h_views = nullptr;
     c->h_views_bytes = 0;
-    UGU_HIP_CHECK(c, hipHostMalloc(&c->h_views, host_bytes, hipHostMallocDefault));
-    c->h_views_bytes = host_bytes;
+    UGU_HIP_CHECK(c, hipHostMalloc(&c->h_views, view_bytes, hipHostMallocDefault));
+    c->h_views_bytes = view_bytes;
   }
   DevView* hv = static_cast<DevView*>(c->h_views);
   for (int i = 0; i < n; i++) {
@@ -1105,7 +1052,6 @@ ugu_hip_ctx* ugu_hip_create(int device) {
   for (auto& e : c->ev) (void)hipEventCreate(&e);
   init_scratch(device);
   c->na_views.resize(kNoAllocMaxViews);
-  c->na_tile_base.resize(kNoAllocMaxViews + 1);
   return c;
 }
 
@@ -1113,11 +1059,10 @@ void ugu_hip_destroy(ugu_hip_ctx* c) {
   if (!c) return;
   (void)hipSetDevice(c->device);
   if (c->stream) (void)hipStreamSynchronize(c->stream);
-  drop_graphs(c);
   DevBuf* bufs[] = {&c->verts, &c->faces, &c->faces_orig, &c->fnormals, &c->normals, &c->nidx,
                     &c->vcolors, &c->uv, &c->uvidx, &c->matid, &c->texinfo,
                     &c->texdata, &c->counts, &c->bins, &c->status,
-                    &c->views, &c->tile_base, &c->stage_out, &c->diff_fn,
+                    &c->views, &c->stage_out, &c->diff_fn,
                     &c->bwd_items, &c->bwd_scratch, &c->soup, &c->diff_soup, &c->shade, &c->blk_off,
                     &c->blk_vid, &c->face_loc, &c->blk_off_o, &c->blk_vid_o, &c->face_loc_o,
                     &c->bvh_nodes, &c->bvh_leaves, &c->bvh_tris, &c->vis_items,
@@ -1168,7 +1113,6 @@ int ugu_hip_prepare_mesh(ugu_hip_ctx* c, const UguMeshDesc* m) {
   UGU_HIP_CHECK(c, hipSetDevice(c->device));
   if (int oe = order_after_user(c)) return oe;
   UGU_HIP_CHECK(c, hipStreamSynchronize(c->stream));
-  drop_graphs(c);
 
   // Relabel vertices, normals and uvs in first-touch order of their index
   // arrays: a screen tile's faces are a compact run of the face array, and
@@ -1281,23 +1225,23 @@ int ugu_hip_prepare_mesh(ugu_hip_ctx* c, const UguMeshDesc* m) {
 int ugu_hip_render(ugu_hip_ctx* c, const UguCamera* cam, const UguOptions* o,
                    const UguOutputs* out, int memory) {
   if (c && cam == nullptr) return fail(c, UGU_HIP_ERR_NO_CAMERA, "camera has not been set\n");
-  return render_common(c, cam, 1, o, out, memory, true);
+  return render_common(c, cam, 1, o, out, memory);
 }
 
 int ugu_hip_render_batch(ugu_hip_ctx* c, const UguCamera* cams, int n,
                          const UguOptions* o, const UguOutputs* outs, int memory) {
-  return render_common(c, cams, n, o, outs, memory, true);
+  return render_common(c, cams, n, o, outs, memory);
 }
 
 int ugu_hip_render_gbuffer(ugu_hip_ctx* c, const UguCamera* cams, int n, const UguOptions* o,
                            const UguOutputs* outs, const UguGBuffer* gbufs, int memory) {
   if (c && !gbufs) return fail(c, UGU_HIP_ERR_INVALID_ARGUMENT, "gbuffers are required");
-  return render_common(c, cams, n, o, outs, memory, true, gbufs);
+  return render_common(c, cams, n, o, outs, memory, gbufs);
 }
 
 int ugu_hip_render_batch_eager(ugu_hip_ctx* c, const UguCamera* cams, int n,
                                const UguOptions* o, const UguOutputs* outs, int memory) {
-  return render_common(c, cams, n, o, outs, memory, false);
+  return render_common(c, cams, n, o, outs, memory);
 }
 
 int ugu_hip_render_batch_noalloc(ugu_hip_ctx* c, const UguCamera* cams, int n,
@@ -1523,7 +1467,6 @@ int ugu_hip_set_tiling(ugu_hip_ctx* c, const UguTiling* t) {
     return fail(c, UGU_HIP_ERR_INVALID_ARGUMENT, "tile must be 8x8, 16x16 or 32x8");
   if (t->bin_capacity < 1) return fail(c, UGU_HIP_ERR_INVALID_ARGUMENT, "bin capacity must be >= 1");
   c->tiling = *t;
-  drop_graphs(c);
   return UGU_HIP_OK;
 }
 
@@ -1588,14 +1531,13 @@ int ugu_hip_autotune(ugu_hip_ctx* c, const UguCamera* cams, int n, const UguOpti
     t.persistent = sh[2];
     t.bin_capacity = 256;
     c->tiling = t;
-    drop_graphs(c);
-    // first render sizes the bins from the measured occupancy
-    err = render_common(c, cams, n, &opt, outs.data(), UGU_HIP_MEMORY_DEVICE, true);
+      // first render sizes the bins from the measured occupancy
+    err = render_common(c, cams, n, &opt, outs.data(), UGU_HIP_MEMORY_DEVICE);
     if (err) break;
     std::vector<double> times;
     for (int r = 0; r < repeats; r++) {
       auto t0 = std::chrono::steady_clock::now();
-      err = render_common(c, cams, n, &opt, outs.data(), UGU_HIP_MEMORY_DEVICE, true);
+      err = render_common(c, cams, n, &opt, outs.data(), UGU_HIP_MEMORY_DEVICE);
       auto t1 = std::chrono::steady_clock::now();
       if (err) break;
       times.push_back(std::chrono::duration<double, std::milli>(t1 - t0).count());
@@ -1609,14 +1551,11 @@ int ugu_hip_autotune(ugu_hip_ctx* c, const UguCamera* cams, int n, const UguOpti
     }
   }
   outbuf.release();
-  c->buf_gen++;
   if (err) {
     c->tiling = saved;
-    drop_graphs(c);
-    return err;
+      return err;
   }
   c->tiling = best;
-  drop_graphs(c);
   if (chosen) *chosen = best;
   return UGU_HIP_OK;
 }
@@ -1665,8 +1604,7 @@ int ugu_hip_autotune_cached(ugu_hip_ctx* c, const UguCamera* cams, int n, const 
       std::fclose(f);
       if (hit) {
         c->tiling = found;
-        drop_graphs(c);
-        if (chosen) *chosen = found;
+              if (chosen) *chosen = found;
         if (from_cache) *from_cache = 1;
         return UGU_HIP_OK;
       }
@@ -1752,7 +1690,7 @@ int ugu_hip_diff_forward(ugu_hip_ctx* c, const UguCamera* cams, int n,
   o.backface_culling = p->backface_culling;
   DevOptions dopt = dev_options(o);
   return run_pipeline(c, cams, n, dm, dopt, 1, nullptr, UGU_HIP_MEMORY_DEVICE, images,
-                      face_ids, true);
+                      face_ids);
 }
 
 int ugu_hip_diff_backward(ugu_hip_ctx* c, const UguCamera* cams, int n,
@@ -1770,7 +1708,7 @@ int ugu_hip_diff_backward(ugu_hip_ctx* c, const UguCamera* cams, int n,
   int max_squares = 0;  // 16 x 16 pixel squares of the largest view
   int64_t total_px = 0;
   if ((err = ensure(c, c->views, size_t(n) * sizeof(DevView)))) return err;
-  const size_t view_bytes = size_t(n) * sizeof(DevView) + size_t(n + 1) * 4;
+  const size_t view_bytes = size_t(n) * sizeof(DevView);
   if (c->h_views_bytes < view_bytes) {
     if (c->h_views) (void)hipHostFree(c->h_views);
     c->h_views = nullptr;
@@ -1805,9 +1743,12 @@ int ugu_hip_diff_backward(ugu_hip_ctx* c, const UguCamera* cams, int n,
   if (!c->bwd_zeroed)
     UGU_HIP_CHECK(c, hipMemsetAsync(c->bwd_scratch.p, 0, scratch_bytes, c->stream));
   c->bwd_zeroed = false;  // until this pass has completed
-  UGU_HIP_CHECK(c, hipMemcpyAsync(c->views.p, c->h_views, size_t(n) * sizeof(DevView),
-                                  hipMemcpyHostToDevice, c->stream));
-  const DevView* dv = c->views.as<DevView>();
+  DevView* dv = c->views.as<DevView>();
+  if (n > kInlineViews)
+    UGU_HIP_CHECK(c, hipMemcpyAsync(dv, c->h_views, size_t(n) * sizeof(DevView),
+                                    hipMemcpyHostToDevice, c->stream));
+  else if (launch_begin(c->stream, hv, n, dv, nullptr, 0, nullptr))
+    return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
   DevGrads g;
   g.verts = grad_vertices;
   g.colors = p->vertex_colors ? grad_vertex_colors : nullptr;

@@ -101,7 +101,9 @@ class MeshDesc:
 
 
 class Rasterizer:
-    """ugu::Rasterizer on the gfx950 pipeline (one HIP context per object)."""
+    """ugu::Rasterizer on the gfx950 pipeline (one HIP context per object).
+    The methods' ``graph`` argument chooses between two entry points that do the
+    same."""
 
     def __init__(self, option=None, device=0):
         self._lib = _abi.load_library()
