@@ -17,6 +17,7 @@
 
 #include "../../include/ugu_hip.h"
 #include "bvh_build.h"
+#include "host_copy.h"
 #include "raster_types.h"
 
 namespace ugu_hip {
@@ -164,6 +165,7 @@ struct ugu_hip_ctx {
   bool rt_bins = false;      // few enough layers of faces for the binned path
   int32_t rt_cap = 1024;     // entries per tile of the raytracer's bins
   int clean_tiles = 0;  // leading tile counters known to be clear, of view 0
+  CopyRing ring;                 // pinned slots of the copies to and from host arrays
   void* h_views = nullptr;
   size_t h_views_bytes = 0;
   int32_t* h_status = nullptr;  // pinned: [0] overflow flag / occupancy, [4] item total
@@ -486,6 +488,25 @@ void fill_view_camera(DevView& v, const UguCamera& cam, int tw, int th, int32_t 
   v.tile_base = tile_base;
 }
 
+// The copies of the planes staged for host memory (offsets >= 0).
+std::vector<HostCopy> staged_copies(ugu_hip_ctx* c, const UguCamera* cams, int n,
+                                    const UguOutputs* outs, const UguGBuffer* gbufs,
+                                    const std::vector<int64_t>& stage_off) {
+  std::vector<HostCopy> copies;
+  for (int i = 0; i < n; i++) {
+    const int64_t px = int64_t(cams[i].width) * cams[i].height;
+    for (int k = 0; k < kPlanes; k++) {
+      const int64_t off = stage_off[size_t(i) * kPlanes + k];
+      if (off < 0) continue;
+      void* dst[kPlanes];
+      plane_ptrs(outs[i], gbufs ? &gbufs[i] : nullptr, dst);
+      copies.push_back(
+          HostCopy{dst[k], c->stage_out.as<uint8_t>() + off, size_t(kPlaneBytes[k] * px)});
+    }
+  }
+  return copies;
+}
+
 int run_pipeline(ugu_hip_ctx* c, const UguCamera* cams, int n, const DevMesh& dm,
                  const DevOptions& dopt, int mode, const UguOutputs* outs,
                  int memory, float* const* images, int32_t* const* fids,
@@ -520,6 +541,8 @@ int run_pipeline(ugu_hip_ctx* c, const UguCamera* cams, int n, const DevMesh& dm
   if ((err = ensure(c, c->status, kStatusBytes))) return err;
   if ((err = ensure(c, c->views, size_t(n) * sizeof(DevView)))) return err;
   if (stage_bytes > 0 && (err = ensure(c, c->stage_out, size_t(stage_bytes)))) return err;
+  const std::vector<HostCopy> copies = staged_copies(c, cams, n, outs, gbufs, stage_off);
+  const Prefault prefault(copies.data(), static_cast<int>(copies.size()));
   const size_t view_bytes = size_t(n) * sizeof(DevView);
   if (c->h_views_bytes < view_bytes) {
     if (c->h_views) (void)hipHostFree(c->h_views);
@@ -613,21 +636,8 @@ int run_pipeline(ugu_hip_ctx* c, const UguCamera* cams, int n, const DevMesh& dm
     if (attempt == 7) return fail(c, UGU_HIP_ERR_OUT_OF_MEMORY, "bin capacity did not converge");
   }
 
-  if (mode == 0 && memory == UGU_HIP_MEMORY_HOST) {
-    const uint8_t* sb = c->stage_out.as<uint8_t>();
-    for (int i = 0; i < n; i++) {
-      const int64_t px = int64_t(cams[i].width) * cams[i].height;
-      void* dst[kPlanes];
-      plane_ptrs(outs[i], gbufs ? &gbufs[i] : nullptr, dst);
-      for (int k = 0; k < kPlanes; k++) {
-        const int64_t off = stage_off[size_t(i) * kPlanes + k];
-        if (off >= 0)
-          UGU_HIP_CHECK(c, hipMemcpyAsync(dst[k], sb + off, size_t(kPlaneBytes[k] * px),
-                                          hipMemcpyDeviceToHost, c->stream));
-      }
-    }
-    UGU_HIP_CHECK(c, hipStreamSynchronize(c->stream));
-  }
+  if (!copies.empty())
+    UGU_HIP_CHECK(c, c->ring.to_host(c->stream, copies.data(), static_cast<int>(copies.size())));
   return UGU_HIP_OK;
 }
 
@@ -941,6 +951,8 @@ int raytrace_common(ugu_hip_ctx* c, const UguCamera* cams, int n, const UguOptio
   int err;
   if ((err = ensure(c, c->views, size_t(n) * sizeof(DevView)))) return err;
   if (stage_bytes > 0 && (err = ensure(c, c->stage_out, size_t(stage_bytes)))) return err;
+  const std::vector<HostCopy> copies = staged_copies(c, cams, n, outs, nullptr, stage_off);
+  const Prefault prefault(copies.data(), static_cast<int>(copies.size()));
   const size_t view_bytes = size_t(n) * sizeof(DevView);
   if (c->h_views_bytes < view_bytes) {
     if (c->h_views) (void)hipHostFree(c->h_views);
@@ -991,20 +1003,8 @@ int raytrace_common(ugu_hip_ctx* c, const UguCamera* cams, int n, const UguOptio
       return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
   }
   if (c->profile) (void)hipEventRecord(c->ev[1], c->stream);
-  if (memory == UGU_HIP_MEMORY_HOST) {
-    const uint8_t* sb = c->stage_out.as<uint8_t>();
-    for (int i = 0; i < n; i++) {
-      const int64_t px = int64_t(cams[i].width) * cams[i].height;
-      void* dst[kPlanes];
-      plane_ptrs(outs[i], nullptr, dst);
-      for (int k = 0; k < kPlanes; k++) {
-        const int64_t off = stage_off[size_t(i) * kPlanes + k];
-        if (off >= 0)
-          UGU_HIP_CHECK(c, hipMemcpyAsync(dst[k], sb + off, size_t(kPlaneBytes[k] * px),
-                                          hipMemcpyDeviceToHost, c->stream));
-      }
-    }
-  }
+  if (!copies.empty())
+    UGU_HIP_CHECK(c, c->ring.to_host(c->stream, copies.data(), static_cast<int>(copies.size())));
   UGU_HIP_CHECK(c, hipStreamSynchronize(c->stream));
   if (c->profile) {
     float ms = 0.0f;
@@ -1068,6 +1068,7 @@ void ugu_hip_destroy(ugu_hip_ctx* c) {
                     &c->bvh_nodes, &c->bvh_leaves, &c->bvh_tris, &c->vis_items,
                     &c->vis_images, &c->vis_out, &c->tm_faces, &c->tm_images, &c->tm_out};
   for (DevBuf* b : bufs) b->release();
+  c->ring.release();
   if (c->h_views) (void)hipHostFree(c->h_views);
   if (c->h_status) (void)hipHostFree(c->h_status);
   for (auto& e : c->ev)
@@ -1345,26 +1346,28 @@ int ugu_hip_visibility_test(ugu_hip_ctx* c, const UguKeyframe* kf, const UguVisi
   UGU_HIP_CHECK(c, hipSetDevice(c->device));
   if (int oe = order_after_user(c)) return oe;
   const size_t px = size_t(kf->width) * size_t(kf->height);
-  const size_t item_bytes = size_t(n) * 12;
+  const size_t item_bytes = size_t(n) * 12, item_stride = (item_bytes + 15) / 16 * 16;
   int err;
-  if ((err = ensure(c, c->vis_items, item_bytes * 3))) return err;
+  if ((err = ensure(c, c->vis_items, item_stride * 3))) return err;
   if ((err = ensure(c, c->vis_images, px * 8 + 512))) return err;  // colour, depth, mask
   if ((err = ensure(c, c->vis_out, size_t(n) * sizeof(UguVertexVisibility)))) return err;
   uint8_t* items = c->vis_items.as<uint8_t>();
   uint8_t* img = c->vis_images.as<uint8_t>();
-  const size_t depth_off = (px * 3 + 255) / 256 * 256, mask_off = depth_off + px * 4;
-  UGU_HIP_CHECK(c, hipMemcpyAsync(items, item_pos, item_bytes, hipMemcpyHostToDevice, c->stream));
-  UGU_HIP_CHECK(c, hipMemcpyAsync(items + item_bytes, item_vertex, item_bytes,
-                                  hipMemcpyHostToDevice, c->stream));
-  UGU_HIP_CHECK(c, hipMemcpyAsync(items + 2 * item_bytes, item_normal, item_bytes,
-                                  hipMemcpyHostToDevice, c->stream));
-  UGU_HIP_CHECK(c, hipMemcpyAsync(img, kf->color, px * 3, hipMemcpyHostToDevice, c->stream));
-  if (o->use_depth)
-    UGU_HIP_CHECK(c, hipMemcpyAsync(img + depth_off, kf->depth, px * 4, hipMemcpyHostToDevice,
-                                    c->stream));
-  if (o->use_mask)
-    UGU_HIP_CHECK(c, hipMemcpyAsync(img + mask_off, kf->mask, px, hipMemcpyHostToDevice,
-                                    c->stream));
+  const size_t depth_off = (px * 3 + 255) / 256 * 256,
+               mask_off = (depth_off + px * 4 + 15) / 16 * 16;
+  const HostCopy result{out, c->vis_out.p, size_t(n) * sizeof(UguVertexVisibility)};
+  const Prefault prefault(&result, 1);
+  auto in = [](const void* host, uint8_t* dev, size_t bytes) {
+    return HostCopy{const_cast<void*>(host), dev, bytes};
+  };
+  HostCopy copies[6] = {in(item_pos, items, item_bytes),
+                        in(item_vertex, items + item_stride, item_bytes),
+                        in(item_normal, items + 2 * item_stride, item_bytes),
+                        in(kf->color, img, px * 3)};
+  int n_copies = 4;
+  if (o->use_depth) copies[n_copies++] = in(kf->depth, img + depth_off, px * 4);
+  if (o->use_mask) copies[n_copies++] = in(kf->mask, img + mask_off, px);
+  UGU_HIP_CHECK(c, c->ring.to_device(c->stream, copies, n_copies));
   DevView v;
   std::memset(&v, 0, sizeof(v));
   v.W = kf->width;
@@ -1390,14 +1393,11 @@ int ugu_hip_visibility_test(ugu_hip_ctx* c, const UguKeyframe* kf, const UguVisi
   bvh.nodes = c->bvh_nodes.as<BvhNode>();
   bvh.leaves = c->bvh_leaves.as<int2>();
   bvh.tris = c->bvh_tris.as<float4>();
-  const float* ip = reinterpret_cast<const float*>(items);
+  auto item = [&](int k) { return reinterpret_cast<const float*>(items + size_t(k) * item_stride); };
   if (launch_visibility(c->stream, v, img, reinterpret_cast<const float*>(img + depth_off),
-                        img + mask_off, d, n, ip, ip + size_t(n) * 3, ip + size_t(n) * 6, bvh,
-                        c->vis_out.p))
+                        img + mask_off, d, n, item(0), item(1), item(2), bvh, c->vis_out.p))
     return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
-  UGU_HIP_CHECK(c, hipMemcpyAsync(out, c->vis_out.p, size_t(n) * sizeof(UguVertexVisibility),
-                                  hipMemcpyDeviceToHost, c->stream));
-  UGU_HIP_CHECK(c, hipStreamSynchronize(c->stream));
+  UGU_HIP_CHECK(c, c->ring.to_host(c->stream, &result, 1));
   return UGU_HIP_OK;
 }
 
@@ -1432,32 +1432,31 @@ int ugu_hip_texture_map(ugu_hip_ctx* c, const UguTexture* images, int n_images,
   if ((err = ensure(c, c->tm_images, desc_bytes + off[size_t(n_images)] + 16))) return err;
   // owner (int32), unpadded texture + mask, padded texture + mask
   const size_t o_tex0 = texels * 4, o_mask0 = o_tex0 + texels * 3,
-               o_tex = (o_mask0 + texels + 255) / 256 * 256, o_mask = o_tex + texels * 3;
+               o_tex = (o_mask0 + texels + 255) / 256 * 256,
+               o_mask = (o_tex + texels * 3 + 15) / 16 * 16;
   if ((err = ensure(c, c->tm_out, o_mask + texels))) return err;
+  uint8_t* ob = c->tm_out.as<uint8_t>();
+  const HostCopy result[2] = {{texture, ob + o_tex, texels * 3}, {mask, ob + o_mask, texels}};
+  const Prefault prefault(result, 2);
   uint8_t* ib = c->tm_images.as<uint8_t>();
   std::vector<Img> desc(static_cast<size_t>(n_images));
+  std::vector<HostCopy> in;
   for (int i = 0; i < n_images; i++) {
     desc[size_t(i)] = Img{images[i].width, images[i].height, ib + desc_bytes + off[size_t(i)]};
-    UGU_HIP_CHECK(c, hipMemcpyAsync(ib + desc_bytes + off[size_t(i)], images[i].data,
-                                    size_t(images[i].width) * size_t(images[i].height) * 3,
-                                    hipMemcpyHostToDevice, c->stream));
+    in.push_back(HostCopy{const_cast<uint8_t*>(images[i].data), ib + desc_bytes + off[size_t(i)],
+                          size_t(images[i].width) * size_t(images[i].height) * 3});
   }
-  if (n_images > 0)
-    UGU_HIP_CHECK(c, hipMemcpyAsync(ib, desc.data(), desc.size() * sizeof(Img),
-                                    hipMemcpyHostToDevice, c->stream));
+  if (n_images > 0) in.push_back(HostCopy{desc.data(), ib, desc.size() * sizeof(Img)});
   if (n_faces > 0)
-    UGU_HIP_CHECK(c, hipMemcpyAsync(c->tm_faces.p, faces, size_t(n_faces) * sizeof(UguTexFace),
-                                    hipMemcpyHostToDevice, c->stream));
-  uint8_t* ob = c->tm_out.as<uint8_t>();
+    in.push_back(HostCopy{const_cast<UguTexFace*>(faces), c->tm_faces.p,
+                          size_t(n_faces) * sizeof(UguTexFace)});
+  UGU_HIP_CHECK(c, c->ring.to_device(c->stream, in.data(), static_cast<int>(in.size())));
   UGU_HIP_CHECK(c, hipMemsetAsync(ob + o_tex0, 0, texels * 4, c->stream));  // texture0 + mask0
   if (launch_texture_map(c->stream, c->tm_faces.p, n_faces, ib, tex_w, tex_h, padding_kernel / 2,
                          reinterpret_cast<int32_t*>(ob), ob + o_tex0, ob + o_mask0, ob + o_tex,
                          ob + o_mask))
     return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
-  UGU_HIP_CHECK(c, hipMemcpyAsync(texture, ob + o_tex, texels * 3, hipMemcpyDeviceToHost,
-                                  c->stream));
-  UGU_HIP_CHECK(c, hipMemcpyAsync(mask, ob + o_mask, texels, hipMemcpyDeviceToHost, c->stream));
-  UGU_HIP_CHECK(c, hipStreamSynchronize(c->stream));
+  UGU_HIP_CHECK(c, c->ring.to_host(c->stream, result, 2));
   return UGU_HIP_OK;
 }
 

@@ -27,16 +27,18 @@ kMaxArea; texture_mapper.cc:924-967), then builds the texture for the uv type:
 
 The result becomes the mesh's single material.
 """
+import atexit
 import collections
 import ctypes
 import enum
 import math
+import os
 import sys
 
 import numpy as np
 
 from . import _abi
-from .visibility import FaceInfo
+from .visibility import FaceInfo, contiguous_u8
 
 
 class ViewSelectionCriteria(enum.IntEnum):
@@ -129,14 +131,38 @@ def face_records(mesh, best, tex_w, tex_h):
     return recs, n
 
 
+# One idle context per device, for the next texture_map_faces call: creating and
+# destroying a context with its workspace takes 400 us of the 1.1 ms of a
+# 1024 x 1024 call. A call takes the context out and puts it back, so calls of
+# several threads never share one; it is kept only while its workspace is small,
+# not across a fork, and given back at exit.
+_SPARE_BYTES = 256 << 20
+_spare = {}
+
+
+def _give_context(lib, device, ctx, workspace_bytes):
+    if workspace_bytes > _SPARE_BYTES or _spare.setdefault((os.getpid(), device), ctx) != ctx:
+        lib.ugu_hip_destroy(ctx)
+
+
+@atexit.register
+def _release_spares():
+    for key in list(_spare):
+        ctx = _spare.pop(key, None)
+        if ctx and key[0] == os.getpid():
+            _abi.load_library().ugu_hip_destroy(ctx)
+
+
 def texture_map_faces(images, recs, n, tex_w, tex_h, padding_kernel, device=0):
     """ugu_hip_texture_map -> (texture (tex_h, tex_w, 3) uint8, mask)."""
     lib = _abi.load_library()
-    ctx = lib.ugu_hip_create(int(device))
+    device = int(device)
+    ctx = _spare.pop((os.getpid(), device), None) or lib.ugu_hip_create(device)
     if not ctx:
         raise RuntimeError(f"ugu_hip_create({device}) failed: no usable HIP device")
+    workspace = sys.maxsize  # not kept after an error
     try:
-        imgs = [np.ascontiguousarray(im, np.uint8) for im in images]
+        imgs = [contiguous_u8(im) for im in images]
         tex_arr = (_abi.UguTexture * max(1, len(imgs)))()
         for i, im in enumerate(imgs):
             tex_arr[i] = _abi.UguTexture(im.shape[1], im.shape[0], im.ctypes.data)
@@ -146,9 +172,11 @@ def texture_map_faces(images, recs, n, tex_w, tex_h, padding_kernel, device=0):
                                      padding_kernel, tex.ctypes.data, mask.ctypes.data)
         if rc != 0:
             raise _abi.HipError(rc, lib.ugu_hip_last_error(ctx).decode())
+        # images, records, and the owner, texture and mask planes
+        workspace = sum(im.size for im in imgs) + ctypes.sizeof(recs) + 13 * tex_w * tex_h
         return tex, mask
     finally:
-        lib.ugu_hip_destroy(ctx)
+        _give_context(lib, device, ctx, workspace)
 
 
 def simple_tile(keyframes, best, mesh, option):
