@@ -203,13 +203,6 @@ struct BwdLds {
   int32_t vkey[kVtx];
 };
 
-// 1 / a: the hardware estimate and two Newton steps (within 2 ulp).
-UGU_DEV double recip(double a) {
-  double r = __builtin_amdgcn_rcp(a);
-  r = __builtin_fma(__builtin_fma(-a, r, 1.0), r, r);
-  return __builtin_fma(__builtin_fma(-a, r, 1.0), r, r);
-}
-
 // First slot of a texel: four neighbouring texels of a row take neighbouring
 // slots, so that the flush writes them together; the quadruples are spread.
 template <int SLOTS>
@@ -230,12 +223,6 @@ UGU_DEV int find_slot(int32_t* keys, int h, int key) {
     if (h >= SLOTS) h -= SLOTS;
   }
   return -1;
-}
-
-UGU_DEV int clamp_cell(double v, int hi) {
-  if (!(v >= 0.0)) return 0;
-  if (v > static_cast<double>(hi)) return hi;
-  return static_cast<int>(v);
 }
 
 // Adds 9 values (3 per corner) to the LDS sums of their corners' vertices.

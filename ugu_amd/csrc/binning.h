@@ -18,10 +18,6 @@ constexpr int kSetupViews = 8;
 // per view.
 constexpr int kAppendRounds = 4;
 
-// Chunks whose faces all have at most this many (face, pixel) pairs expand
-// them through an LDS pair list; otherwise by binary search over the prefix.
-constexpr int kScatterMaxPairs = 32;
-
 // Faces whose pixel bbox holds at most this many pixel centres are tested at
 // those centres before they are binned.
 constexpr int kCoverProbe = 4;
@@ -125,6 +121,97 @@ UGU_DEV int2 bin_entry(const int2* bin, int nA, int cap, int i) {
 // True when the tile's current depth bound proves the face hidden.
 UGU_DEV bool skip_face(float zskip, float dmax) {
   return dmax >= 1e-18f && zskip > dmax * 1.00390625f;
+}
+
+// (face, pixel) pairs of a tile's chunk of NT staged faces (NT threads, one face
+// slot each), numbered slot by slot.
+template <int NT>
+struct PairLds {
+  uint16_t pre[NT];          // pairs before the slot's among its wavefront's slots
+  int32_t wsum[2][NT / 64];  // pairs of each wavefront's slots, by chunk parity
+  int32_t mark[NT];          // starts of the faces of a wavefront's 64 pairs
+  uint16_t queue[2 * NT];    // a wavefront's pairs that passed the first test
+};
+
+// Publishes this thread's pair count; a barrier and walk_pairs follow. The
+// parity of the chunk keeps a wavefront that has gone on to the next chunk from
+// overwriting the sums that a slower one still reads.
+template <int NT>
+UGU_DEV void publish_pairs(PairLds<NT>& s, int parity, int c) {
+  const int x = wave_incl_sum(c);
+  s.pre[threadIdx.x] = static_cast<uint16_t>(x - c);  // at most 64 NT - 1
+  if ((threadIdx.x & 63) == 63) s.wsum[parity][threadIdx.x >> 6] = x;
+}
+
+// Runs first(slot, r, pix) for every pair (r: the pair's index in its face,
+// 0 <= r < NT; it sets the tile pixel) and second(slot, pix) for those where first
+// returned true, 64 of them at a time. Returns the number of pairs.
+// Each wavefront takes 64 consecutive pairs at a time without the others: every
+// lane holds the first pairs of NT / 64 slots, marks those in the wavefront's
+// window at their place in LDS, and a running maximum carries each mark to the
+// pairs of its face. The cost does not depend on the faces' sizes (a list that
+// each face's thread writes costs the largest face's pairs, a binary search per
+// pair eight dependent LDS reads), and no barrier lies between two windows.
+template <int NT, class First, class Second>
+UGU_DEV int walk_pairs(PairLds<NT>& s, int parity, First first, Second second) {
+  constexpr int K = NT / 64;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  int base = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < K; w++) {
+    if (w < lane * K / 64) base += s.wsum[parity][w];
+    total += s.wsum[parity][w];
+  }
+  if (total == 0) return 0;
+  int q[K + 1];
+#pragma unroll
+  for (int k = 0; k < K; k++) q[k] = base + s.pre[lane * K + k];
+  q[K] = __shfl_down(q[0], 1);
+  if (lane == 63) q[K] = total;
+  int32_t* mark = s.mark + wid * 64;
+  uint16_t* queue = s.queue + wid * 128;
+  int queued = 0;
+  for (int g = wid * 64; g < total; g += NT) {
+    // mark = slot << 17 | (first pair - g + 65536); a face that starts before the
+    // window marks its first place
+    mark[lane] = 0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+    for (int k = 0; k < K; k++)
+      if (q[k] < q[k + 1] && q[k + 1] > g && q[k] < g + 64)
+        mark[max(q[k] - g, 0)] = ((lane * K + k) << 17) | (q[k] - g + 65536);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const int m = wave_incl_max(mark[lane]);
+    const int j = m >> 17;
+    int pix = 0;
+    const bool keep = g + lane < total && first(j, lane + 65536 - (m & 0x1ffff), pix);
+    const uint64_t kept = __builtin_amdgcn_ballot_w64(keep);
+    if (keep)
+      queue[queued + static_cast<int>(__builtin_amdgcn_mbcnt_hi(
+                         static_cast<uint32_t>(kept >> 32),
+                         __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(kept), 0u)))] =
+          static_cast<uint16_t>(j | (pix << 8));
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    queued += __popcll(kept);
+    if (queued >= 64) {
+      queued -= 64;
+      const int e = queue[queued + lane];
+      second(e & 0xff, e >> 8);
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  if (lane < queued) {
+    const int e = queue[lane];
+    second(e & 0xff, e >> 8);
+  }
+  return total;
+}
+
+// Row of pair r in a box nx pixels wide (r, nx < 1024): r / nx, as the quotient
+// of r + 1/2 is at least 1 / (2 nx) away from an integer.
+UGU_DEV int pair_row(int r, int nx) {
+  return static_cast<int>((static_cast<float>(r) + 0.5f) *
+                          __builtin_amdgcn_rcpf(static_cast<float>(nx)));
 }
 
 }  // namespace ugu_hip

@@ -136,6 +136,19 @@ UGU_DEV float edge_fn(float ax, float ay, float bx, float by, float cx, float cy
   return (cx - ax) * (by - ay) - (cy - ay) * (bx - ax);
 }
 
+// 1 / a: the hardware estimate and two Newton steps (within 2 ulp).
+UGU_DEV double recip(double a) {
+  double r = __builtin_amdgcn_rcp(a);
+  r = __builtin_fma(__builtin_fma(-a, r, 1.0), r, r);
+  return __builtin_fma(__builtin_fma(-a, r, 1.0), r, r);
+}
+
+UGU_DEV int clamp_cell(double v, int hi) {
+  if (!(v >= 0.0)) return 0;
+  if (v > static_cast<double>(hi)) return hi;
+  return static_cast<int>(v);
+}
+
 // float -> int32 as x86-64 cvttss2si (what the reference's static_cast
 // compiles to): truncation, INT32_MIN for NaN and out-of-range values.
 UGU_DEV int32_t f2i_x86(float f) {

@@ -503,12 +503,8 @@ struct RasterLds {
   float ray[3][NT];            // ray_w of each tile pixel
   float fv[13][NT];            // staged faces: 3 projected verts, area, face normal
   int32_t fid[NT];
-  int32_t box[NT];             // lx0 | ly0 << 8 | nx << 16 (tile-local pixel bbox)
-  // exclusive prefix of pair counts (binary-search expansion) or the
-  // (face slot | pair index << 8) list of one round (pair-list expansion)
-  int32_t pairs[2 * NT + 1];
-  int32_t wsum[NT / 64 + 1];
-  int32_t wbig[NT / 64];       // per-wave largest pair count of a face
+  uint16_t box[NT];            // lx0 | ly0 << 5 | (nx - 1) << 10 (tile-local pixel bbox)
+  PairLds<NT> pairs;
   uint32_t flag[NT / 32];      // pixel saw a depth outside [FLT_MIN, inf] (bit per pixel)
   uint32_t wmax[NT / 64];       // per-wave max of the pixels' depth bits
   int32_t any_flag;
@@ -605,123 +601,74 @@ UGU_DEV void sequential_pixel(const DevView& v, const DevMesh& mesh,
 }
 
 
-// Bilinear sample of an f32 RGB texture with clamp-to-edge addressing
-// (differentiable path). Returns the top-left texel and the local weights.
-UGU_DEV void ftex_coords(int tw, int th, float iu, float iv, int& x0, int& y0,
-                         int& x1, int& y1, float& lu, float& lv) {
-  const float fx = iu * static_cast<float>(tw - 1);
-  const float fy = (1.0f - iv) * static_cast<float>(th - 1);
-  const float flx = floorf(fx), fly = floorf(fy);
-  lu = fx - flx;
-  lv = fy - fly;
-  int ix = f2i_sat(flx), iy = f2i_sat(fly);
-  x0 = min(max(ix, 0), tw - 1);
-  y0 = min(max(iy, 0), th - 1);
-  x1 = min(max(ix + 1, 0), tw - 1);
-  y1 = min(max(iy + 1, 0), th - 1);
-}
-
-// ---------------------------------------------------------------------------
-// Differentiable image model, evaluated in float64 for one pixel of a given
-// face (visibility comes from the float32 rasterizer; the shading and its
-// derivatives are computed in double so the gradients match the exact model,
-// not the reference's float32 rounding of thin triangles).
-
-struct DiffEval {
-  double X[3], Y[3], iZ[3], Qx[3], Qy[3];  // iZ = 1 / camera depth
-  double e[3], A, iA, q[3], s, is, b0, b1, b2;
-  double c[3], t[3], dcdu[3], dcdv[3], dtdu[3], dtdv[3];
-  double lu, lv;
-  int tx0, ty0, tx1, ty1;
-};
-
-UGU_DEV int clamp_texel(double v, int hi) {
-  if (!(v >= 0.0)) return 0;
-  if (v > static_cast<double>(hi)) return hi;
-  return static_cast<int>(v);
-}
-
-UGU_DEV void diff_eval(const DevView& v, const DevMesh& m, int fid, int px, int py,
-                       const int32_t* vid, DiffEval& e) {
-  const double x = px, y = py;
-  for (int i = 0; i < 3; i++) {
-    const float* P = m.verts + int64_t(vid[i]) * 3;
-    double Q[3];
-    for (int r = 0; r < 3; r++)
-      Q[r] = double(v.w2c_R[r * 3 + 0]) * P[0] + double(v.w2c_R[r * 3 + 1]) * P[1] +
-             double(v.w2c_R[r * 3 + 2]) * P[2] + double(v.w2c_t[r]);
-    e.Qx[i] = Q[0];
-    e.Qy[i] = Q[1];
-    e.iZ[i] = 1.0 / Q[2];
-    e.X[i] = double(v.fx) * Q[0] * e.iZ[i] + double(v.cx);
-    e.Y[i] = double(v.fy) * Q[1] * e.iZ[i] + double(v.cy);
+// Differentiable image model in float64 for one covered pixel: colour term times
+// texture term (visibility comes from the float32 rasterizer; in double, so that
+// the image matches the exact model, not the float32 rounding of thin triangles).
+// With x, y the corners' camera positions sheared so that the pixel's ray is their
+// z axis (x = fx Qx - (px - cx) Qz, y likewise), the perspective-correct weight of
+// a corner is proportional to the cross product of the other two.
+// The arrays are gathered by index: on a mesh of a face per pixel they are 40
+// bytes a face, the face and shading records 112, and the gathers' L2 misses bound
+// the pass (64 views of 1.3 M faces: 1011 against 1038 us). The model without the
+// derivatives and without the corners' screen positions needs 40 float64
+// operations instead of 130 and no spilled registers: 1003 -> 895 us. (In a kernel
+// of its own after k_raster: 624 + 639 us.)
+UGU_DEV void diff_image(const DevView& v, const DevMesh& m, int fid, int px, int py, float img[3]) {
+#pragma clang fp contract(fast)
+  int32_t vid[3], uid[3] = {0, 0, 0};
+  for (int j = 0; j < 3; j++) vid[j] = m.faces[int64_t(fid) * 3 + j];
+  if (m.ftex)
+    for (int j = 0; j < 3; j++) uid[j] = m.uvidx[int64_t(fid) * 3 + j];
+  const double u = px - static_cast<double>(v.cx), w = py - static_cast<double>(v.cy);
+  double ax[4], ay[4];
+  for (int k = 0; k < 4; k++) {
+    const double c0 = k < 3 ? v.w2c_R[k] : v.w2c_t[0], c1 = k < 3 ? v.w2c_R[3 + k] : v.w2c_t[1],
+                 c2 = k < 3 ? v.w2c_R[6 + k] : v.w2c_t[2];
+    ax[k] = v.fx * c0 - u * c2;
+    ay[k] = v.fy * c1 - w * c2;
   }
-  auto E = [](double ax, double ay, double bx, double by, double cx, double cy) {
-    return (cx - ax) * (by - ay) - (cy - ay) * (bx - ax);
-  };
-  e.A = E(e.X[0], e.Y[0], e.X[1], e.Y[1], e.X[2], e.Y[2]);
-  e.e[0] = E(e.X[1], e.Y[1], e.X[2], e.Y[2], x, y);
-  e.e[1] = E(e.X[2], e.Y[2], e.X[0], e.Y[0], x, y);
-  e.e[2] = E(e.X[0], e.Y[0], e.X[1], e.Y[1], x, y);
-  // reciprocals once, then products: the model is evaluated in float64 and
-  // compared with a float64 reference, so a few ulps of rounding are free
-  e.iA = 1.0 / e.A;
-  for (int i = 0; i < 3; i++) e.q[i] = e.e[i] * e.iA * e.iZ[i];
-  e.s = e.q[0] + e.q[1] + e.q[2];
-  e.is = 1.0 / e.s;
-  e.b1 = e.q[1] * e.is;
-  e.b2 = e.q[2] * e.is;
-  e.b0 = 1.0 - e.b1 - e.b2;
-  for (int k = 0; k < 3; k++) {
-    e.c[k] = 1.0;
-    e.t[k] = 1.0;
-    e.dcdu[k] = e.dcdv[k] = e.dtdu[k] = e.dtdv[k] = 0.0;
+  double X[3], Y[3];
+  for (int j = 0; j < 3; j++) {
+    const float* P = m.verts + int64_t(vid[j]) * 3;
+    const double p0 = P[0], p1 = P[1], p2 = P[2];
+    X[j] = ax[0] * p0 + ax[1] * p1 + ax[2] * p2 + ax[3];
+    Y[j] = ay[0] * p0 + ay[1] * p1 + ay[2] * p2 + ay[3];
   }
-  e.lu = e.lv = 0.0;
-  e.tx0 = e.ty0 = e.tx1 = e.ty1 = 0;
+  const double q0 = X[2] * Y[1] - X[1] * Y[2];
+  const double q1 = X[0] * Y[2] - X[2] * Y[0];
+  const double q2 = X[1] * Y[0] - X[0] * Y[1];
+  const double is = recip(q0 + q1 + q2);
+  const double b1 = q1 * is, b2 = q2 * is, b0 = 1.0 - b1 - b2;
+  double col[3] = {1.0, 1.0, 1.0};
   if (m.vcolors) {
-    const float* C0 = m.vcolors + int64_t(vid[0]) * 3;
-    const float* C1 = m.vcolors + int64_t(vid[1]) * 3;
-    const float* C2 = m.vcolors + int64_t(vid[2]) * 3;
-    for (int k = 0; k < 3; k++) {
-      e.c[k] = e.b0 * C0[k] + e.b1 * C1[k] + e.b2 * C2[k];
-      e.dcdu[k] = double(C1[k]) - C0[k];
-      e.dcdv[k] = double(C2[k]) - C0[k];
-    }
+    const float* ca = m.vcolors + int64_t(vid[0]) * 3;
+    const float* cb = m.vcolors + int64_t(vid[1]) * 3;
+    const float* cc = m.vcolors + int64_t(vid[2]) * 3;
+    for (int k = 0; k < 3; k++) col[k] = b0 * ca[k] + b1 * cb[k] + b2 * cc[k];
   }
   if (m.ftex) {
-    const int32_t* ui = m.uvidx + int64_t(fid) * 3;
-    const float* a = m.uv + int64_t(ui[0]) * 2;
-    const float* b = m.uv + int64_t(ui[1]) * 2;
-    const float* c = m.uv + int64_t(ui[2]) * 2;
-    const double iu = e.b0 * a[0] + e.b1 * b[0] + e.b2 * c[0];
-    const double iv = e.b0 * a[1] + e.b1 * b[1] + e.b2 * c[1];
+    const float* ua = m.uv + int64_t(uid[0]) * 2;
+    const float* ub = m.uv + int64_t(uid[1]) * 2;
+    const float* uc = m.uv + int64_t(uid[2]) * 2;
+    const double iu = b0 * ua[0] + b1 * ub[0] + b2 * uc[0];
+    const double iv = b0 * ua[1] + b1 * ub[1] + b2 * uc[1];
     const int tw = m.ftex_w, th = m.ftex_h;
     const double fxp = iu * (tw - 1), fyp = (1.0 - iv) * (th - 1);
     const double flx = floor(fxp), fly = floor(fyp);
-    e.lu = fxp - flx;
-    e.lv = fyp - fly;
-    e.tx0 = clamp_texel(flx, tw - 1);
-    e.ty0 = clamp_texel(fly, th - 1);
-    e.tx1 = clamp_texel(flx + 1.0, tw - 1);
-    e.ty1 = clamp_texel(fly + 1.0, th - 1);
-    const float* p00 = m.ftex + (int64_t(e.ty0) * tw + e.tx0) * 3;
-    const float* p01 = m.ftex + (int64_t(e.ty0) * tw + e.tx1) * 3;
-    const float* p10 = m.ftex + (int64_t(e.ty1) * tw + e.tx0) * 3;
-    const float* p11 = m.ftex + (int64_t(e.ty1) * tw + e.tx1) * 3;
-    const double sx = tw - 1, sy = -(th - 1.0);
-    const double dlu_du = sx * (double(b[0]) - a[0]), dlu_dv = sx * (double(c[0]) - a[0]);
-    const double dlv_du = sy * (double(b[1]) - a[1]), dlv_dv = sy * (double(c[1]) - a[1]);
-    const double lu = e.lu, lv = e.lv;
+    const double lu = fxp - flx, lv = fyp - fly;
+    const int tx0 = clamp_cell(flx, tw - 1), tx1 = clamp_cell(flx + 1.0, tw - 1);
+    const int ty0 = clamp_cell(fly, th - 1), ty1 = clamp_cell(fly + 1.0, th - 1);
+    const float* p00 = m.ftex + (int64_t(ty0) * tw + tx0) * 3;
+    const float* p01 = m.ftex + (int64_t(ty0) * tw + tx1) * 3;
+    const float* p10 = m.ftex + (int64_t(ty1) * tw + tx0) * 3;
+    const float* p11 = m.ftex + (int64_t(ty1) * tw + tx1) * 3;
     for (int k = 0; k < 3; k++) {
-      e.t[k] = (1 - lu) * (1 - lv) * p00[k] + lu * (1 - lv) * p01[k] +
-               (1 - lu) * lv * p10[k] + lu * lv * p11[k];
-      const double da = (1 - lv) * (double(p01[k]) - p00[k]) + lv * (double(p11[k]) - p10[k]);
-      const double db = (1 - lu) * (double(p10[k]) - p00[k]) + lu * (double(p11[k]) - p01[k]);
-      e.dtdu[k] = da * dlu_du + db * dlv_du;
-      e.dtdv[k] = da * dlu_dv + db * dlv_dv;
+      const double r0 = p00[k] + lu * (static_cast<double>(p01[k]) - p00[k]);
+      const double r1 = p10[k] + lu * (static_cast<double>(p11[k]) - p10[k]);
+      col[k] *= r0 + lv * (r1 - r0);
     }
   }
+  for (int k = 0; k < 3; k++) img[k] = static_cast<float>(col[k]);
 }
 
 // G-buffer planes of one pixel (see UguGBuffer in ugu_hip.h). u, v: the
@@ -767,7 +714,7 @@ UGU_DEV void write_gbuffer(const DevView& v, int64_t pidx, bool covered, float u
 
 // One screen tile; `seg` is the tile's counter record (front count, back
 // count, back-segment minimum skip depth, view index).
-template <int TW, int TH, int MODE>
+template <int TW, int TH, bool DIFF>
 UGU_DEV void raster_tile(RasterLds<TW * TH>& s, int gtile, const int4 seg, const DevView* views,
                          const DevMesh& mesh,
                          const DevBins& bins, const DevOptions& opt) {
@@ -791,15 +738,16 @@ UGU_DEV void raster_tile(RasterLds<TW * TH>& s, int gtile, const int4 seg, const
     // ValidateAndInitBeforeRender (util_private.cc:68-87)
     if (gx < v.W && gy < v.H) {
       const int64_t pidx = int64_t(gy) * v.W + gx;
-      if (MODE == 0) {
-        if (v.color) put3<S>(v.color, pidx, uint8_t(0), uint8_t(0), uint8_t(0));
-        if (v.depth) put<S>(v.depth, pidx, 0.0f);
-        if (v.normal) put3<S>(v.normal, pidx, 0.0f, 0.0f, 0.0f);
-        if (v.mask) put<S>(v.mask, pidx, uint8_t(0));
-        write_gbuffer<S>(v, pidx, false, 0.0f, 0.0f, false, nullptr, nullptr, 0.0f, 0.0f, 0.0f);
-      } else {
+      if (DIFF) {
         put3<S>(v.image, pidx, 0.0f, 0.0f, 0.0f);
+        put<S>(v.face_id, pidx, -1);
+        return;
       }
+      if (v.color) put3<S>(v.color, pidx, uint8_t(0), uint8_t(0), uint8_t(0));
+      if (v.depth) put<S>(v.depth, pidx, 0.0f);
+      if (v.normal) put3<S>(v.normal, pidx, 0.0f, 0.0f, 0.0f);
+      if (v.mask) put<S>(v.mask, pidx, uint8_t(0));
+      write_gbuffer<S>(v, pidx, false, 0.0f, 0.0f, false, nullptr, nullptr, 0.0f, 0.0f, 0.0f);
       if (v.face_id) put<S>(v.face_id, pidx, -1);
     }
     return;
@@ -815,13 +763,16 @@ UGU_DEV void raster_tile(RasterLds<TW * TH>& s, int gtile, const int4 seg, const
   int2 e_next = make_int2(0, 0);
   if (t < (chunks_a > 0 ? nA : n)) e_next = bin_entry(bin, nA, bins.cap, t);
 
-  float r0, r1, r2;
-  ray_w_at(v, static_cast<float>(gx), static_cast<float>(gy), r0, r1, r2);
+  // the rays stay in LDS: 72 registers leave no room for them in the pair loop
+  {
+    float r0, r1, r2;
+    ray_w_at(v, static_cast<float>(gx), static_cast<float>(gy), r0, r1, r2);
+    s.ray[0][t] = r0;
+    s.ray[1][t] = r1;
+    s.ray[2][t] = r2;
+  }
   s.key[t] = ~0ull;
   if (t < NT / 32) s.flag[t] = 0u;
-  s.ray[0][t] = r0;
-  s.ray[1][t] = r1;
-  s.ray[2][t] = r2;
   if (t == 0) s.any_flag = 0;
   // When face ids fit 24 bits the depth key also carries the LDS slot of the
   // face (below the id, so ties still go to the lowest id). After every chunk
@@ -878,7 +829,7 @@ UGU_DEV void raster_tile(RasterLds<TW * TH>& s, int gtile, const int4 seg, const
         if (lx0 <= lx1 && ly0 <= ly1) {
           const int nx = lx1 - lx0 + 1;
           c = nx * (ly1 - ly0 + 1);
-          s.box[t] = lx0 | (ly0 << 8) | (nx << 16);
+          s.box[t] = static_cast<uint16_t>(lx0 | (ly0 << 5) | ((nx - 1) << 10));
         }
       }
       s.fv[0][t] = a.x; s.fv[1][t] = a.y; s.fv[2][t] = a.z;
@@ -888,23 +839,8 @@ UGU_DEV void raster_tile(RasterLds<TW * TH>& s, int gtile, const int4 seg, const
       s.fv[10][t] = N[0]; s.fv[11][t] = N[1]; s.fv[12][t] = N[2];
       s.fid[t] = f;
     }
-    // block exclusive scan of the pair counts; a chunk without any pair
-    // (every face skipped or off the tile) ends at the barrier
-    const int lane = t & 63, wid = t >> 6;
-    const int x = wave_incl_sum(c);
-    const int cmax = wave_incl_max(c);
-    if (lane == 63) {
-      s.wsum[wid] = x;
-      s.wbig[wid] = cmax;
-    }
-    if (!__syncthreads_or(c > 0)) continue;
-    int wbase = 0, total = 0, big = 0;
-    for (int w = 0; w < NT / 64; w++) {
-      if (w < wid) wbase += s.wsum[w];
-      total += s.wsum[w];
-      big = max(big, s.wbig[w]);
-    }
-    const int pre = wbase + x - c;  // first pair of this thread's face
+    publish_pairs(s.pairs, ch & 1, c);
+    __syncthreads();
     const bool has_fn = mesh.fnormals != nullptr;
     // One (face slot, tile pixel) pair: coverage, depth and the packed LDS
     // atomicMin.
@@ -931,55 +867,26 @@ UGU_DEV void raster_tile(RasterLds<TW * TH>& s, int gtile, const int4 seg, const
         }
       }
     };
-    if (big <= kScatterMaxPairs) {
-      // small faces: every face writes its pairs (slot | tile pixel << 8)
-      // into an LDS list, then every lane takes one pair
-      for (int r0 = 0; r0 < total; r0 += 2 * NT) {
-        const int lo = max(pre, r0), hi = min(pre + c, r0 + 2 * NT);
-        if (lo < hi) {
-          const int bx = s.box[t];
-          const int nx = (bx >> 16) & 0xff, x0l = bx & 0xff;
-          int ry = (lo - pre) / nx;
-          int rx = (lo - pre) - ry * nx;
-          int pix = (((bx >> 8) & 0xff) + ry) * TW + x0l + rx;
-          for (int q = lo; q < hi; q++) {
-            s.pairs[q - r0] = t | (pix << 8);
-            if (++rx == nx) {
-              rx = 0;
-              pix += TW - nx + 1;
-            } else {
-              pix++;
-            }
-          }
-        }
-        __syncthreads();
-        const int np = min(total - r0, 2 * NT);
-        for (int pp = t; pp < np; pp += NT) {
-          const int pr = s.pairs[pp];
-          test_pair(pr & 0xff, pr >> 8);
-        }
-        __syncthreads();
-      }
-    } else {
-      // some face covers many pixels: binary search of the pair's face over
-      // the prefix (balanced whatever the face sizes)
-      s.pairs[t] = pre;
-      if (t == NT - 1) s.pairs[NT] = total;
-      __syncthreads();
-      for (int p = t; p < total; p += NT) {
-        int jl = 0, jh = NT - 1;
-        while (jl < jh) {
-          const int mid = (jl + jh + 1) >> 1;
-          if (s.pairs[mid] <= p) jl = mid; else jh = mid - 1;
-        }
-        const int r = p - s.pairs[jl];
-        const int bx = s.box[jl];
-        const int nx = (bx >> 16) & 0xff;
-        const int qy = r / nx;
-        test_pair(jl, (((bx >> 8) & 0xff) + qy) * TW + (bx & 0xff) + (r - qy * nx));
-      }
-      __syncthreads();
-    }
+    // Most pairs of a box are not covered: a pair first needs edge functions of
+    // one sign (cover_test's, same bits; a NaN only keeps it), and the pairs
+    // that pass are tested 64 at a time.
+    auto one_sign = [&](int j, int r, int& pix) {
+      const int bx = s.box[j];
+      const int nx = (bx >> 10) + 1;
+      const int qy = pair_row(r, nx);
+      const int pxl = (bx & 31) + (r - qy * nx), pyl = ((bx >> 5) & 31) + qy;
+      pix = pyl * TW + pxl;
+      const float x = static_cast<float>(px0 + pxl), y = static_cast<float>(py0 + pyl);
+      const float ax = s.fv[0][j], ay = s.fv[1][j], bx_ = s.fv[3][j], by = s.fv[4][j],
+                  cx = s.fv[6][j], cy = s.fv[7][j];
+      const float w0 = edge_fn(bx_, by, cx, cy, x, y);
+      const float w1 = edge_fn(cx, cy, ax, ay, x, y);
+      const float w2 = edge_fn(ax, ay, bx_, by, x, y);
+      return fminf(fminf(w0, w1), w2) >= 0.0f || fmaxf(fmaxf(w0, w1), w2) <= 0.0f;
+    };
+    // a chunk without any pair (every face skipped or off the tile) ends here
+    if (walk_pairs(s.pairs, ch & 1, one_sign, test_pair) == 0) continue;
+    __syncthreads();
     const unsigned long long k = s.key[t];
     if (more) {
       // depth bits of this pixel: all ones when it has no key yet, 0 outside
@@ -993,7 +900,8 @@ UGU_DEV void raster_tile(RasterLds<TW * TH>& s, int gtile, const int4 seg, const
       // record with the pair test's arithmetic (same bits), so the resolve
       // needs neither the record nor a second test
       const int sl = static_cast<int>(k & 0xffull);
-      wbf = has_fn && sum3(s.fv[10][sl] * r0, s.fv[11][sl] * r1, s.fv[12][sl] * r2) > 0.0f;
+      wbf = has_fn && sum3(s.fv[10][sl] * s.ray[0][t], s.fv[11][sl] * s.ray[1][t],
+                           s.fv[12][sl] * s.ray[2][t]) > 0.0f;
       cover_test(s.fv[0][sl], s.fv[1][sl], s.fv[2][sl], s.fv[3][sl], s.fv[4][sl], s.fv[5][sl],
                  s.fv[6][sl], s.fv[7][sl], s.fv[8][sl], s.fv[9][sl], wbf,
                  static_cast<float>(gx), static_cast<float>(gy), wz, ww0, ww1, ww2);
@@ -1011,6 +919,7 @@ UGU_DEV void raster_tile(RasterLds<TW * TH>& s, int gtile, const int4 seg, const
   // ---- resolve (rasterizer.cc:243-301) for this thread's pixel; the
   // winner's depth, weights and back-face flag are in registers (slot keys)
   // or computed again below
+  const float r0 = s.ray[0][t], r1 = s.ray[1][t], r2 = s.ray[2][t];
   int fid = -1;
   bool have = false;
   if (s.any_flag && ((s.flag[t >> 5] >> (t & 31)) & 1u)) {
@@ -1052,12 +961,19 @@ UGU_DEV void raster_tile(RasterLds<TW * TH>& s, int gtile, const int4 seg, const
   }
   const int64_t pidx = int64_t(gy) * v.W + gx;
 
-  if (MODE == 0) {
+  if (DIFF) {
+    // differentiable forward: image = colour term * texture term (float64)
+    float img[3] = {0.0f, 0.0f, 0.0f};
+    if (fid > 0) diff_image(v, mesh, fid, gx, gy, img);
+    put3<S>(v.image, pidx, img[0], img[1], img[2]);
+    put<S>(v.face_id, pidx, fid);
+  } else {
     uint8_t col[3] = {0, 0, 0};
     float nrm[3] = {0.0f, 0.0f, 0.0f};
     uint8_t msk = 0;
-    if (fid > 0) {
-      msk = 255;
+    const bool gbuf = v.bary || v.uvo || v.pos_wld || v.pos_cam || v.nrm_wld || v.geo_id;
+    if (fid > 0) msk = 255;
+    if (fid > 0 && (v.color || v.normal || gbuf)) {
       float n0, n1, n2;
       FaceShade fs;
       face_shade(mesh, fid, opt.shading_normal != 0, v.color && opt.diffuse_color == 1, fs);
@@ -1078,7 +994,7 @@ UGU_DEV void raster_tile(RasterLds<TW * TH>& s, int gtile, const int4 seg, const
         nrm[2] = sum3(v.w2c_R[6] * n0, v.w2c_R[7] * n1, v.w2c_R[8] * n2);
       }
       if (v.color) shade_u8(mesh, opt, fid, fs, w1, w2, r0, r1, r2, n0, n1, n2, col);
-      if (v.bary || v.uvo || v.pos_wld || v.pos_cam || v.nrm_wld || v.geo_id) {
+      if (gbuf) {
         // P is passed with a flag, not as a pointer that may be null: a select
         // between pointers would keep the array out of registers
         float P[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0}, N[3];
@@ -1087,23 +1003,13 @@ UGU_DEV void raster_tile(RasterLds<TW * TH>& s, int gtile, const int4 seg, const
         write_gbuffer<S>(v, pidx, true, w1, w2, pos, P,
                          v.uvo && mesh.uv && mesh.uvidx ? &mesh : nullptr, n0, n1, n2, fid);
       }
-    } else {
+    } else if (gbuf) {
       write_gbuffer<S>(v, pidx, false, 0.0f, 0.0f, false, nullptr, nullptr, 0.0f, 0.0f, 0.0f);
     }
     if (v.color) put3<S>(v.color, pidx, col[0], col[1], col[2]);
     if (v.depth) put<S>(v.depth, pidx, z);
     if (v.normal) put3<S>(v.normal, pidx, nrm[0], nrm[1], nrm[2]);
     if (v.mask) put<S>(v.mask, pidx, msk);
-    if (v.face_id) put<S>(v.face_id, pidx, fid);
-  } else {
-    // differentiable forward: image = colour term * texture term (float64)
-    float img[3] = {0.0f, 0.0f, 0.0f};
-    if (fid > 0) {
-      DiffEval e;
-      diff_eval(v, mesh, fid, gx, gy, mesh.faces + int64_t(fid) * 3, e);
-      for (int k = 0; k < 3; k++) img[k] = static_cast<float>(e.c[k] * e.t[k]);
-    }
-    put3<S>(v.image, pidx, img[0], img[1], img[2]);
     if (v.face_id) put<S>(v.face_id, pidx, fid);
   }
   // The tile's counters, cleared for the next pass (an empty tile's are clear).
@@ -1112,20 +1018,26 @@ UGU_DEV void raster_tile(RasterLds<TW * TH>& s, int gtile, const int4 seg, const
   if (t == 0) reinterpret_cast<int4*>(bins.counts)[gtile] = make_int4(0, 0, 0x7f800000, seg.w);
 }
 
-template <int TW, int TH, int MODE>
-// 7 waves per SIMD for the rendering kernels (72 VGPRs, no scratch; 7 blocks
-// of 22.9 KB fill the 160 KB of LDS), 6 for the differentiable forward, whose
-// extra saved values would spill at 72: the kernel is latency-bound
-// (dependent gathers, LDS round trips, barriers), so occupancy pays
-// (64-view batch: 0.90 -> 0.87 ms at 7).
-__global__ __launch_bounds__(TW * TH, MODE == 0 ? 7 : 6) void k_raster(
+template <int TW, int TH, bool DIFF>
+// A tile is a chain of dependent steps (counters, entries, face records, pairs,
+// the winners' shading inputs): a pass of one view ends with its slowest tile, a
+// pass of many is bound by how many tiles are in flight. So 7 waves per SIMD for
+// rendering (72 VGPRs; 7 blocks of 22.7 KB fill the 160 KB of LDS); the
+// differentiable forward needs 91 VGPRs and takes 5 (6 would spill: 896 against
+// 911 us for the case below).
+// Slowest tile of 1.3 M faces at 1080p: 130,000 cycles with its faces' pairs
+// written one by one by the faces' threads (93,000 of them in the pairs, silhouette
+// slivers), 65 -> 46 us for the kernel with walk_pairs; 640x480, 32 k faces:
+// 35 -> 22 us. 64 mixed views: 825 -> 815 us; differentiable forward of them
+// 1003 -> 895 us.
+__global__ __launch_bounds__(TW * TH, DIFF ? 5 : 7) void k_raster(
     const DevView* __restrict__ views, DevMesh mesh,
     DevBins bins, DevOptions opt,
     int persistent) {
   __shared__ RasterLds<TW * TH> s;
   if (!persistent) {
     const int gtile = xcd_remap(blockIdx.x, gridDim.x);
-    raster_tile<TW, TH, MODE>(s, gtile, reinterpret_cast<const int4*>(bins.counts)[gtile], views,
+    raster_tile<TW, TH, DIFF>(s, gtile, reinterpret_cast<const int4*>(bins.counts)[gtile], views,
                               mesh, bins, opt);
     return;
   }
@@ -1166,7 +1078,7 @@ __global__ __launch_bounds__(TW * TH, MODE == 0 ? 7 : 6) void k_raster(
     __syncthreads();
     for (int it = item; it < end; it++) {
       if (it == end - 1 && threadIdx.x == 0) s.item = claim();
-      raster_tile<TW, TH, MODE>(s, it, s.runseg[it - item], views, mesh, bins, opt);
+      raster_tile<TW, TH, DIFF>(s, it, s.runseg[it - item], views, mesh, bins, opt);
     }
     __syncthreads();
     item = s.item;
@@ -1251,27 +1163,17 @@ int launch_setup_bin(hipStream_t st, int tw, int th, const DevView* one, DevView
   return -2;
 }
 
-template <int TW, int TH, int MODE>
-static int launch_raster_t(hipStream_t st, const DevView* views,
-                           const DevMesh& mesh,
-                           const DevBins& bins, const DevOptions& opt,
+template <bool DIFF>
+static int launch_raster_t(hipStream_t st, int tw, int th, const DevView* views,
+                           const DevMesh& mesh, const DevBins& bins, const DevOptions& opt,
                            int persistent_blocks) {
-  if (bins.total_tiles <= 0) return 0;
   const int grid = persistent_blocks > 0 ? persistent_blocks : bins.total_tiles;
-  hipLaunchKernelGGL((k_raster<TW, TH, MODE>), dim3(grid), dim3(TW * TH), 0, st,
-                     views, mesh, bins, opt, persistent_blocks > 0 ? 1 : 0);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
-}
-
-int launch_raster(hipStream_t st, int tw, int th, int mode, const DevView* views,
-                  const DevMesh& mesh, const DevBins& bins,
-                  const DevOptions& opt, int persistent_blocks) {
-#define UGU_RASTER_CASE(TWV, THV)                                                  \
-  if (tw == TWV && th == THV)                                                      \
-    return mode == 0 ? launch_raster_t<TWV, THV, 0>(st, views, mesh, bins,   \
-                                                    opt, persistent_blocks)        \
-                     : launch_raster_t<TWV, THV, 1>(st, views, mesh, bins,   \
-                                                    opt, persistent_blocks);
+#define UGU_RASTER_CASE(TWV, THV)                                                              \
+  if (tw == TWV && th == THV) {                                                                \
+    hipLaunchKernelGGL((k_raster<TWV, THV, DIFF>), dim3(grid), dim3(TWV * THV), 0, st, views,  \
+                       mesh, bins, opt, persistent_blocks > 0 ? 1 : 0);                        \
+    return hipGetLastError() == hipSuccess ? 0 : -1;                                           \
+  }
   UGU_RASTER_CASE(8, 8)
   UGU_RASTER_CASE(16, 16)
   UGU_RASTER_CASE(32, 8)
@@ -1279,23 +1181,31 @@ int launch_raster(hipStream_t st, int tw, int th, int mode, const DevView* views
   return -2;
 }
 
-int raster_blocks_per_cu(int tw, int th, int mode) {
+int launch_raster(hipStream_t st, int tw, int th, int mode, const DevView* views,
+                  const DevMesh& mesh, const DevBins& bins, const DevOptions& opt,
+                  int persistent_blocks) {
+  if (bins.total_tiles <= 0) return 0;
+  return mode == 0
+             ? launch_raster_t<false>(st, tw, th, views, mesh, bins, opt, persistent_blocks)
+             : launch_raster_t<true>(st, tw, th, views, mesh, bins, opt, persistent_blocks);
+}
+
+template <bool DIFF>
+static int raster_occupancy(int tw, int th) {
   int nb = 0;
   hipError_t e = hipErrorInvalidValue;
-#define UGU_OCC_CASE(TWV, THV)                                                       \
-  if (tw == TWV && th == THV) {                                                      \
-    if (mode == 0)                                                                   \
-      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_raster<TWV, THV, 0>,   \
-                                                       TWV * THV, 0);                \
-    else                                                                             \
-      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_raster<TWV, THV, 1>,   \
-                                                       TWV * THV, 0);                \
-  }
+#define UGU_OCC_CASE(TWV, THV)                                                               \
+  if (tw == TWV && th == THV)                                                                \
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_raster<TWV, THV, DIFF>, TWV * THV, 0);
   UGU_OCC_CASE(8, 8)
   UGU_OCC_CASE(16, 16)
   UGU_OCC_CASE(32, 8)
 #undef UGU_OCC_CASE
   return e == hipSuccess ? nb : 0;
+}
+
+int raster_blocks_per_cu(int tw, int th, int mode) {
+  return mode == 0 ? raster_occupancy<false>(tw, th) : raster_occupancy<true>(tw, th);
 }
 
 int launch_depth_to_u16(hipStream_t st, const float* d, int64_t n, uint16_t* out) {

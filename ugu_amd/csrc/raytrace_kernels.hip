@@ -439,9 +439,7 @@ struct RtLds {
   float p[9][256];              // staged faces: corner positions
   int32_t fid[256];
   uint16_t box[256];            // rt_entry's pixel box
-  int32_t pairs[2 * 256 + 1];   // as RasterLds::pairs
-  int32_t wsum[4];
-  int32_t wbig[4];
+  PairLds<256> pairs;
   uint32_t wmax[4];
 };
 
@@ -455,8 +453,8 @@ struct RtLds {
 // rounding of either) is hit later than what each pixel holds.
 // Bound by the latency of a tile's dependent loads (counters, entries, face
 // records, the winner's record and shading inputs), like k_raster. 1.3 M faces
-// at 1080p: setup 26 us + tiles 61 us, where the hierarchy walk (k_raytrace)
-// takes 836 us; 24 mixed views of 492 k faces: 153 + 323 us against 2505 us.
+// at 1080p: setup 26 us + tiles 57 us, where the hierarchy walk (k_raytrace)
+// takes 836 us; 24 mixed views of 492 k faces: 153 + 330 us against 2505 us.
 __global__ __launch_bounds__(256) void k_rt_tiles(const DevView* __restrict__ views, DevMesh m,
                                                   DevBins bins, DevOptions o) {
   constexpr int NT = 256;
@@ -521,20 +519,8 @@ __global__ __launch_bounds__(256) void k_rt_tiles(const DevView* __restrict__ vi
         c = (((e.y >> 8) & 15) + 1) * (((e.y >> 12) & 15) + 1);
       }
       const int lane = t & 63, wid = t >> 6;
-      const int x = wave_incl_sum(c);
-      const int cmax = wave_incl_max(c);
-      if (lane == 63) {
-        s.wsum[wid] = x;
-        s.wbig[wid] = cmax;
-      }
-      if (!__syncthreads_or(c > 0)) continue;
-      int wbase = 0, total = 0, big = 0;
-      for (int w = 0; w < NT / 64; w++) {
-        if (w < wid) wbase += s.wsum[w];
-        total += s.wsum[w];
-        big = max(big, s.wbig[w]);
-      }
-      const int pre = wbase + x - c;
+      publish_pairs(s.pairs, ch & 1, c);
+      __syncthreads();
       auto test_pair = [&](int j, int pix) {
         const float3 p0 = make_float3(s.p[0][j], s.p[1][j], s.p[2][j]);
         const float3 p1 = make_float3(s.p[3][j], s.p[4][j], s.p[5][j]);
@@ -550,51 +536,15 @@ __global__ __launch_bounds__(256) void k_rt_tiles(const DevView* __restrict__ vi
           atomicMin(&s.key[pix], key);
         }
       };
-      if (big <= kScatterMaxPairs) {
-        for (int q0 = 0; q0 < total; q0 += 2 * NT) {
-          const int lo = max(pre, q0), hi = min(pre + c, q0 + 2 * NT);
-          if (lo < hi) {
-            const int bx = s.box[t];
-            const int nx = ((bx >> 8) & 15) + 1;
-            int ry = (lo - pre) / nx;
-            int rx = (lo - pre) - ry * nx;
-            int pix = (((bx >> 4) & 15) + ry) * kRtTile + (bx & 15) + rx;
-            for (int q = lo; q < hi; q++) {
-              s.pairs[q - q0] = t | (pix << 8);
-              if (++rx == nx) {
-                rx = 0;
-                pix += kRtTile - nx + 1;
-              } else {
-                pix++;
-              }
-            }
-          }
-          __syncthreads();
-          const int np = min(total - q0, 2 * NT);
-          for (int pp = t; pp < np; pp += NT) {
-            const int pr = s.pairs[pp];
-            test_pair(pr & 0xff, pr >> 8);
-          }
-          __syncthreads();
-        }
-      } else {
-        s.pairs[t] = pre;
-        if (t == NT - 1) s.pairs[NT] = total;
-        __syncthreads();
-        for (int p = t; p < total; p += NT) {
-          int jl = 0, jh = NT - 1;
-          while (jl < jh) {
-            const int mid = (jl + jh + 1) >> 1;
-            if (s.pairs[mid] <= p) jl = mid; else jh = mid - 1;
-          }
-          const int r = p - s.pairs[jl];
-          const int bx = s.box[jl];
-          const int nx = ((bx >> 8) & 15) + 1;
-          const int qy = r / nx;
-          test_pair(jl, (((bx >> 4) & 15) + qy) * kRtTile + (bx & 15) + (r - qy * nx));
-        }
-        __syncthreads();
-      }
+      auto locate = [&](int j, int r, int& pix) {
+        const int bx = s.box[j];
+        const int nx = ((bx >> 8) & 15) + 1;
+        const int qy = pair_row(r, nx);
+        pix = (((bx >> 4) & 15) + qy) * kRtTile + (bx & 15) + (r - qy * nx);
+        return true;
+      };
+      if (walk_pairs(s.pairs, ch & 1, locate, test_pair) == 0) continue;
+      __syncthreads();
       if (more) {
         const unsigned long long k = s.key[t];
         // depth of the pixel's hit: all ones when it has none, 0 outside the image
