@@ -145,14 +145,15 @@ UGU_DEV void publish_pairs(PairLds<NT>& s, int parity, int c) {
 
 // Runs first(slot, r, pix) for every pair (r: the pair's index in its face,
 // 0 <= r < NT; it sets the tile pixel) and second(slot, pix) for those where first
-// returned true, 64 of them at a time. Returns the number of pairs.
+// returned true, 64 of them at a time (ALL: where it returns true for all of
+// them). Returns the number of pairs.
 // Each wavefront takes 64 consecutive pairs at a time without the others: every
 // lane holds the first pairs of NT / 64 slots, marks those in the wavefront's
 // window at their place in LDS, and a running maximum carries each mark to the
 // pairs of its face. The cost does not depend on the faces' sizes (a list that
 // each face's thread writes costs the largest face's pairs, a binary search per
 // pair eight dependent LDS reads), and no barrier lies between two windows.
-template <int NT, class First, class Second>
+template <int NT, bool ALL = false, class First, class Second>
 UGU_DEV int walk_pairs(PairLds<NT>& s, int parity, First first, Second second) {
   constexpr int K = NT / 64;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -185,6 +186,10 @@ UGU_DEV int walk_pairs(PairLds<NT>& s, int parity, First first, Second second) {
     const int j = m >> 17;
     int pix = 0;
     const bool keep = g + lane < total && first(j, lane + 65536 - (m & 0x1ffff), pix);
+    if (ALL) {
+      if (keep) second(j, pix);
+      continue;
+    }
     const uint64_t kept = __builtin_amdgcn_ballot_w64(keep);
     if (keep)
       queue[queued + static_cast<int>(__builtin_amdgcn_mbcnt_hi(

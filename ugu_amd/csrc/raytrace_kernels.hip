@@ -453,9 +453,10 @@ struct RtLds {
 // rounding of either) is hit later than what each pixel holds.
 // Bound by the latency of a tile's dependent loads (counters, entries, face
 // records, the winner's record and shading inputs), like k_raster. 1.3 M faces
-// at 1080p: setup 26 us + tiles 57 us, where the hierarchy walk (k_raytrace)
-// takes 836 us; 24 mixed views of 492 k faces: 153 + 330 us against 2505 us.
-__global__ __launch_bounds__(256) void k_rt_tiles(const DevView* __restrict__ views, DevMesh m,
+// at 1080p: setup 26 us + tiles 52 us, where the hierarchy walk (k_raytrace)
+// takes 836 us; 24 mixed views of 492 k faces: 153 + 295 us against 2505 us. 6
+// waves per SIMD (78 VGPRs, the rays in LDS only): 5 take 330 us, 7 spill, 333 us.
+__global__ __launch_bounds__(256, 6) void k_rt_tiles(const DevView* __restrict__ views, DevMesh m,
                                                   DevBins bins, DevOptions o) {
   constexpr int NT = 256;
   __shared__ RtLds s;
@@ -484,16 +485,19 @@ __global__ __launch_bounds__(256) void k_rt_tiles(const DevView* __restrict__ vi
     const int chunks_a = (nA + NT - 1) / NT, chunks = chunks_a + (nB + NT - 1) / NT;
     int2 e_next = make_int2(0, 0);
     if (t < (chunks_a > 0 ? nA : n)) e_next = bin_entry(bin, nA, bins.cap, t);
-    ray_w_at(v, static_cast<float>(gx), static_cast<float>(gy), r0, r1, r2);
+    {
+      float w0, w1, w2;
+      ray_w_at(v, static_cast<float>(gx), static_cast<float>(gy), w0, w1, w2);
+      s.ray[0][t] = w0;
+      s.ray[1][t] = w1;
+      s.ray[2][t] = w2;
+    }
     // z of the pixel's normalized camera-space ray: q.z of a hit at distance 1
     const float u0 = (static_cast<float>(gx) - v.cx) / v.fx;
     const float u1 = (static_cast<float>(gy) - v.cy) / v.fy;
     const float zray = __builtin_amdgcn_rsqf(u0 * u0 + u1 * u1 + 1.0f);
     const double ox = v.c2w_t[0], oy = v.c2w_t[1], oz = v.c2w_t[2];
     s.key[t] = ~0ull;
-    s.ray[0][t] = r0;
-    s.ray[1][t] = r1;
-    s.ray[2][t] = r2;
     float dmax = __uint_as_float(0xffffffffu);  // NaN: some pixel has no hit yet
     for (int ch = 0; ch < chunks; ch++) {
       if (ch == chunks_a && skip_face(__uint_as_float(static_cast<uint32_t>(seg.z)), dmax)) break;
@@ -543,7 +547,7 @@ __global__ __launch_bounds__(256) void k_rt_tiles(const DevView* __restrict__ vi
         pix = (((bx >> 4) & 15) + qy) * kRtTile + (bx & 15) + (r - qy * nx);
         return true;
       };
-      if (walk_pairs(s.pairs, ch & 1, locate, test_pair) == 0) continue;
+      if (walk_pairs<NT, true>(s.pairs, ch & 1, locate, test_pair) == 0) continue;
       __syncthreads();
       if (more) {
         const unsigned long long k = s.key[t];
@@ -563,6 +567,9 @@ __global__ __launch_bounds__(256) void k_rt_tiles(const DevView* __restrict__ vi
     }
     const unsigned long long k = s.key[t];
     if (k != ~0ull) bf = static_cast<int>(static_cast<unsigned int>(k & 0xffffffffull));
+    r0 = s.ray[0][t];
+    r1 = s.ray[1][t];
+    r2 = s.ray[2][t];
   }
   if (!act) return;
   float bt = 0.0f, bu = 0.0f, bv = 0.0f;
