@@ -1451,7 +1451,6 @@ int ugu_hip_texture_map(ugu_hip_ctx* c, const UguTexture* images, int n_images,
     in.push_back(HostCopy{const_cast<UguTexFace*>(faces), c->tm_faces.p,
                           size_t(n_faces) * sizeof(UguTexFace)});
   UGU_HIP_CHECK(c, c->ring.to_device(c->stream, in.data(), static_cast<int>(in.size())));
-  UGU_HIP_CHECK(c, hipMemsetAsync(ob + o_tex0, 0, texels * 4, c->stream));  // texture0 + mask0
   if (launch_texture_map(c->stream, c->tm_faces.p, n_faces, ib, tex_w, tex_h, padding_kernel / 2,
                          reinterpret_cast<int32_t*>(ob), ob + o_tex0, ob + o_mask0, ob + o_tex,
                          ob + o_mask))
