@@ -24,19 +24,6 @@ struct HostCopy {
 
 struct HostJob;
 
-// Populates the pages of host arrays that are about to be written, on the pool's
-// threads, while the device still works on what goes there. Changes no byte.
-class Prefault {
- public:
-  Prefault(const HostCopy* c, int n);
-  ~Prefault();
-  Prefault(const Prefault&) = delete;
-  Prefault& operator=(const Prefault&) = delete;
-
- private:
-  HostJob* job_ = nullptr;
-};
-
 // The slots of one context; allocated by the first copy that uses them.
 class CopyRing {
  public:
@@ -52,12 +39,29 @@ class CopyRing {
   void release();
 
  private:
+  friend class Prefault;
   hipError_t prepare();
   hipError_t wait_groups();
   unsigned char* pinned_ = nullptr;
   hipEvent_t ev_[kGroups] = {};
   bool used_[kGroups] = {};  // the group's event has been recorded
   uint32_t seq_ = 0;         // sequence number of the last chunk
+};
+
+// Populates the pages of host arrays that are about to be written, on the pool's
+// threads, while the device still works on what goes there. Changes no byte. To be
+// made after the call's allocations: both need the process's memory map (a first
+// 1080p pass took 1 ms longer with its buffers allocated beside it), so the ring's
+// slots are allocated first.
+class Prefault {
+ public:
+  Prefault(CopyRing& ring, const HostCopy* c, int n);
+  ~Prefault();
+  Prefault(const Prefault&) = delete;
+  Prefault& operator=(const Prefault&) = delete;
+
+ private:
+  HostJob* job_ = nullptr;
 };
 
 }  // namespace ugu_hip

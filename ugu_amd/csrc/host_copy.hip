@@ -259,8 +259,9 @@ void split(const HostCopy* c, int n, std::vector<HostJob::Chunk>* out) {
 
 }  // namespace
 
-Prefault::Prefault(const HostCopy* c, int n) {
+Prefault::Prefault(CopyRing& ring, const HostCopy* c, int n) {
   if (total(c, n) < kPoolBytes) return;
+  if (ring.prepare() != hipSuccess) (void)hipGetLastError();
   auto job = std::make_unique<HostJob>();
   for (int i = 0; i < n; i++) {
     uintptr_t at = reinterpret_cast<uintptr_t>(c[i].host);

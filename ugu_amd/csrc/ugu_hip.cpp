@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstring>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <vector>
 
@@ -542,7 +543,7 @@ int run_pipeline(ugu_hip_ctx* c, const UguCamera* cams, int n, const DevMesh& dm
   if ((err = ensure(c, c->views, size_t(n) * sizeof(DevView)))) return err;
   if (stage_bytes > 0 && (err = ensure(c, c->stage_out, size_t(stage_bytes)))) return err;
   const std::vector<HostCopy> copies = staged_copies(c, cams, n, outs, gbufs, stage_off);
-  const Prefault prefault(copies.data(), static_cast<int>(copies.size()));
+  std::optional<Prefault> prefault;
   const size_t view_bytes = size_t(n) * sizeof(DevView);
   if (c->h_views_bytes < view_bytes) {
     if (c->h_views) (void)hipHostFree(c->h_views);
@@ -583,6 +584,7 @@ int run_pipeline(ugu_hip_ctx* c, const UguCamera* cams, int n, const DevMesh& dm
   c->tm = UguTimings{};
   for (int attempt = 0; attempt < 8; attempt++) {
     if ((err = ensure(c, c->bins, size_t(total_tiles) * size_t(c->tiling.bin_capacity) * 8))) return err;
+    if (!prefault) prefault.emplace(c->ring, copies.data(), static_cast<int>(copies.size()));
     DevBins b;
     b.counts = c->counts.as<int32_t>();
     b.bins = c->bins.as<int2>();
@@ -952,7 +954,9 @@ int raytrace_common(ugu_hip_ctx* c, const UguCamera* cams, int n, const UguOptio
   if ((err = ensure(c, c->views, size_t(n) * sizeof(DevView)))) return err;
   if (stage_bytes > 0 && (err = ensure(c, c->stage_out, size_t(stage_bytes)))) return err;
   const std::vector<HostCopy> copies = staged_copies(c, cams, n, outs, nullptr, stage_off);
-  const Prefault prefault(copies.data(), static_cast<int>(copies.size()));
+  // not beside the allocations of a first pass
+  std::optional<Prefault> prefault;
+  if (!c->rt_bins || c->bins.p) prefault.emplace(c->ring, copies.data(), static_cast<int>(copies.size()));
   const size_t view_bytes = size_t(n) * sizeof(DevView);
   if (c->h_views_bytes < view_bytes) {
     if (c->h_views) (void)hipHostFree(c->h_views);
@@ -1356,7 +1360,7 @@ int ugu_hip_visibility_test(ugu_hip_ctx* c, const UguKeyframe* kf, const UguVisi
   const size_t depth_off = (px * 3 + 255) / 256 * 256,
                mask_off = (depth_off + px * 4 + 15) / 16 * 16;
   const HostCopy result{out, c->vis_out.p, size_t(n) * sizeof(UguVertexVisibility)};
-  const Prefault prefault(&result, 1);
+  const Prefault prefault(c->ring, &result, 1);
   auto in = [](const void* host, uint8_t* dev, size_t bytes) {
     return HostCopy{const_cast<void*>(host), dev, bytes};
   };
@@ -1437,7 +1441,7 @@ int ugu_hip_texture_map(ugu_hip_ctx* c, const UguTexture* images, int n_images,
   if ((err = ensure(c, c->tm_out, o_mask + texels))) return err;
   uint8_t* ob = c->tm_out.as<uint8_t>();
   const HostCopy result[2] = {{texture, ob + o_tex, texels * 3}, {mask, ob + o_mask, texels}};
-  const Prefault prefault(result, 2);
+  const Prefault prefault(c->ring, result, 2);
   uint8_t* ib = c->tm_images.as<uint8_t>();
   std::vector<Img> desc(static_cast<size_t>(n_images));
   std::vector<HostCopy> in;
