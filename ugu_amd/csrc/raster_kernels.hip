@@ -137,7 +137,7 @@ UGU_DEV bool cover_test(float ax, float ay, float az, float bx, float by,
 
 
 // ---------------------------------------------------------------------------
-// k_clear
+// k_begin
 
 // Starts a pass: clears the tiles' counters and the status words and, with
 // N > 0, writes the view descriptors it got as arguments to device memory (one
