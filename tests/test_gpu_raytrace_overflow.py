@@ -1,0 +1,64 @@
+"""Passes of the raytracer in which a tile's bin overflows only when its front and
+back faces are taken together: each segment fits the bin's first 1024 entries, so
+the setup kernel sees no overflow and the tile kernel finds it, in some tiles,
+while the others work. Against oracle_raytrace, every output exactly but depth and
+normal (within 1e-5 relative, as the raytracer's other parity tests)."""
+import numpy as np
+import pytest
+
+import oracle as O
+from ugu_amd import DiffuseColor, Mesh, PinholeCamera, Raytracer, RendererCpuOption
+
+pytestmark = pytest.mark.gpu
+
+TILE = 16
+
+
+def _clusters(w, h, full, per_side, others, seed):
+    """Triangles three pixels wide, whole inside one tile each: `per_side` clockwise
+    and as many counter-clockwise ones on screen in every tile of `full`, `others`
+    of each in every other tile."""
+    rng = np.random.default_rng(seed)
+    tx, ty = -(-w // TILE), -(-h // TILE)
+    f = 0.9 * h
+    c = np.array([w * 0.5 - 0.5, h * 0.5 - 0.5])
+    shape = np.array([[-1.5, -1.2], [1.5, -1.0], [0.2, 1.6]])
+    pts = []
+    for t in range(tx * ty):
+        n = per_side if t in full else others
+        lo = np.array([t % tx, t // tx]) * TILE + 2.0
+        for flip in (False, True):
+            at = lo + rng.uniform(0.0, TILE - 5.0, (n, 1, 2))
+            xy = at + (shape[::-1] if flip else shape)
+            z = rng.uniform(2.0, 5.0, (n, 1, 1)).repeat(3, 1)
+            pts.append(np.concatenate([(xy - c) / f * z, z], -1))
+    p = np.concatenate(pts)
+    p = p[rng.permutation(len(p))]
+    m = Mesh(p.reshape(-1, 3).astype(np.float32), np.arange(p.shape[0] * 3, dtype=np.int32))
+    m.CalcFaceNormal()
+    m.set_normals(np.repeat(m.face_normals, 3, axis=0))
+    m.set_normal_indices(m.vertex_indices)
+    m.set_vertex_colors(rng.random((len(m.vertices), 3), np.float32) * 255)
+    return m, PinholeCamera(w, h, np.eye(4), tuple(c), (f, f))
+
+
+def _check(out, ref, label):
+    for k in ("face_id", "mask", "color"):
+        assert np.array_equal(out[k], ref[k]), (label, k)
+    for k in ("depth", "normal"):
+        np.testing.assert_allclose(out[k], ref[k], rtol=1e-5, atol=1e-7)
+
+
+@pytest.mark.parametrize("full", [(0,), (3, 17, 29, 59), tuple(range(0, 60, 6))])
+@pytest.mark.parametrize("views", [1, 3])
+def test_segments_overflow_together(gpu_available, full, views):
+    mesh, cam = _clusters(160, 96, full, 700, 20, len(full))
+    opt = RendererCpuOption(diffuse_color=DiffuseColor.kVertex)
+    rc, ref, _ = O.raytrace(mesh, O.camera_from_abi(cam.to_abi()), opt, c2w_t=cam.c2w[:3, 3])
+    assert rc == 0 and (ref["face_id"] >= 0).sum() > 1000
+    r = Raytracer(opt)
+    r.set_mesh(mesh)
+    assert r.PrepareMesh()
+    for call in range(2):
+        for out in r.render_batch([cam] * views):
+            _check(out, ref, call)

@@ -122,8 +122,8 @@ struct DevBins {
                      // entry = (face id, bits of its skip depth)
   int32_t cap;
   int32_t total_tiles;
-  int32_t* status;   // [0] max bin count seen; [kQueueStride (q + 1)] head of
-                     // work queue q (kStatusBytes in all)
+  int32_t* status;   // max bin count seen: [0], and [1] by k_rt_tiles; [kQueueStride
+                     // (q + 1)] head of work queue q (kStatusBytes in all)
   int32_t* host_flag;  // pinned host word, set when a bin overflows: the host
                        // reads the status only then
 };

@@ -463,11 +463,15 @@ __global__ __launch_bounds__(256, 6) void k_rt_tiles(const DevView* __restrict__
   const int t = threadIdx.x;
   const int gtile = xcd_remap(blockIdx.x, gridDim.x);
   const int4 seg = reinterpret_cast<const int4*>(bins.counts)[gtile];
-  // some bin overflowed (this one: published, the two segments share it): the
-  // host renders again, nothing here is worth finishing
+  // Some bin overflowed: the host renders again, nothing here is worth finishing.
+  // Both conditions are the same in every thread of the block: status[0] is the
+  // setup kernel's and no block writes it here (a word that blocks of this launch
+  // raise would let a block's wavefronts differ, and those that stay read LDS that
+  // the leavers never wrote). A tile that its two segments overflow together is
+  // first seen here, and published in status[1].
   if (seg.x + seg.y > bins.cap || bins.status[0] > bins.cap) {
     if (t == 0 && seg.x + seg.y > bins.cap) {
-      atomicMax(&bins.status[0], seg.x + seg.y);
+      atomicMax(&bins.status[1], seg.x + seg.y);
       *bins.host_flag = 1;
     }
     return;

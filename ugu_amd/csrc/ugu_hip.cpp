@@ -226,9 +226,9 @@ int order_after_user(ugu_hip_ctx* c) {
 int read_overflow(ugu_hip_ctx* c, const int32_t* status, int32_t* most) {
   *most = 0;
   if (*static_cast<volatile int32_t*>(c->h_status) == 0) return 0;
-  UGU_HIP_CHECK(c, hipMemcpyAsync(c->h_status, status, 4, hipMemcpyDeviceToHost, c->stream));
+  UGU_HIP_CHECK(c, hipMemcpyAsync(c->h_status, status, 8, hipMemcpyDeviceToHost, c->stream));
   UGU_HIP_CHECK(c, hipStreamSynchronize(c->stream));
-  *most = c->h_status[0];
+  *most = std::max(c->h_status[0], c->h_status[1]);
   return 0;
 }
 
