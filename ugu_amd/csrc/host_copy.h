@@ -1,4 +1,4 @@
-// Copies between the device and pageable host arrays through pinned slots: a
+// Copies between the device and host arrays, through pinned slots if pageable: a
 // copy kernel moves chunks between the device and the slots while host threads
 // move them between the slots and the caller's arrays.
 //
@@ -33,7 +33,8 @@ class CopyRing {
   static constexpr int kSlots = kGroups * kGroupChunks;
 
   // Queues the copies after the stream's work. to_host returns when the host
-  // arrays hold the data, to_device when the host arrays have been read.
+  // arrays hold the data, to_device when the pageable host arrays have been read
+  // (pinned ones are read in the stream's order).
   hipError_t to_host(hipStream_t st, const HostCopy* c, int n);
   hipError_t to_device(hipStream_t st, const HostCopy* c, int n);
   void release();
