@@ -10,6 +10,7 @@
 #include <memory>
 #include <mutex>
 #include <thread>
+#include <utility>
 #include <vector>
 
 #ifndef MADV_POPULATE_WRITE
@@ -267,9 +268,24 @@ hipError_t queue(hipStream_t st, const HostCopy& c, bool out) {
              : hipMemcpyAsync(c.dev, c.host, c.bytes, hipMemcpyHostToDevice, st);
 }
 
+// Whether two of the host arrays share bytes. Copies out are then made in their
+// order, so that the last one's bytes stay, as in a loop of copies.
+bool overlap(const HostCopy* c, int n) {
+  std::vector<std::pair<uintptr_t, uintptr_t>> r;
+  for (int i = 0; i < n; i++) {
+    const uintptr_t at = reinterpret_cast<uintptr_t>(c[i].host);
+    if (c[i].bytes > 0) r.emplace_back(at, at + c[i].bytes);
+  }
+  std::sort(r.begin(), r.end());
+  for (size_t i = 1; i < r.size(); i++)
+    if (r[i].first < r[i - 1].second) return true;
+  return false;
+}
+
 // Queues the copies that the engine makes: of pinned arrays (from kMinDirect bytes
 // of them in all on), of memory that is not the host's, and, where fewer than
-// `least` bytes would be left, all of them. The others are returned in *slots.
+// `least` bytes would be left or results overlap, all of them. The others are
+// returned in *slots.
 hipError_t queue_direct(hipStream_t st, const HostCopy* c, int n, bool out, size_t least,
                         std::vector<HostCopy>* slots) {
   std::vector<Memory> kind(static_cast<size_t>(n), Memory::kOther);
@@ -281,10 +297,11 @@ hipError_t queue_direct(hipStream_t st, const HostCopy* c, int n, bool out, size
     if (kind[size_t(i)] == Memory::kPageable) left += c[i].bytes;
   }
   if (pinned < kMinDirect) left += pinned;
+  const bool use = left >= least && !(out && overlap(c, n));
   for (int i = 0; i < n; i++) {
     if (c[i].bytes == 0) continue;
-    if (left >= least && (kind[size_t(i)] == Memory::kPageable ||
-                          (kind[size_t(i)] == Memory::kPinned && pinned < kMinDirect))) {
+    if (use && (kind[size_t(i)] == Memory::kPageable ||
+                (kind[size_t(i)] == Memory::kPinned && pinned < kMinDirect))) {
       slots->push_back(c[i]);
     } else if (hipError_t e = queue(st, c[i], out)) {
       return e;
