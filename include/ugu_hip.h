@@ -177,6 +177,9 @@ typedef struct {
   float setup_bin_ms;
   float raster_ms;
   float total_ms;
+  /* largest occupancy of a bin that overflowed (0: none did) and the passes
+   * that were repeated for it; also of ugu_hip_raytrace, whose repeated pass may
+   * be the hierarchy's */
   int32_t max_bin_count;
   int32_t retries;
   /* last ugu_hip_diff_backward: the per-face item sort (count, scan,

@@ -62,3 +62,38 @@ def test_segments_overflow_together(gpu_available, full, views):
     for call in range(2):
         for out in r.render_batch([cam] * views):
             _check(out, ref, call)
+
+
+def _retries(r, cam, calls):
+    """Repeated passes of each of `calls` calls, whose outputs are all equal."""
+    out, first = [], None
+    for _ in range(calls):
+        got = r.render_batch([cam], outputs=("face_id", "depth"))[0]
+        out.append(r.timings()["retries"])
+        first = first or got
+        for k in got:
+            assert np.array_equal(got[k], first[k])
+    return out
+
+
+def test_dense_tile_is_not_tried_on_every_call(gpu_available):
+    """2500 front and 2500 back faces on a tile exceed what a bin may hold (4096): the
+    hierarchy traces the view, and the bins are tried again ever more rarely. After
+    PrepareMesh, and for a view of other tiles, they are tried at once."""
+    mesh, cam = _clusters(160, 96, (17,), 2500, 20, 3)
+    corner = PinholeCamera(64, 48, np.eye(4), tuple(cam.principal_point), tuple(cam.focal_length))
+    r = Raytracer(RendererCpuOption(diffuse_color=DiffuseColor.kVertex))
+    r.set_mesh(mesh)
+    for _ in range(2):
+        assert r.PrepareMesh()
+        tried = [k for k, n in enumerate(_retries(r, cam, 300)) if n > 0]
+        assert tried == [0, 2, 6, 14, 30, 62, 126, 254]
+    assert _retries(r, corner, 2) == [0, 0]  # its tiles hold few faces
+
+
+def test_bins_that_grew_are_kept(gpu_available):
+    mesh, cam = _clusters(160, 96, (17,), 1500, 20, 4)
+    r = Raytracer(RendererCpuOption(diffuse_color=DiffuseColor.kVertex))
+    r.set_mesh(mesh)
+    assert r.PrepareMesh()
+    assert _retries(r, cam, 4) == [1, 0, 0, 0]

@@ -127,6 +127,14 @@ struct DevBuf {
   T* as() const { return static_cast<T*>(p); }
 };
 
+// Views (their count and tiles) whose bins did not fit in a pass of the raytracer:
+// how often in a row, and how many further passes go straight to the hierarchy.
+struct RtRefusal {
+  int n;
+  int64_t tiles;
+  int count, skip;
+};
+
 }  // namespace
 
 struct ugu_hip_ctx {
@@ -165,6 +173,7 @@ struct ugu_hip_ctx {
   float rt_max_coord = 0.0f, rt_max_edge = 0.0f;  // 1-norms, for the binned path's bounds
   bool rt_bins = false;      // few enough layers of faces for the binned path
   int32_t rt_cap = 1024;     // entries per tile of the raytracer's bins
+  std::vector<RtRefusal> rt_refusals;
   int clean_tiles = 0;  // leading tile counters known to be clear, of view 0
   CopyRing ring;                 // pinned slots of the copies to and from host arrays
   void* h_views = nullptr;
@@ -849,6 +858,30 @@ double rt_layers(const float* rec, int64_t F) {
 }
 
 constexpr int32_t kRtMaxCap = 4096;
+
+// A pass whose bins do not fit has cost its setup, a part of its tiles and a wait
+// before the hierarchy traces it. So views that were refused are not tried again at
+// once: after the k-th refusal in a row 2^k - 1 passes of as many tiles skip the
+// bins, at most 127 (the camera may move away from what did not fit). 6000 faces on
+// one tile of 160 x 96 pixels: 338 us tried on every call, 298 so, 297 by the
+// hierarchy alone.
+RtRefusal* rt_refusal(ugu_hip_ctx* c, int n, int64_t tiles) {
+  for (RtRefusal& r : c->rt_refusals)
+    if (r.n == n && r.tiles == tiles) return &r;
+  return nullptr;
+}
+
+void rt_refused(ugu_hip_ctx* c, int n, int64_t tiles) {
+  RtRefusal* r = rt_refusal(c, n, tiles);
+  if (!r) {
+    if (c->rt_refusals.size() >= 16) c->rt_refusals.erase(c->rt_refusals.begin());
+    c->rt_refusals.push_back(RtRefusal{n, tiles, 0, 0});
+    r = &c->rt_refusals.back();
+  }
+  r->count = std::min(r->count + 1, 7);
+  r->skip = (1 << r->count) - 1;
+}
+
 int raytrace_binned(ugu_hip_ctx* c, DevView* hv, int n, const DevMesh& dm, const DevOptions& dopt) {
   if (!c->rt_bins) return 0;
   int64_t total = 0;
@@ -859,6 +892,10 @@ int raytrace_binned(ugu_hip_ctx* c, DevView* hv, int n, const DevMesh& dm, const
     hv[i].tile_base = static_cast<int32_t>(total);
     total += int64_t(hv[i].tiles_x) * hv[i].tiles_y;
     if (total > INT32_MAX / 2) return 0;
+  }
+  if (RtRefusal* r = rt_refusal(c, n, total); r && r->skip > 0) {
+    r->skip--;
+    return 0;
   }
   int err;
   if ((err = ensure(c, c->status, kStatusBytes))) return err;
@@ -875,6 +912,7 @@ int raytrace_binned(ugu_hip_ctx* c, DevView* hv, int n, const DevMesh& dm, const
     if (total * c->rt_cap * 8 > (int64_t(32) << 30)) return 0;
     if (ensure(c, c->bins, size_t(total) * size_t(c->rt_cap) * 8)) {
       (void)hipGetLastError();
+      rt_refused(c, n, total);
       return 0;
     }
     DevBins b;
@@ -899,8 +937,17 @@ int raytrace_binned(ugu_hip_ctx* c, DevView* hv, int n, const DevMesh& dm, const
     if ((err = read_overflow(c, b.status, &most))) return err;
     // tiles that saw an overflow left their counters as they were
     if (n == 1 && most == 0) c->clean_tiles = std::max(clean, b.total_tiles);
-    if (most <= c->rt_cap) return 1;
-    if (most > kRtMaxCap) return 0;
+    c->tm.max_bin_count = std::max(c->tm.max_bin_count, most);
+    if (most <= c->rt_cap) {
+      if (RtRefusal* r = rt_refusal(c, n, total))
+        c->rt_refusals.erase(c->rt_refusals.begin() + (r - c->rt_refusals.data()));
+      return 1;
+    }
+    c->tm.retries++;
+    if (most > kRtMaxCap) {
+      rt_refused(c, n, total);
+      return 0;
+    }
     c->rt_cap = static_cast<int32_t>(std::min<int64_t>(kRtMaxCap, (int64_t(most) + most / 8 + 63) / 64 * 64));
   }
 }
@@ -1317,6 +1364,7 @@ int ugu_hip_prepare_raytracer(ugu_hip_ctx* c) {
     }
   }
   c->rt_bins = rt_layers(rec.data(), c->F) <= kRtMaxLayers;
+  c->rt_refusals.clear();
   c->rt_mesh_gen = c->mesh_gen;
   c->rt_ready = true;
   return UGU_HIP_OK;
