@@ -97,3 +97,29 @@ def test_bins_that_grew_are_kept(gpu_available):
     r.set_mesh(mesh)
     assert r.PrepareMesh()
     assert _retries(r, cam, 4) == [1, 0, 0, 0]
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
+def test_faces_that_are_not_finite_fill_no_bins(gpu_available, value):
+    """5000 faces with such a coordinate can be hit nowhere. Put into every tile's bin
+    they would exceed it and send each call to the hierarchy."""
+    mesh, cam = _clusters(160, 96, (17,), 100, 20, 5)
+    rng = np.random.default_rng(6)
+    more = rng.uniform(-1, 1, (15000, 3)).astype(np.float32)
+    more[np.arange(0, 15000, 3) + rng.integers(0, 3, 5000), rng.integers(0, 3, 5000)] = value
+    v = np.concatenate([more, mesh.vertices])
+    m = Mesh(v, np.arange(len(v), dtype=np.int32))
+    m.set_face_normals(np.concatenate([np.tile(np.float32([0, 0, 1]), (5000, 1)),
+                                       mesh.face_normals]))
+    m.set_normals(np.tile(np.float32([0, 0, -1]), (len(v), 1)))
+    m.set_normal_indices(m.vertex_indices)
+    m.set_vertex_colors(rng.random((len(v), 3), np.float32) * 255)
+    opt = RendererCpuOption(diffuse_color=DiffuseColor.kVertex)
+    rc, ref, _ = O.raytrace(m, O.camera_from_abi(cam.to_abi()), opt, c2w_t=cam.c2w[:3, 3])
+    assert rc == 0 and (ref["face_id"] >= 5000).sum() > 1000
+    r = Raytracer(opt)
+    r.set_mesh(m)
+    assert r.PrepareMesh()
+    for call in range(2):
+        _check(r.render_batch([cam])[0], ref, value)
+        assert r.timings()["retries"] == 0

@@ -226,9 +226,13 @@ UGU_DEV float4 project_ray(const DevView& v, float px, float py, float pz) {
 
 // True when every point of the face lies outside one side of the image's
 // frustum (a pixel wider than the image on each side, minus the error of q),
-// or behind the camera: no ray of the view can hit it. For faces with a corner
+// or behind the camera: no ray of the view can hit it. Nor can one hit a face with
+// a corner that is not finite: its hit distances are NaN. For faces with a corner
 // that project_ray gives no bound for.
 UGU_DEV bool outside_frustum(const DevView& v, const float* P) {
+  float sum = 0.0f;  // 0 x inf and NaN propagate
+  for (int k = 0; k < 9; k++) sum += 0.0f * P[k];
+  if (sum != sum) return true;
   int out = 31;
   for (int k = 0; k < 3; k++) {
     const float dx = P[3 * k] - v.c2w_t[0], dy = P[3 * k + 1] - v.c2w_t[1],
@@ -247,7 +251,7 @@ UGU_DEV bool outside_frustum(const DevView& v, const float* P) {
     if (gy + (v.cy + 1.0f) * qz < -ey) o |= 4;
     if (gy + (v.cy - static_cast<float>(v.H)) * qz > ey) o |= 8;
     if (qz < -s) o |= 16;
-    out &= o;  // a NaN coordinate sets no bit
+    out &= o;
   }
   return out != 0;
 }
