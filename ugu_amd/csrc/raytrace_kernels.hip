@@ -275,12 +275,15 @@ UGU_DEV int2 rt_entry(int f, float zskip, int x0, int x1, int y0, int y1, int tx
 template <bool INL>
 __global__ __launch_bounds__(256) void k_rt_setup(InlineViews<1> arg,
                                                   const DevView* __restrict__ views, DevView* out,
-                                                  int n_views, DevMesh mesh, DevBins bins) {
+                                                  int n_views, DevMesh mesh, DevBins bins,
+                                                  RtLarge large) {
   if (INL && blockIdx.x == 0) {
     // an occupancy published before this store is published again by its tile
     clear_status(bins.status);
     store_inline_views(out, 1);
   }
+  if (blockIdx.x == 0 && blockIdx.y == 0)
+    for (int k = threadIdx.x; k < n_views; k += blockDim.x) large.clear[k] = 0;
   __shared__ float4 sp[768];
   const int f = blockIdx.x * blockDim.x + threadIdx.x;
   const int vbase = mesh.blk_off[blockIdx.x];
@@ -376,6 +379,22 @@ __global__ __launch_bounds__(256) void k_rt_setup(InlineViews<1> arg,
         y1 = v.H - 1;
       }
     }
+    // A large face would be appended to its bins by this wavefront alone, 64 tiles at
+    // a time: a ball in a room of 12 faces at 1080p 2330 us, listed 121 (hierarchy
+    // 319); 82 k faces seen from close by at 640x480 107 and 78 (81).
+    const int tiles = (x1 / kRtTile - x0 / kRtTile + 1) * (y1 / kRtTile - y0 / kRtTile + 1);
+    const uint64_t big = __builtin_amdgcn_ballot_w64(has && tiles > kRtLargeTiles);
+    if (big) {
+      const int lane = __lane_id(), lead = __ffsll(static_cast<unsigned long long>(big)) - 1;
+      int slot = 0;
+      if (lane == lead) slot = atomicAdd(&large.count[vi], __popcll(big));
+      slot = __shfl(slot, lead) + __popcll(big & ((1ull << lane) - 1ull));
+      if (((big >> lane) & 1ull) && slot < kRtLargeFaces) {
+        large.list[int64_t(vi) * kRtLargeFaces + slot] =
+            make_int4(f, __float_as_int(zskip), x0 | (x1 << 16), y0 | (y1 << 16));
+        has = false;
+      }
+    }
     const int tx0 = x0 / kRtTile, tx1 = has ? x1 / kRtTile : -1;
     const int ty0 = y0 / kRtTile, ty1 = has ? y1 / kRtTile : -1;
     const uint32_t zmin = back_zmin(has && back, __uint_as_float(__float_as_uint(zskip) & 0xffff0000u));
@@ -428,10 +447,17 @@ __global__ __launch_bounds__(256) void k_rt_setup(InlineViews<1> arg,
         const int stx = sx0 / kRtTile + k % snx;
         const int sback = __shfl(back ? 1 : 0, src);
         const int2 e = rt_entry(__shfl(f, src), __shfl(zskip, src), sx0, sx1, sy0, sy1, stx, sty);
-        const bool act = p < total;
-        const AppendTicket t1 = append_issue(
-            bins, act ? 4 * (v.tile_base + sty * v.tiles_x + stx) + sback : -1, zmin, act);
-        append_finish<1, true>(bins, &t1, &e);
+        // mostly different tiles, so every lane appends its own (grouped by tile as in
+        // append_issue: 10 k faces of 100 tiles at 1080p 857 us, so 429)
+        if (p < total) {
+          const int tile = v.tile_base + sty * v.tiles_x + stx;
+          const int slot = atomicAdd(&bins.counts[4 * tile + sback], 1);
+          if (sback) atomicMin(reinterpret_cast<unsigned int*>(bins.counts) + (4 * tile + 2), zmin);
+          if (slot < bins.cap)
+            bins.bins[int64_t(tile) * bins.cap + (sback ? bins.cap - 1 - slot : slot)] = e;
+          else
+            atomicMax(&bins.status[0], slot + 1);
+        }
       }
     }
   }
@@ -461,7 +487,7 @@ struct RtLds {
 // takes 836 us; 24 mixed views of 492 k faces: 153 + 295 us against 2505 us. 6
 // waves per SIMD (78 VGPRs, the rays in LDS only): 5 take 330 us, 7 spill, 333 us.
 __global__ __launch_bounds__(256, 6) void k_rt_tiles(const DevView* __restrict__ views, DevMesh m,
-                                                  DevBins bins, DevOptions o) {
+                                                  DevBins bins, RtLarge large, DevOptions o) {
   constexpr int NT = 256;
   __shared__ RtLds s;
   const int t = threadIdx.x;
@@ -486,10 +512,15 @@ __global__ __launch_bounds__(256, 6) void k_rt_tiles(const DevView* __restrict__
   const int gx = txi * kRtTile + t % kRtTile, gy = tyi * kRtTile + t / kRtTile;
   const bool act = gx < v.W && gy < v.H;
   const int nA = seg.x, nB = seg.y, n = nA + nB;
+  const int n_large = min(large.count[seg.w], kRtLargeFaces);
   int bf = -1;
   float r0 = 0.0f, r1 = 0.0f, r2 = 0.0f;
-  if (n > 0) {
+  if (n + n_large > 0) {
     const int2* bin = bins.bins + int64_t(gtile) * bins.cap;
+    const int4* list = large.list + int64_t(seg.w) * kRtLargeFaces;
+    // chunks of 256 faces: of the view's large faces (ch < 0), of the bin's front
+    // and of its back segment
+    const int chunks_l = (n_large + NT - 1) / NT;
     const int chunks_a = (nA + NT - 1) / NT, chunks = chunks_a + (nB + NT - 1) / NT;
     int2 e_next = make_int2(0, 0);
     if (t < (chunks_a > 0 ? nA : n)) e_next = bin_entry(bin, nA, bins.cap, t);
@@ -507,13 +538,26 @@ __global__ __launch_bounds__(256, 6) void k_rt_tiles(const DevView* __restrict__
     const double ox = v.c2w_t[0], oy = v.c2w_t[1], oz = v.c2w_t[2];
     s.key[t] = ~0ull;
     float dmax = __uint_as_float(0xffffffffu);  // NaN: some pixel has no hit yet
-    for (int ch = 0; ch < chunks; ch++) {
+    for (int ch = -chunks_l; ch < chunks; ch++) {
       if (ch == chunks_a && skip_face(__uint_as_float(static_cast<uint32_t>(seg.z)), dmax)) break;
-      const int base = ch < chunks_a ? ch * NT : nA + (ch - chunks_a) * NT;
-      const int end = ch < chunks_a ? nA : n;
+      int base = ch < chunks_a ? ch * NT : nA + (ch - chunks_a) * NT;
+      int end = ch < chunks_a ? nA : n;
       const bool more = ch + 1 < chunks;
-      const int2 e = e_next;
-      if (more) {
+      int2 e = e_next;
+      if (ch < 0) {
+        base = (ch + chunks_l) * NT;
+        end = 0;  // unless the face's box meets the tile
+        if (base + t < n_large) {
+          const int4 q = list[base + t];
+          const int x0 = q.z & 0xffff, x1 = static_cast<uint32_t>(q.z) >> 16;
+          const int y0 = q.w & 0xffff, y1 = static_cast<uint32_t>(q.w) >> 16;
+          if (x0 < (txi + 1) * kRtTile && x1 >= txi * kRtTile && y0 < (tyi + 1) * kRtTile &&
+              y1 >= tyi * kRtTile) {
+            e = rt_entry(q.x, __int_as_float(q.y), x0, x1, y0, y1, txi, tyi);
+            end = n_large;
+          }
+        }
+      } else if (more) {
         const int nbase = ch + 1 < chunks_a ? (ch + 1) * NT : nA + (ch + 1 - chunks_a) * NT;
         const int nend = ch + 1 < chunks_a ? nA : n;
         e_next = nbase + t < nend ? bin_entry(bin, nA, bins.cap, nbase + t) : make_int2(0, 0);
@@ -763,17 +807,21 @@ int launch_visibility(hipStream_t st, const DevView& v, const uint8_t* color, co
 // views[i].tile_base = first 16x16 tile of view i; the bins' counters cleared.
 // one: as launch_setup_bin's
 int launch_raytrace_binned(hipStream_t st, const DevView* one, DevView* views, int n_views,
-                           const DevMesh& m, const DevBins& bins, const DevOptions& o) {
+                           const DevMesh& m, const DevBins& bins, const RtLarge& large,
+                           const DevOptions& o) {
   if (n_views < 1 || bins.total_tiles < 1 || m.F < 1) return 0;
   const dim3 grid((m.F + 255) / 256, (n_views + kSetupViews - 1) / kSetupViews);
   InlineViews<1> a{};
   if (one) {
     a.v[0] = *one;
-    hipLaunchKernelGGL(k_rt_setup<true>, grid, dim3(256), 0, st, a, nullptr, views, 1, m, bins);
+    hipLaunchKernelGGL(k_rt_setup<true>, grid, dim3(256), 0, st, a, nullptr, views, 1, m, bins,
+                       large);
   } else {
-    hipLaunchKernelGGL(k_rt_setup<false>, grid, dim3(256), 0, st, a, views, nullptr, n_views, m, bins);
+    hipLaunchKernelGGL(k_rt_setup<false>, grid, dim3(256), 0, st, a, views, nullptr, n_views, m, bins,
+                       large);
   }
-  hipLaunchKernelGGL(k_rt_tiles, dim3(bins.total_tiles), dim3(256), 0, st, views, m, bins, o);
+  hipLaunchKernelGGL(k_rt_tiles, dim3(bins.total_tiles), dim3(256), 0, st, views, m, bins, large,
+                     o);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -44,7 +44,8 @@ int launch_depth_to_u16(hipStream_t st, const float* d, int64_t n, uint16_t* out
 int launch_raytrace(hipStream_t st, const DevView* views, int n_views, int total_tiles,
                     const DevBvh& bvh, const DevMesh& m, const DevOptions& o);
 int launch_raytrace_binned(hipStream_t st, const DevView* one, DevView* views, int n_views,
-                           const DevMesh& m, const DevBins& bins, const DevOptions& o);
+                           const DevMesh& m, const DevBins& bins, const RtLarge& large,
+                           const DevOptions& o);
 int launch_texture_map(hipStream_t st, const void* faces, int n, const void* images, int cols,
                        int rows, int hk, int32_t* owner, uint8_t* tex0, uint8_t* mask0,
                        uint8_t* tex, uint8_t* mask);
@@ -174,6 +175,9 @@ struct ugu_hip_ctx {
   bool rt_bins = false;      // few enough layers of faces for the binned path
   int32_t rt_cap = 1024;     // entries per tile of the raytracer's bins
   std::vector<RtRefusal> rt_refusals;
+  DevBuf rt_large;           // counters (two sets) and lists of large faces
+  int rt_large_views = 0;    // views whose next set of counters is clear
+  int rt_large_set = 0;
   int clean_tiles = 0;  // leading tile counters known to be clear, of view 0
   CopyRing ring;                 // pinned slots of the copies to and from host arrays
   void* h_views = nullptr;
@@ -905,6 +909,13 @@ int raytrace_binned(ugu_hip_ctx* c, DevView* hv, int n, const DevMesh& dm, const
     return 0;
   }
   const bool inline_views = n <= kInlineViews;
+  const size_t count_bytes = (size_t(n) * 4 + 255) / 256 * 256;
+  const int lr = c->rt_large.ensure(2 * count_bytes + size_t(n) * kRtLargeFaces * 16);
+  if (lr != 0) c->rt_large_views = 0;
+  if (lr < 0) {
+    (void)hipGetLastError();
+    return 0;
+  }
   if (!inline_views)
     UGU_HIP_CHECK(c, hipMemcpyAsync(c->views.p, hv, size_t(n) * sizeof(DevView),
                                     hipMemcpyHostToDevice, c->stream));
@@ -923,6 +934,16 @@ int raytrace_binned(ugu_hip_ctx* c, DevView* hv, int n, const DevMesh& dm, const
     b.status = c->status.as<int32_t>();
     b.host_flag = c->h_status;
     c->h_status[0] = 0;
+    uint8_t* lp = c->rt_large.as<uint8_t>();
+    if (c->rt_large_views != n) {
+      UGU_HIP_CHECK(c, hipMemsetAsync(lp, 0, 2 * count_bytes, c->stream));
+      c->rt_large_set = 0;
+    }
+    c->rt_large_views = 0;  // until the pass has completed
+    RtLarge large;
+    large.list = reinterpret_cast<int4*>(lp + 2 * count_bytes);
+    large.count = reinterpret_cast<int32_t*>(lp + size_t(c->rt_large_set) * count_bytes);
+    large.clear = reinterpret_cast<int32_t*>(lp + size_t(1 - c->rt_large_set) * count_bytes);
     DevView* dv = c->views.as<DevView>();
     const bool fresh = n == 1 && b.total_tiles <= c->clean_tiles;
     const int clean = c->clean_tiles;
@@ -930,9 +951,11 @@ int raytrace_binned(ugu_hip_ctx* c, DevView* hv, int n, const DevMesh& dm, const
     if (!fresh &&
         launch_begin(c->stream, inline_views ? hv : nullptr, n, dv, b.counts, b.total_tiles, b.status))
       return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
-    if (launch_raytrace_binned(c->stream, fresh ? hv : nullptr, dv, n, dm, b, dopt))
+    if (launch_raytrace_binned(c->stream, fresh ? hv : nullptr, dv, n, dm, b, large, dopt))
       return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
     UGU_HIP_CHECK(c, hipStreamSynchronize(c->stream));
+    c->rt_large_views = n;
+    c->rt_large_set = 1 - c->rt_large_set;
     int32_t most = 0;
     if ((err = read_overflow(c, b.status, &most))) return err;
     // tiles that saw an overflow left their counters as they were
@@ -1117,7 +1140,7 @@ void ugu_hip_destroy(ugu_hip_ctx* c) {
                     &c->bwd_items, &c->bwd_scratch, &c->soup, &c->diff_soup, &c->shade, &c->blk_off,
                     &c->blk_vid, &c->face_loc, &c->blk_off_o, &c->blk_vid_o, &c->face_loc_o,
                     &c->bvh_nodes, &c->bvh_leaves, &c->bvh_tris, &c->vis_items,
-                    &c->vis_images, &c->vis_out, &c->tm_faces, &c->tm_images, &c->tm_out};
+                    &c->vis_images, &c->vis_out, &c->rt_large, &c->tm_faces, &c->tm_images, &c->tm_out};
   for (DevBuf* b : bufs) b->release();
   c->ring.release();
   if (c->h_views) (void)hipHostFree(c->h_views);
