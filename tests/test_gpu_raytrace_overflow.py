@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 TILE = 16
 
 
-def _clusters(w, h, full, per_side, others, seed):
+def _clusters(w, h, full, per_side, others, seed, far=5.0):
     """Triangles three pixels wide, whole inside one tile each: `per_side` clockwise
     and as many counter-clockwise ones on screen in every tile of `full`, `others`
     of each in every other tile."""
@@ -30,7 +30,7 @@ def _clusters(w, h, full, per_side, others, seed):
         for flip in (False, True):
             at = lo + rng.uniform(0.0, TILE - 5.0, (n, 1, 2))
             xy = at + (shape[::-1] if flip else shape)
-            z = rng.uniform(2.0, 5.0, (n, 1, 1)).repeat(3, 1)
+            z = rng.uniform(2.0, far, (n, 1, 1)).repeat(3, 1)
             pts.append(np.concatenate([(xy - c) / f * z, z], -1))
     p = np.concatenate(pts)
     p = p[rng.permutation(len(p))]
@@ -80,7 +80,7 @@ def test_dense_tile_is_not_tried_on_every_call(gpu_available):
     """2500 front and 2500 back faces on a tile exceed what a bin may hold (4096): the
     hierarchy traces the view, and the bins are tried again ever more rarely. After
     PrepareMesh, and for a view of other tiles, they are tried at once."""
-    mesh, cam = _clusters(160, 96, (17,), 2500, 20, 3)
+    mesh, cam = _clusters(160, 96, (17,), 2500, 20, 3, far=9.0)  # few layers from the side
     corner = PinholeCamera(64, 48, np.eye(4), tuple(cam.principal_point), tuple(cam.focal_length))
     r = Raytracer(RendererCpuOption(diffuse_color=DiffuseColor.kVertex))
     r.set_mesh(mesh)

@@ -317,4 +317,51 @@ int build_bvh(const float* faces12, int32_t F, int max_inner_depth, BvhBuild* ou
   return 0;
 }
 
+double max_layers(const BvhBuild& b, int min_faces) {
+  struct Part {
+    double area = 0.0;  // of the faces below the node
+    int64_t faces = 0;
+  };
+  const size_t nn = b.nodes.size() / 16;
+  std::vector<Part> part(nn);
+  double most = 0.0;
+  for (size_t i = nn; i-- > 0;) {  // children follow their parent
+    Part& p = part[i];
+    double lo[3], hi[3];
+    for (int slot = 0; slot < 2; slot++) {
+      const float* c = &b.nodes[i * 16 + size_t(slot) * 8];
+      const int32_t ref = float_bits(c[3]);
+      if (ref == INT32_MIN) continue;
+      for (int k = 0; k < 3; k++) {
+        lo[k] = slot == 0 ? double(c[k]) : std::min(lo[k], double(c[k]));
+        hi[k] = slot == 0 ? double(c[4 + k]) : std::max(hi[k], double(c[4 + k]));
+      }
+      if (ref >= 0) {
+        p.area += part[size_t(ref)].area;
+        p.faces += part[size_t(ref)].faces;
+        continue;
+      }
+      const int32_t* leaf = &b.leaves[size_t(~ref) * 2];
+      p.faces += leaf[1];
+      for (int32_t f = leaf[0]; f < leaf[0] + leaf[1]; f++) {
+        const float* t = &b.tris[size_t(f) * 12];
+        double e1[3], e2[3];
+        for (int k = 0; k < 3; k++) {
+          e1[k] = double(t[4 + k]) - t[k];
+          e2[k] = double(t[8 + k]) - t[k];
+        }
+        const double x = e1[1] * e2[2] - e1[2] * e2[1];
+        const double y = e1[2] * e2[0] - e1[0] * e2[2];
+        const double z = e1[0] * e2[1] - e1[1] * e2[0];
+        p.area += 0.5 * std::sqrt(x * x + y * y + z * z);
+      }
+    }
+    if (p.faces < min_faces && i > 0) continue;
+    const double d[3] = {hi[0] - lo[0], hi[1] - lo[1], hi[2] - lo[2]};
+    const double face = (d[0] * d[1] + d[1] * d[2] + d[2] * d[0]) / 3.0;
+    if (face > 0.0) most = std::max(most, 0.5 * p.area / face);
+  }
+  return most;
+}
+
 }  // namespace ugu_hip

@@ -28,4 +28,11 @@ struct BvhBuild {
 // depth bound).
 int build_bvh(const float* faces12, int32_t F, int max_inner_depth, BvhBuild* out);
 
+// Mean number of faces that a line through a part of the mesh meets, where it meets
+// most: the largest of half the faces' area (a face's mean projection) over the mean
+// face of the box, over the nodes with at least min_faces faces and the root. A
+// closed surface has about 1.6, two plates close to each other 3. (Over the whole
+// mesh's box alone, one far face would hide any dense part.)
+double max_layers(const BvhBuild& b, int min_faces);
+
 }  // namespace ugu_hip

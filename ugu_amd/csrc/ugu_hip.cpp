@@ -826,40 +826,15 @@ bool rt_view_bounds(const ugu_hip_ctx* c, DevView* v) {
 //
 // The bins test every face over a pixel that nothing nearer hides yet, the
 // hierarchy's cost grows with the number of faces but hardly with the layers
-// behind the first. So the line is drawn at the mesh's mean number of layers
-// (rt_layers). Both sides, one 640x480 view, bins against hierarchy, random
-// triangles of half extent s: 1 M, s 0.01 (2.4 layers) 138 / 875 us; 1 M, s 0.03
-// (21) 348 / 378; 100 k, s 0.1 (24) 193 / 192; 10 k, s 0.3 (21) 165 / 138; 1 k, s 1
-// (24) 311 / 120; 1 M, s 0.1 (240) 1010 / 282. Closed surfaces have about two:
-// the 1.3 M-face sphere at 1080p 126 / 846 us, 327 k faces at 64x64 88 / 463,
-// 5 k faces at 160x120 59 / 105.
-constexpr double kRtMaxLayers = 8.0;
-
-// Mean number of faces a line through the mesh's bounding box meets: half the
-// faces' area (a face's mean projection) over the box's mean face.
-double rt_layers(const float* rec, int64_t F) {
-  double area = 0.0, lo[3] = {1e300, 1e300, 1e300}, hi[3] = {-1e300, -1e300, -1e300};
-  for (int64_t f = 0; f < F; f++) {
-    const float* p = rec + f * 12;
-    double e[2][3];
-    bool finite = true;
-    for (int k = 0; k < 9; k++) finite = finite && std::isfinite(p[k]);
-    if (!finite) continue;
-    for (int k = 0; k < 3; k++) {
-      e[0][k] = double(p[3 + k]) - p[k];
-      e[1][k] = double(p[6 + k]) - p[k];
-      lo[k] = std::min({lo[k], double(p[k]), double(p[3 + k]), double(p[6 + k])});
-      hi[k] = std::max({hi[k], double(p[k]), double(p[3 + k]), double(p[6 + k])});
-    }
-    const double x = e[0][1] * e[1][2] - e[0][2] * e[1][1];
-    const double y = e[0][2] * e[1][0] - e[0][0] * e[1][2];
-    const double z = e[0][0] * e[1][1] - e[0][1] * e[1][0];
-    area += 0.5 * std::sqrt(x * x + y * y + z * z);
-  }
-  const double d[3] = {hi[0] - lo[0], hi[1] - lo[1], hi[2] - lo[2]};
-  const double face = (d[0] * d[1] + d[1] * d[2] + d[2] * d[0]) / 3.0;
-  return face > 0.0 ? 0.5 * area / face : 0.0;
-}
+// behind the first. So the line is drawn at the number of layers where the mesh is
+// densest (max_layers; a mean over the mesh's box would be fooled by one far face).
+// Both sides, one 1080p view, bins against hierarchy, random triangles: 100 k of
+// them, 1 layer 178 / 498 us, 4 layers 313 / 349, 8 408 / 327, 16 504 / 338; 10 k
+// 148 / 257, 246 / 249, 320 / 282, 405 / 426; 1 k 137 / 171, 197 / 250, 262 / 316,
+// 387 / 457. Closed surfaces have about two: the 1.3 M-face sphere at 1080p
+// 106 / 846 us, 327 k faces at 64x64 88 / 463, 5 k faces at 160x120 59 / 105.
+constexpr double kRtMaxLayers = 5.0;
+constexpr int kRtLayerFaces = 128;  // a part of fewer faces costs little either way
 
 constexpr int32_t kRtMaxCap = 4096;
 
@@ -1386,7 +1361,7 @@ int ugu_hip_prepare_raytracer(ugu_hip_ctx* c) {
       if (std::isfinite(l)) c->rt_max_edge = std::max(c->rt_max_edge, l);
     }
   }
-  c->rt_bins = rt_layers(rec.data(), c->F) <= kRtMaxLayers;
+  c->rt_bins = max_layers(b, kRtLayerFaces) <= kRtMaxLayers;
   c->rt_refusals.clear();
   c->rt_mesh_gen = c->mesh_gen;
   c->rt_ready = true;
