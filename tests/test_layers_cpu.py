@@ -64,7 +64,7 @@ def test_plates(layers, n):
 @pytest.mark.parametrize("scale,offset", [(1.0, 0.0), (1e-3, 0.0), (0.05, 40.0)])
 def test_dense_part_is_found(layers, n, size, scale, offset):
     """One face far away does not thin out the dense part. A large sphere around it may
-    (no node need hold just the part), but not to fewer than the 5 layers that rule."""
+    where its nodes are split through the part: to 5 layers at the least here."""
     soup = _soup(n, size)
     alone = layers(soup)
     assert alone > 10.0

@@ -829,11 +829,13 @@ bool rt_view_bounds(const ugu_hip_ctx* c, DevView* v) {
 // behind the first. So the line is drawn at the number of layers where the mesh is
 // densest (max_layers; a mean over the mesh's box would be fooled by one far face).
 // Both sides, one 1080p view, bins against hierarchy, random triangles: 100 k of
-// them, 1 layer 178 / 498 us, 4 layers 313 / 349, 8 408 / 327, 16 504 / 338; 10 k
-// 148 / 257, 246 / 249, 320 / 282, 405 / 426; 1 k 137 / 171, 197 / 250, 262 / 316,
-// 387 / 457. Closed surfaces have about two: the 1.3 M-face sphere at 1080p
-// 106 / 846 us, 327 k faces at 64x64 88 / 463, 5 k faces at 160x120 59 / 105.
-constexpr double kRtMaxLayers = 5.0;
+// them, 3.7 layers 178 / 498 us, 14 313 / 349, 27 408 / 327; 10 k, 3.4 layers
+// 148 / 257, 12 246 / 249, 22 320 / 282; 1 k, 2.6 layers 137 / 171, 7.6 197 / 250,
+// 12 262 / 316. First calls of a mesh are even at 10 k and 7 layers (315 / 346), so
+// the line lies below the crossing of later ones. Closed surfaces have about 1.6: the
+// 1.3 M-face sphere at 1080p 106 / 846 us, 327 k faces at 64x64 88 / 463, 5 k faces at
+// 160x120 59 / 105.
+constexpr double kRtMaxLayers = 8.0;
 constexpr int kRtLayerFaces = 128;  // a part of fewer faces costs little either way
 
 constexpr int32_t kRtMaxCap = 4096;
