@@ -49,8 +49,25 @@ def _check(out, ref, label):
         np.testing.assert_allclose(out[k], ref[k], rtol=1e-5, atol=1e-7)
 
 
+AT = 960  # where the small view lies in the large one, in x and y
+
+
+def _large(cam):
+    """A view with the small one at (AT, AT), of so many tiles (16641) that the bins
+    start with 1024 entries each; fewer tiles get more of the same memory."""
+    c = np.asarray(cam.principal_point) + AT
+    return PinholeCamera(2064, 2064, np.eye(4), tuple(c), tuple(cam.focal_length))
+
+
+def _crop(out, w, h):
+    mask = out["mask"].copy()
+    mask[AT:AT + h, AT:AT + w] = 0
+    assert not mask.any()
+    return {k: v[AT:AT + h, AT:AT + w] for k, v in out.items()}
+
+
 @pytest.mark.parametrize("full", [(0,), (3, 17, 29, 59), tuple(range(0, 60, 6))])
-@pytest.mark.parametrize("views", [1, 3])
+@pytest.mark.parametrize("views", [1, 2])
 def test_segments_overflow_together(gpu_available, full, views):
     mesh, cam = _clusters(160, 96, full, 700, 20, len(full))
     opt = RendererCpuOption(diffuse_color=DiffuseColor.kVertex)
@@ -60,8 +77,11 @@ def test_segments_overflow_together(gpu_available, full, views):
     r.set_mesh(mesh)
     assert r.PrepareMesh()
     for call in range(2):
-        for out in r.render_batch([cam] * views):
-            _check(out, ref, call)
+        for out in r.render_batch([_large(cam)] * views):
+            _check(_crop(out, 160, 96), ref, call)
+        assert r.timings()["retries"] == 1 - call
+    for out in r.render_batch([cam] * views):
+        _check(out, ref, "small")
 
 
 def _retries(r, cam, calls):
@@ -96,7 +116,8 @@ def test_bins_that_grew_are_kept(gpu_available):
     r = Raytracer(RendererCpuOption(diffuse_color=DiffuseColor.kVertex))
     r.set_mesh(mesh)
     assert r.PrepareMesh()
-    assert _retries(r, cam, 4) == [1, 0, 0, 0]
+    assert _retries(r, _large(cam), 4) == [1, 0, 0, 0]
+    assert _retries(r, cam, 2) == [0, 0]
 
 
 @pytest.mark.parametrize("value", [np.nan, np.inf, -np.inf])
@@ -123,3 +144,46 @@ def test_faces_that_are_not_finite_fill_no_bins(gpu_available, value):
     for call in range(2):
         _check(r.render_batch([cam])[0], ref, value)
         assert r.timings()["retries"] == 0
+
+
+def _used():
+    import torch
+    torch.cuda.synchronize()
+    free, total = torch.cuda.mem_get_info()
+    return total - free
+
+
+def _masks(r, cams):
+    import torch
+    bufs = [{"mask": torch.zeros((c.height, c.width), dtype=torch.uint8, device="cuda")}
+            for c in cams]
+    torch.cuda.synchronize()
+    r.render_device(cams, bufs)
+    return [b["mask"] for b in bufs]
+
+
+def test_memory_of_the_bins(gpu_available):
+    """A dense tile of one mesh does not size the bins of the next mesh's views (262144
+    tiles: 2 GiB for 1024 faces each, 7 GiB for what the first mesh needed), and views
+    whose bins would take more than 8 GiB go to the hierarchy."""
+    import torch
+    r = Raytracer(RendererCpuOption(diffuse_color=DiffuseColor.kVertex))
+    dense, cam = _clusters(160, 96, (17,), 1500, 20, 4)
+    r.set_mesh(dense)
+    assert r.PrepareMesh()
+    _retries(r, cam, 2)
+    ball, _ = _clusters(160, 96, (17,), 100, 20, 5)
+    r.set_mesh(ball)
+    assert r.PrepareMesh()
+    cams = [PinholeCamera(2048, 2048, np.eye(4), (1023.5 - k, 1000.0), (1800.0, 1800.0))
+            for k in range(80)]
+    one = _masks(r, cams[:1])[0].cpu()
+    before = _used()
+    few = _masks(r, cams[:16])
+    assert _used() - before < 3 << 30
+    assert torch.equal(few[0].cpu(), one) and bool(one.any())
+    held = _used()
+    many = _masks(r, cams)
+    assert _used() - held < 1 << 30
+    for a, b in zip(few, many):
+        assert torch.equal(a, b)

@@ -173,7 +173,7 @@ struct ugu_hip_ctx {
   int64_t rt_mesh_gen = -1;  // mesh generation the hierarchy was built for
   float rt_max_coord = 0.0f, rt_max_edge = 0.0f;  // 1-norms, for the binned path's bounds
   bool rt_bins = false;      // few enough layers of faces for the binned path
-  int32_t rt_cap = 1024;     // entries per tile of the raytracer's bins
+  int32_t rt_cap = 0;        // entries per tile that the mesh's passes needed
   std::vector<RtRefusal> rt_refusals;
   DevBuf rt_large;           // counters (two sets) and lists of large faces
   int rt_large_views = 0;    // views whose next set of counters is clear
@@ -838,7 +838,30 @@ bool rt_view_bounds(const ugu_hip_ctx* c, DevView* v) {
 constexpr double kRtMaxLayers = 8.0;
 constexpr int kRtLayerFaces = 128;  // a part of fewer faces costs little either way
 
-constexpr int32_t kRtMaxCap = 4096;
+// Entries per tile of the bins: kRtMinCap, or more where the memory at hand, or
+// kRtBinBytes of it, holds more, up to kRtMaxCap. (A pass that overflows is paid twice
+// and allocates: a terrain of 320 k faces, first call at 640x480 1346 us with 1024
+// entries, 686 with 4096; at 1080p 1470 with 1024, 879 with 2056.) Passes that would
+// need more than kRtBinLimit, or more than a quarter of the free memory, go to the
+// hierarchy.
+constexpr int32_t kRtMinCap = 1024, kRtMaxCap = 4096;
+constexpr int64_t kRtBinBytes = int64_t(128) << 20, kRtBinLimit = int64_t(8) << 30;
+
+// Capacity of a pass over `total` tiles that needs rt_cap entries; 0: too large.
+int32_t rt_capacity(ugu_hip_ctx* c, int64_t total) {
+  const int64_t least = total * c->rt_cap * 8, have = static_cast<int64_t>(c->bins.bytes);
+  if (least > kRtBinLimit) return 0;
+  if (least > have && least > kRtBinBytes) {
+    size_t free_bytes = 0, all = 0;
+    if (hipMemGetInfo(&free_bytes, &all) != hipSuccess) {
+      (void)hipGetLastError();
+      return 0;
+    }
+    if (least > (static_cast<int64_t>(free_bytes) + have) / 4) return 0;
+  }
+  const int64_t room = std::max(have, kRtBinBytes) / 8 / total;
+  return static_cast<int32_t>(std::max<int64_t>(c->rt_cap, std::min<int64_t>(room, kRtMaxCap)));
+}
 
 // A pass whose bins do not fit has cost its setup, a part of its tiles and a wait
 // before the hierarchy traces it. So views that were refused are not tried again at
@@ -897,8 +920,8 @@ int raytrace_binned(ugu_hip_ctx* c, DevView* hv, int n, const DevMesh& dm, const
     UGU_HIP_CHECK(c, hipMemcpyAsync(c->views.p, hv, size_t(n) * sizeof(DevView),
                                     hipMemcpyHostToDevice, c->stream));
   for (;;) {
-    if (total * c->rt_cap * 8 > (int64_t(32) << 30)) return 0;
-    if (ensure(c, c->bins, size_t(total) * size_t(c->rt_cap) * 8)) {
+    const int32_t cap = rt_capacity(c, total);
+    if (cap == 0 || ensure(c, c->bins, size_t(total) * size_t(cap) * 8)) {
       (void)hipGetLastError();
       rt_refused(c, n, total);
       return 0;
@@ -906,7 +929,7 @@ int raytrace_binned(ugu_hip_ctx* c, DevView* hv, int n, const DevMesh& dm, const
     DevBins b;
     b.counts = c->counts.as<int32_t>();
     b.bins = c->bins.as<int2>();
-    b.cap = c->rt_cap;
+    b.cap = cap;
     b.total_tiles = static_cast<int32_t>(total);
     b.status = c->status.as<int32_t>();
     b.host_flag = c->h_status;
@@ -938,7 +961,7 @@ int raytrace_binned(ugu_hip_ctx* c, DevView* hv, int n, const DevMesh& dm, const
     // tiles that saw an overflow left their counters as they were
     if (n == 1 && most == 0) c->clean_tiles = std::max(clean, b.total_tiles);
     c->tm.max_bin_count = std::max(c->tm.max_bin_count, most);
-    if (most <= c->rt_cap) {
+    if (most <= cap) {
       if (RtRefusal* r = rt_refusal(c, n, total))
         c->rt_refusals.erase(c->rt_refusals.begin() + (r - c->rt_refusals.data()));
       return 1;
@@ -948,7 +971,8 @@ int raytrace_binned(ugu_hip_ctx* c, DevView* hv, int n, const DevMesh& dm, const
       rt_refused(c, n, total);
       return 0;
     }
-    c->rt_cap = static_cast<int32_t>(std::min<int64_t>(kRtMaxCap, (int64_t(most) + most / 8 + 63) / 64 * 64));
+    const int64_t grown = (int64_t(most) + most / 8 + 63) / 64 * 64;
+    c->rt_cap = static_cast<int32_t>(std::min<int64_t>(kRtMaxCap, grown));
   }
 }
 
@@ -1365,6 +1389,7 @@ int ugu_hip_prepare_raytracer(ugu_hip_ctx* c) {
   }
   c->rt_bins = max_layers(b, kRtLayerFaces) <= kRtMaxLayers;
   c->rt_refusals.clear();
+  c->rt_cap = kRtMinCap;
   c->rt_mesh_gen = c->mesh_gen;
   c->rt_ready = true;
   return UGU_HIP_OK;
