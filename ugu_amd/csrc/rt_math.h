@@ -57,6 +57,32 @@ RT_HD bool mt_hit(double ox, double oy, double oz, double dx, double dy, double 
   return true;
 }
 
+// At least the length of c2w_R times a unit vector, the rays' length: with q the mean
+// of the diagonal of B = R^T R and p^2 a sixth of |B - q|^2 (Frobenius), the
+// eigenvalues of B are q + 2 p cos(.), and the largest is at most q + 2 p (a rotation:
+// 1). NaN or infinite if R is not finite.
+inline double max_ray_length(const float* R) {
+  double q = 0.0, d2 = 0.0, b[3][3];
+  for (int i = 0; i < 3; i++)
+    for (int j = 0; j < 3; j++)
+      b[i][j] = double(R[i]) * R[j] + double(R[3 + i]) * R[3 + j] + double(R[6 + i]) * R[6 + j];
+  for (int i = 0; i < 3; i++) q += b[i][i] / 3.0;
+  for (int i = 0; i < 3; i++)
+    for (int j = 0; j < 3; j++) {
+      const double d = b[i][j] - (i == j ? q : 0.0);
+      d2 += d * d;
+    }
+  return sqrt(q + 2.0 * sqrt(d2 / 6.0));
+}
+
+// Bound of the absolute rounding error of mt_hit's det and of the numerators of its
+// two barycentrics: a dozen roundings of 2^-53 of products that sum to at most
+// ray (length) x edge x (reach + edge) (1-norms of the longest edge and of the largest
+// distance of a corner from the origin).
+inline double hit_rounding(double ray, double edge, double reach) {
+  return 0x1p-49 * ray * edge * (reach + edge);
+}
+
 // Relative slack of the box test (2^-20): covers the float rounding of the
 // slab arithmetic (a few ulp).
 constexpr float kBoxSlack = 9.5367431640625e-07f;

@@ -783,9 +783,9 @@ int run_noalloc(ugu_hip_ctx* c, uint8_t* base, const UguCamera* cams, int n, con
 // The binned raytracer's numbers of one view (project_ray): the inverse of
 // c2w_R and the rounding bounds. False where the bounds do not hold or would
 // be too wide to prune anything: the view goes through the hierarchy. Bounds:
-// a hit the float64 test accepts has |det| >= 1e-8, so its barycentrics carry
-// at most 2^-49 1e8 L (S + L) of absolute error (L: longest edge, S: largest
-// corner distance, 1-norms; 2^-49: a dozen roundings of 2^-53).
+// a hit the float64 test accepts has |det| >= 1e-8, so its barycentrics carry at most
+// 1e8 hit_rounding of absolute error (longest edge, largest corner distance, longest
+// ray of the view).
 bool rt_view_bounds(const ugu_hip_ctx* c, DevView* v) {
   double a[9], inv[9], na = 0.0, ni = 0.0;
   for (int k = 0; k < 9; k++) {
