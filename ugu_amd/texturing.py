@@ -135,32 +135,39 @@ def face_records(mesh, best, tex_w, tex_h):
 # destroying a context with its workspace takes 400 us of the 1.1 ms of a
 # 1024 x 1024 call. A call takes the context out and puts it back, so calls of
 # several threads never share one; it is kept only while its workspace is small,
-# not across a fork, and given back at exit.
+# not across a fork, and given back at exit. The workspace's parts (images, records,
+# planes) only grow: each is as large as the largest call so far made it.
 _SPARE_BYTES = 256 << 20
 _spare = {}
 
 
-def _give_context(lib, device, ctx, workspace_bytes):
-    if workspace_bytes > _SPARE_BYTES or _spare.setdefault((os.getpid(), device), ctx) != ctx:
+def _take_context(lib, device):
+    return _spare.pop((os.getpid(), device), None) or (lib.ugu_hip_create(device), (0, 0, 0))
+
+
+def _give_context(lib, device, ctx, held):
+    spare = (ctx, held)
+    if held is None or sum(held) > _SPARE_BYTES \
+            or _spare.setdefault((os.getpid(), device), spare) is not spare:
         lib.ugu_hip_destroy(ctx)
 
 
 @atexit.register
 def _release_spares():
     for key in list(_spare):
-        ctx = _spare.pop(key, None)
-        if ctx and key[0] == os.getpid():
-            _abi.load_library().ugu_hip_destroy(ctx)
+        spare = _spare.pop(key, None)
+        if spare and key[0] == os.getpid():
+            _abi.load_library().ugu_hip_destroy(spare[0])
 
 
 def texture_map_faces(images, recs, n, tex_w, tex_h, padding_kernel, device=0):
     """ugu_hip_texture_map -> (texture (tex_h, tex_w, 3) uint8, mask)."""
     lib = _abi.load_library()
     device = int(device)
-    ctx = _spare.pop((os.getpid(), device), None) or lib.ugu_hip_create(device)
+    ctx, held = _take_context(lib, device)
     if not ctx:
         raise RuntimeError(f"ugu_hip_create({device}) failed: no usable HIP device")
-    workspace = sys.maxsize  # not kept after an error
+    kept = None  # not after an error
     try:
         imgs = [contiguous_u8(im) for im in images]
         tex_arr = (_abi.UguTexture * max(1, len(imgs)))()
@@ -173,10 +180,11 @@ def texture_map_faces(images, recs, n, tex_w, tex_h, padding_kernel, device=0):
         if rc != 0:
             raise _abi.HipError(rc, lib.ugu_hip_last_error(ctx).decode())
         # images, records, and the owner, texture and mask planes
-        workspace = sum(im.size for im in imgs) + ctypes.sizeof(recs) + 13 * tex_w * tex_h
+        parts = (sum(im.size for im in imgs), ctypes.sizeof(recs), 13 * tex_w * tex_h)
+        kept = tuple(map(max, held, parts))
         return tex, mask
     finally:
-        _give_context(lib, device, ctx, workspace)
+        _give_context(lib, device, ctx, kept)
 
 
 def simple_tile(keyframes, best, mesh, option):
