@@ -2,9 +2,10 @@
 // vertex colours, texture) at fixed visibility. The covered pixels of all views
 // are sorted into (face, view, pixel) items by groups of consecutive faces with
 // a counting sort:
-//   k_bwd_count    one thread per pixel: pixels per face group
-//   k_bwd_offsets  exclusive scan of the counts (one block)
-//   k_bwd_scatter  one thread per pixel: the items
+//   k_bwd_count    four pixels per thread: pixels per face group
+//   k_bwd_offsets  exclusive scan of the counts (one launch, at most 16 blocks, each
+//                  of which sums the counts before its own)
+//   k_bwd_scatter  four pixels per thread: the items
 //   k_bwd_items    one thread per item: derivatives in float64, summed per
 //                  vertex and texel in a block's LDS tables before the global
 //                  atomics
@@ -22,7 +23,7 @@ namespace ugu_hip {
 // Faces fid >> shift share a group; the shift keeps the groups below kBwdGroups.
 // Coarse groups give long runs: 64 views of 1.3 M faces take 0.5 M counter atomics
 // per pass instead of 6.8 M with a counter per face (count 281 -> 130 us, scatter
-// 404 -> 166 us), and the one-block offsets fit one kernel instead of three.
+// 404 -> 166 us), and the offsets fit one kernel instead of three.
 constexpr int kBwdGroups = 16384;
 
 int backward_group_shift(int32_t F) {

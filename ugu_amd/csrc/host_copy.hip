@@ -48,24 +48,14 @@ struct DevChunk {
   uint32_t seq;  // to the host: the value the slot's flag takes
 };
 
-template <class T>
-__device__ __forceinline__ void copy_words(unsigned char* dst, const unsigned char* src, uint32_t n) {
-  for (uint32_t i = threadIdx.x; i < n; i += kCopyThreads)
-    reinterpret_cast<T*>(dst)[i] = reinterpret_cast<const T*>(src)[i];
-}
-
+// Slots and, by queue_direct's check, device addresses are multiples of 16.
 __device__ __forceinline__ void copy_chunk(unsigned char* dst, const unsigned char* src,
-                                           uint32_t bytes, const unsigned char* dev) {
-  const uint32_t mis = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(dev));
-  uint32_t done = 0;
-  if ((mis & 15u) == 0) {
-    copy_words<uint4>(dst, src, bytes / 16);
-    done = bytes & ~15u;
-  } else if ((mis & 3u) == 0) {
-    copy_words<uint32_t>(dst, src, bytes / 4);
-    done = bytes & ~3u;
-  }
-  copy_words<unsigned char>(dst + done, src + done, bytes - done);
+                                           uint32_t bytes) {
+  const uint32_t words = bytes / 16;
+  for (uint32_t i = threadIdx.x; i < words; i += kCopyThreads)
+    reinterpret_cast<uint4*>(dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+  const uint32_t i = words * 16 + threadIdx.x;
+  if (i < bytes) dst[i] = src[i];
 }
 
 // A block per chunk in turn; `slots`, `table` and `flags` are pinned host memory.
@@ -74,7 +64,7 @@ __global__ __launch_bounds__(kCopyThreads) void k_to_slots(const DevChunk* table
                                                            unsigned char* slots, uint32_t* flags) {
   for (int k = blockIdx.x; k < n; k += gridDim.x) {
     const DevChunk c = table[k];
-    copy_chunk(slots + size_t(k) * kChunkBytes, c.dev, c.bytes, c.dev);
+    copy_chunk(slots + size_t(k) * kChunkBytes, c.dev, c.bytes);
     __threadfence_system();
     __syncthreads();
     if (threadIdx.x == 0)
@@ -86,7 +76,7 @@ __global__ __launch_bounds__(kCopyThreads) void k_from_slots(const DevChunk* tab
                                                              const unsigned char* slots) {
   for (int k = blockIdx.x; k < n; k += gridDim.x) {
     const DevChunk c = table[k];
-    copy_chunk(c.dev, slots + size_t(k) * kChunkBytes, c.bytes, c.dev);
+    copy_chunk(c.dev, slots + size_t(k) * kChunkBytes, c.bytes);
   }
 }
 
@@ -283,8 +273,8 @@ bool overlap(const HostCopy* c, int n) {
 }
 
 // Queues the copies that the engine makes: of pinned arrays (from kMinDirect bytes
-// of them in all on), of memory that is not the host's, and, where fewer than
-// `least` bytes would be left or results overlap, all of them. The others are
+// of them in all on), of memory that is not the host's or not aligned on the device, and,
+// where fewer than `least` bytes would be left or results overlap, all of them. The others are
 // returned in *slots.
 hipError_t queue_direct(hipStream_t st, const HostCopy* c, int n, bool out, size_t least,
                         std::vector<HostCopy>* slots) {
@@ -292,7 +282,7 @@ hipError_t queue_direct(hipStream_t st, const HostCopy* c, int n, bool out, size
   size_t pinned = 0, left = 0;
   for (int i = 0; i < n; i++) {
     if (c[i].bytes == 0) continue;
-    kind[size_t(i)] = memory_of(c[i]);
+    if (reinterpret_cast<uintptr_t>(c[i].dev) % 16 == 0) kind[size_t(i)] = memory_of(c[i]);
     if (kind[size_t(i)] == Memory::kPinned) pinned += c[i].bytes;
     if (kind[size_t(i)] == Memory::kPageable) left += c[i].bytes;
   }

@@ -13,7 +13,8 @@
 // The closest hit is the smallest float t; equal t resolve to the lowest face
 // id. The box test is float32 with widened boxes and a relative slack on the
 // ray interval, so it only prunes boxes that cannot hold a hit the float64 test
-// would accept; the bins' bounds are those of project_ray. Then the pixel is culled or shaded as in raytracer.cc:160-218.
+// would accept; the bins' bounds are those of project_ray. Then the pixel is
+// culled or shaded as in raytracer.cc:160-218.
 
 #include "binning.h"
 #include "device_common.h"

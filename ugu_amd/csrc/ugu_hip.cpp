@@ -69,7 +69,8 @@ namespace {
 constexpr int kNoAllocMaxViews = 1024;
 constexpr int kMaxDevices = 64;
 // Layout of the scratch array (offsets 256-B aligned): status words (max bin
-// count, work-queue heads), the view descriptors, then per render group the tiles' counters and the bins.
+// count, work-queue heads), the view descriptors, then per render group the
+// tiles' counters and the bins.
 constexpr size_t kNaViewsOff = (size_t(kStatusBytes) + 255) / 256 * 256;
 constexpr size_t kNaCountsOff =
     (kNaViewsOff + size_t(kNoAllocMaxViews) * sizeof(DevView) + 255) / 256 * 256;
@@ -678,7 +679,8 @@ int render_common(ugu_hip_ctx* c, const UguCamera* cams, int n, const UguOptions
   return run_pipeline(c, cams, n, dm, dev_options(*o), 0, outs, memory, nullptr, nullptr, gbufs);
 }
 
-// The pipeline of run_pipeline (begin, setup+bin, raster) over the scratch array at `base` instead of the context's buffers.
+// The pipeline of run_pipeline (begin, setup+bin, raster) over the scratch array
+// at `base` instead of the context's buffers.
 // Views are rendered in consecutive groups whose tiles all get at least
 // `want` bin entries; a group in which a tile overflows is rendered again as
 // smaller groups with the measured occupancy as the new `want` (the tiles of
@@ -1606,7 +1608,7 @@ int ugu_hip_autotune(ugu_hip_ctx* c, const UguCamera* cams, int n, const UguOpti
     t.persistent = sh[2];
     t.bin_capacity = 256;
     c->tiling = t;
-      // first render sizes the bins from the measured occupancy
+    // first render sizes the bins from the measured occupancy
     err = render_common(c, cams, n, &opt, outs.data(), UGU_HIP_MEMORY_DEVICE);
     if (err) break;
     std::vector<double> times;
@@ -1628,7 +1630,7 @@ int ugu_hip_autotune(ugu_hip_ctx* c, const UguCamera* cams, int n, const UguOpti
   outbuf.release();
   if (err) {
     c->tiling = saved;
-      return err;
+    return err;
   }
   c->tiling = best;
   if (chosen) *chosen = best;
@@ -1679,7 +1681,7 @@ int ugu_hip_autotune_cached(ugu_hip_ctx* c, const UguCamera* cams, int n, const 
       std::fclose(f);
       if (hit) {
         c->tiling = found;
-              if (chosen) *chosen = found;
+        if (chosen) *chosen = found;
         if (from_cache) *from_cache = 1;
         return UGU_HIP_OK;
       }
