@@ -141,3 +141,27 @@ def test_large_faces_do_not_serialize_the_setup(gpu_available):
     alone = gpu_ms(v)
     room = gpu_ms(np.concatenate([v, np.asarray(quads)]))
     assert room < 4.0 * alone, (room, alone)
+
+
+def test_share_of_the_tiles(gpu_available):
+    """In a view of 16641 tiles the list takes faces over more than 32 of them."""
+    small = _camera(333, 241, f=220.0)
+    mesh = _mesh(_boxes(small, 400, (4, 5, 6, 9), 8))
+    ref = _reference(mesh, small)
+    at = 16 * 50
+    c = np.asarray(small.principal_point) + at
+    cam = PinholeCamera(2064, 2064, np.eye(4), tuple(c), tuple(small.focal_length))
+    r = _renderer(mesh)
+    for call in range(2):
+        out = r.render_batch([cam])[0]
+        _check({k: v[at:at + 241, at:at + 333] for k, v in out.items()}, ref, call)
+
+
+@pytest.mark.parametrize("views", [1, 5, 40])
+def test_few_faces_many_views(gpu_available, views):
+    """Blocks of the setup take one view each where they are few."""
+    cams = [_camera(64 + k % 5, 48, 0.02 * k) for k in range(views)]
+    mesh = _mesh(_boxes(cams[0], 50, (1, 2), 9))
+    r = _renderer(mesh)
+    for k, out in enumerate(r.render_batch(cams)):
+        _check(out, _reference(mesh, cams[k]), k)

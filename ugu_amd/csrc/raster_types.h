@@ -128,13 +128,15 @@ struct DevBins {
                        // reads the status only then
 };
 
-// The raytracer's large faces: faces over more than kRtLargeTiles tiles of a view are
-// kept in the view's list, which each of its tiles goes through, instead of in all
-// those bins. (A limit of 8 tiles: 300 k random faces at 1080p, most of them over 8 to
-// 16 tiles, 470 us, 16 tiles 359, 32 tiles 325; 82 k faces seen from close by at
-// 640x480 74, 78 and 85.) Two sets of counters take turns: a pass counts in one and clears the
-// other for the next pass (no block may clear a count that another still reads).
-constexpr int kRtLargeTiles = 16;
+// The raytracer's large faces: faces over more than kRtLargeTiles tiles of a view, and
+// more than one of kRtLargeShare tiles, are kept in the view's list, which each of its
+// tiles goes through, instead of in all those bins. (A limit of 8 tiles: 300 k random
+// faces at 1080p, most of them over 8 to 16 tiles, 470 us, 16 tiles 359, 32 tiles 325;
+// 82 k faces seen from close by at 640x480 74, 78 and 85. 5 k faces of 50 tiles at
+// 7680x4320: listed 1113 us, in the bins 559.) Two sets of counters take turns: a
+// pass counts in one and clears the other for the next pass (no block may clear a
+// count that another still reads).
+constexpr int kRtLargeTiles = 16, kRtLargeShare = 512;
 constexpr int kRtLargeFaces = 4096;  // per view; further ones go into the bins
 struct RtLarge {
   int4* list;      // kRtLargeFaces per view: face id, depth bound, x0 | x1 << 16, y0 | y1 << 16

@@ -20,6 +20,8 @@
 #include "device_common.h"
 #include "rt_math.h"
 
+#include <algorithm>
+
 #pragma clang fp contract(off)
 
 namespace ugu_hip {
@@ -276,8 +278,8 @@ UGU_DEV int2 rt_entry(int f, float zskip, int x0, int x1, int y0, int y1, int tx
 template <bool INL>
 __global__ __launch_bounds__(256) void k_rt_setup(InlineViews<1> arg,
                                                   const DevView* __restrict__ views, DevView* out,
-                                                  int n_views, DevMesh mesh, DevBins bins,
-                                                  RtLarge large) {
+                                                  int n_views, int block_views, DevMesh mesh,
+                                                  DevBins bins, RtLarge large) {
   if (INL && blockIdx.x == 0) {
     // an occupancy published before this store is published again by its tile
     clear_status(bins.status);
@@ -306,8 +308,8 @@ __global__ __launch_bounds__(256) void k_rt_setup(InlineViews<1> arg,
       P[j * 3 + 2] = q[2];
     }
   }
-  const int vb = blockIdx.y * kSetupViews;
-  const int ve = min(vb + kSetupViews, n_views);
+  const int vb = blockIdx.y * block_views;
+  const int ve = min(vb + block_views, n_views);
   for (int vi = vb; vi < ve; vi++) {
     const DevView& v = INL ? arg.v[0] : views[vi];
     for (int j = 0; j < 3; j++) {
@@ -384,7 +386,8 @@ __global__ __launch_bounds__(256) void k_rt_setup(InlineViews<1> arg,
     // a time: a ball in a room of 12 faces at 1080p 2330 us, listed 121 (hierarchy
     // 319); 82 k faces seen from close by at 640x480 107 and 78 (81).
     const int tiles = (x1 / kRtTile - x0 / kRtTile + 1) * (y1 / kRtTile - y0 / kRtTile + 1);
-    const uint64_t big = __builtin_amdgcn_ballot_w64(has && tiles > kRtLargeTiles);
+    const uint64_t big = __builtin_amdgcn_ballot_w64(
+        has && tiles > max(kRtLargeTiles, v.tiles_x * v.tiles_y / kRtLargeShare));
     if (big) {
       const int lane = __lane_id(), lead = __ffsll(static_cast<unsigned long long>(big)) - 1;
       int slot = 0;
@@ -811,15 +814,20 @@ int launch_raytrace_binned(hipStream_t st, const DevView* one, DevView* views, i
                            const DevMesh& m, const DevBins& bins, const RtLarge& large,
                            const DevOptions& o) {
   if (n_views < 1 || bins.total_tiles < 1 || m.F < 1) return 0;
-  const dim3 grid((m.F + 255) / 256, (n_views + kSetupViews - 1) / kSetupViews);
+  // a block's faces stay for kSetupViews views, fewer where the blocks would not fill
+  // the chip (320 faces, 24 views of 640x480: 661 us with eight,
+  // 550 with one)
+  const int fb = (m.F + 255) / 256;
+  const int per = std::max(1, std::min<int>(kSetupViews, int64_t(fb) * n_views / 1024));
+  const dim3 grid(fb, (n_views + per - 1) / per);
   InlineViews<1> a{};
   if (one) {
     a.v[0] = *one;
-    hipLaunchKernelGGL(k_rt_setup<true>, grid, dim3(256), 0, st, a, nullptr, views, 1, m, bins,
+    hipLaunchKernelGGL(k_rt_setup<true>, grid, dim3(256), 0, st, a, nullptr, views, 1, 1, m, bins,
                        large);
   } else {
-    hipLaunchKernelGGL(k_rt_setup<false>, grid, dim3(256), 0, st, a, views, nullptr, n_views, m, bins,
-                       large);
+    hipLaunchKernelGGL(k_rt_setup<false>, grid, dim3(256), 0, st, a, views, nullptr, n_views, per, m,
+                       bins, large);
   }
   hipLaunchKernelGGL(k_rt_tiles, dim3(bins.total_tiles), dim3(256), 0, st, views, m, bins, large,
                      o);

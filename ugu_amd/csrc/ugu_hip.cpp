@@ -849,6 +849,8 @@ constexpr int kRtLayerFaces = 128;  // a part of fewer faces costs little either
 constexpr int32_t kRtMinCap = 1024, kRtMaxCap = 4096;
 constexpr int64_t kRtBinBytes = int64_t(128) << 20, kRtBinLimit = int64_t(8) << 30;
 
+int64_t rt_all_faces(const ugu_hip_ctx* c) { return (int64_t(c->F) + 63) / 64 * 64; }
+
 // Capacity of a pass over `total` tiles that needs rt_cap entries; 0: too large.
 int32_t rt_capacity(ugu_hip_ctx* c, int64_t total) {
   const int64_t least = total * c->rt_cap * 8, have = static_cast<int64_t>(c->bins.bytes);
@@ -861,8 +863,9 @@ int32_t rt_capacity(ugu_hip_ctx* c, int64_t total) {
     }
     if (least > (static_cast<int64_t>(free_bytes) + have) / 4) return 0;
   }
-  const int64_t room = std::max(have, kRtBinBytes) / 8 / total;
-  return static_cast<int32_t>(std::max<int64_t>(c->rt_cap, std::min<int64_t>(room, kRtMaxCap)));
+  const int64_t room = std::min<int64_t>(std::max(have, kRtBinBytes) / 8 / total, kRtMaxCap);
+  // no tile can hold more than all faces
+  return static_cast<int32_t>(std::max<int64_t>(c->rt_cap, std::min(room, rt_all_faces(c))));
 }
 
 // A pass whose bins do not fit has cost its setup, a part of its tiles and a wait
@@ -1391,7 +1394,7 @@ int ugu_hip_prepare_raytracer(ugu_hip_ctx* c) {
   }
   c->rt_bins = max_layers(b, kRtLayerFaces) <= kRtMaxLayers;
   c->rt_refusals.clear();
-  c->rt_cap = kRtMinCap;
+  c->rt_cap = static_cast<int32_t>(std::min<int64_t>(kRtMinCap, rt_all_faces(c)));
   c->rt_mesh_gen = c->mesh_gen;
   c->rt_ready = true;
   return UGU_HIP_OK;
