@@ -622,15 +622,15 @@ UGU_DEV void diff_image(const DevView& v, const DevMesh& m, int fid, int px, int
   const double u = px - static_cast<double>(v.cx), w = py - static_cast<double>(v.cy);
   double ax[4], ay[4];
   for (int k = 0; k < 4; k++) {
-    const double c0 = k < 3 ? v.w2c_R[k] : v.w2c_t[0], c1 = k < 3 ? v.w2c_R[3 + k] : v.w2c_t[1],
-                 c2 = k < 3 ? v.w2c_R[6 + k] : v.w2c_t[2];
+    const double c0 = k < 3 ? v.w2c_R[k] : v.trel[0], c1 = k < 3 ? v.w2c_R[3 + k] : v.trel[1],
+                 c2 = k < 3 ? v.w2c_R[6 + k] : v.trel[2];
     ax[k] = v.fx * c0 - u * c2;
     ay[k] = v.fy * c1 - w * c2;
   }
   double X[3], Y[3];
   for (int j = 0; j < 3; j++) {
     const float* P = m.verts + int64_t(vid[j]) * 3;
-    const double p0 = P[0], p1 = P[1], p2 = P[2];
+    const double p0 = P[0] - v.org[0], p1 = P[1] - v.org[1], p2 = P[2] - v.org[2];
     X[j] = ax[0] * p0 + ax[1] * p1 + ax[2] * p2 + ax[3];
     Y[j] = ay[0] * p0 + ay[1] * p1 + ay[2] * p2 + ay[3];
   }

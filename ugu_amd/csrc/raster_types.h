@@ -32,13 +32,21 @@ struct DevView {
   float* pos_cam;
   float* nrm_wld;
   int32_t* geo_id;
-  // raytracer, binned path: inverse of c2w_R, and the error bounds of a point
-  // projected through it (see project_ray)
-  float inv[9];
-  float rt_rel;   // relative error of the projected camera coordinates
-  float rt_abs;   // pixel margin that every point gets
-  float rt_f;     // max(|fx|, |fy|)
-  float rt_bary;  // bound of the hit test's barycentric rounding
+  union {
+    struct {
+      // raytracer, binned path: inverse of c2w_R, and the error bounds of a point
+      // projected through it (see project_ray)
+      float inv[9];
+      float rt_rel;   // relative error of the projected camera coordinates
+      float rt_abs;   // pixel margin that every point gets
+      float rt_f;     // max(|fx|, |fy|)
+      float rt_bary;  // bound of the hit test's barycentric rounding
+    };
+    struct {
+      // differentiable forward: a point near the camera, and w2c_R org + w2c_t
+      double org[3], trel[3];
+    };
+  };
 };
 
 struct TexInfo {

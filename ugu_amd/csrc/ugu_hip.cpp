@@ -503,6 +503,23 @@ void fill_view_camera(DevView& v, const UguCamera& cam, int tw, int th, int32_t 
   v.tile_base = tile_base;
 }
 
+// The point that the differentiable forward takes positions from: where the camera is,
+// if the pose is a rotation, in float32 so that differences of positions are exact. The
+// rest of the pose, R org + t, is small and carries no rounding of t's size.
+void set_view_origin(DevView& v) {
+  for (int k = 0; k < 3; k++) {
+    long double o = 0.0L;
+    for (int r = 0; r < 3; r++) o -= static_cast<long double>(v.w2c_R[3 * r + k]) * v.w2c_t[r];
+    v.org[k] = static_cast<float>(o);
+    if (!std::isfinite(v.org[k])) v.org[k] = 0.0;
+  }
+  for (int r = 0; r < 3; r++) {
+    long double t = v.w2c_t[r];
+    for (int k = 0; k < 3; k++) t += static_cast<long double>(v.w2c_R[3 * r + k]) * v.org[k];
+    v.trel[r] = static_cast<double>(t);
+  }
+}
+
 // The copies of the planes staged for host memory (offsets >= 0).
 std::vector<HostCopy> staged_copies(ugu_hip_ctx* c, const UguCamera* cams, int n,
                                     const UguOutputs* outs, const UguGBuffer* gbufs,
@@ -586,6 +603,7 @@ int run_pipeline(ugu_hip_ctx* c, const UguCamera* cams, int n, const DevMesh& dm
     } else {
       v.image = images[i];
       v.face_id = fids[i];
+      set_view_origin(v);
     }
   }
   int persistent_blocks = 0;
