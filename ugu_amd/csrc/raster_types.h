@@ -17,7 +17,7 @@ struct DevView {
   float c2w_t[3];     // camera position: the raytracer's ray origin
   int32_t tiles_x, tiles_y;
   int32_t tile_base;  // first global tile of this view
-  int32_t pad0;
+  float rt_bary;      // raytracer, binned path: bound of the hit test's barycentric rounding
   uint8_t* color;
   float* depth;
   float* normal;
@@ -25,14 +25,16 @@ struct DevView {
   int32_t* face_id;
   float* image;        // differentiable forward: H x W x 3 f32
   const float* grad;   // differentiable backward: H x W x 3 f32
-  // G-buffer planes (null: not written)
-  float* bary;
-  float* uvo;
-  float* pos_wld;
-  float* pos_cam;
-  float* nrm_wld;
-  int32_t* geo_id;
   union {
+    struct {
+      // rasterizer: G-buffer planes (null: not written)
+      float* bary;
+      float* uvo;
+      float* pos_wld;
+      float* pos_cam;
+      float* nrm_wld;
+      int32_t* geo_id;
+    };
     struct {
       // raytracer, binned path: inverse of c2w_R, and the error bounds of a point
       // projected through it (see project_ray)
@@ -40,7 +42,6 @@ struct DevView {
       float rt_rel;   // relative error of the projected camera coordinates
       float rt_abs;   // pixel margin that every point gets
       float rt_f;     // max(|fx|, |fy|)
-      float rt_bary;  // bound of the hit test's barycentric rounding
     };
     struct {
       // differentiable forward: a point near the camera, and w2c_R org + w2c_t
@@ -48,6 +49,9 @@ struct DevView {
     };
   };
 };
+// 68 descriptors are 16 KB. A larger copy to the device is made by the copy engine,
+// whose first use takes 5 to 7 ms.
+static_assert(sizeof(DevView) == 240, "members of the union share 48 bytes");
 
 struct TexInfo {
   int64_t offset;  // byte offset (u8 textures) into the texture pool
