@@ -249,8 +249,8 @@ UGU_DEV void add_corners(double (*sum)[N], const int* slot, const int* vid, cons
 // dL/dZ_j = -G_j b_j / Z_j + the terms through X, Y.
 //
 // 4 wavefronts per SIMD (128 VGPRs; 3 take 1980 us on the case below): no unit is
-// saturated (VALU 35%, LDS 51%, texture addresser 51% busy), the wavefronts wait
-// for the gathers and for memory-side atomics. 19.8 M items of 64 views on 1.3 M
+// saturated (VALU 35%, LDS 51% busy), the wavefronts wait 60% of their cycles for
+// the gathers and for memory-side atomics. 19.8 M items of 64 views on 1.3 M
 // faces, all gradients: 2595 us with one thread per face-sorted item, float32 LDS
 // sums of the texels and 18 global atomics per run of a face; 1377 us here (TCC
 // atomics 44 M -> 13 M). Texture alone, 8.1 M items: 865 -> 328 us.

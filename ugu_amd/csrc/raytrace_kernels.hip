@@ -487,7 +487,7 @@ struct RtLds {
 // rounding of either) is hit later than what each pixel holds.
 // Bound by the latency of a tile's dependent loads (counters, entries, face
 // records, the winner's record and shading inputs), like k_raster. 1.3 M faces
-// at 1080p: setup 26 us + tiles 52 us, where the hierarchy walk (k_raytrace)
+// at 1080p: setup 27 us + tiles 53 us, where the hierarchy walk (k_raytrace)
 // takes 836 us; 24 mixed views of 492 k faces: 153 + 295 us against 2505 us. 6
 // waves per SIMD (78 VGPRs, the rays in LDS only): 5 take 330 us, 7 spill, 333 us.
 __global__ __launch_bounds__(256, 6) void k_rt_tiles(const DevView* __restrict__ views, DevMesh m,
