@@ -976,6 +976,7 @@ int raytrace_binned(ugu_hip_ctx* c, DevView* hv, int n, const DevMesh& dm, const
       return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
     if (launch_raytrace_binned(c->stream, fresh ? hv : nullptr, dv, n, dm, b, large, dopt))
       return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
+    if (c->profile) (void)hipEventRecord(c->ev[1], c->stream);  // before the wait below
     UGU_HIP_CHECK(c, hipStreamSynchronize(c->stream));
     c->rt_large_views = n;
     c->rt_large_set = 1 - c->rt_large_set;
@@ -1099,8 +1100,8 @@ int raytrace_common(ugu_hip_ctx* c, const UguCamera* cams, int n, const UguOptio
     bvh.tris = c->bvh_tris.as<float4>();
     if (launch_raytrace(c->stream, c->views.as<DevView>(), n, rt_tile_base[size_t(n)], bvh, dm, dopt))
       return fail(c, UGU_HIP_ERR_HIP, "kernel launch failed");
+    if (c->profile) (void)hipEventRecord(c->ev[1], c->stream);
   }
-  if (c->profile) (void)hipEventRecord(c->ev[1], c->stream);
   if (!copies.empty())
     UGU_HIP_CHECK(c, c->ring.to_host(c->stream, copies.data(), static_cast<int>(copies.size())));
   UGU_HIP_CHECK(c, hipStreamSynchronize(c->stream));
